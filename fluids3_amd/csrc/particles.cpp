@@ -22,7 +22,9 @@ static const char* kKernelNames[FUNC_MAX] = {
     "computeForceBatch", "advanceParticlesBatch", "fxCountPairsBatch", "sampleParticles",
     "emitParticles",     "fxMaxWords",       "fxMaxWordsBatch",  "fxMark",
     "insertParticlesBatchP", "countingSortIndexBatchP", "countingSortFullBatchP", "computePressureBatchP",
-    "computeForceBatchP", "advanceParticlesBatchP", "fxScanSums", "fxScanApply"};
+    "computeForceBatchP", "advanceParticlesBatchP", "fxScanSums", "fxScanApply",
+    "computePressureWave1", "computePressureWave2", "computePressureWave4",
+    "computePressureWaveBatch1", "computePressureWaveBatch2", "computePressureWaveBatch4"};
 
 Particles::Particles() { memset(&m_Params, 0, sizeof(m_Params)); }
 
@@ -100,9 +102,9 @@ int Particles::Initialize(const char* path) {
   return FX_OK;
 }
 
-int Particles::Launch(int fid, unsigned blocks, unsigned threads, void** args) {
+int Particles::Launch(int fid, unsigned blocks, unsigned threads, void** args, unsigned lds) {
   if (blocks == 0) return FX_OK;
-  FX_HIP(hipModuleLaunchKernel(m_Func[fid], blocks, 1, 1, threads, 1, 1, 0, m_Stream, args, nullptr),
+  FX_HIP(hipModuleLaunchKernel(m_Func[fid], blocks, 1, 1, threads, 1, 1, lds, m_Stream, args, nullptr),
          kKernelNames[fid]);
   return FX_OK;
 }
@@ -171,6 +173,7 @@ int Particles::Restart(const fx_scene& sc) {
   mNumPoints = 0;
   mMaxPoints = sc.num_points;
   m_ScanCells = m_Params.gridTotal + 1;
+  m_MaxSrch = P.gridSrch;
   m_PBase = {0, sc.num_points};
   m_CBase = {0, m_ScanCells};
   FX_TRY(ReallocateParticles(mMaxPoints));
@@ -208,6 +211,8 @@ int Particles::RestartBatch(const fx_scene* scenes, int count) {
   m_SceneParams = ps;
   m_PBase = pb;
   m_CBase = cb;
+  m_MaxSrch = 0;
+  for (const FParams_t& q : ps) m_MaxSrch = q.gridSrch > m_MaxSrch ? q.gridSrch : m_MaxSrch;
   m_Params = ps[0];  // time, dt and the single-scene symbol
   mNumPoints = 0;
   mMaxPoints = pb[count];
@@ -242,23 +247,50 @@ int Particles::BuildBlockTables() {
     if (e.second.first) (void)hipFree(e.second.first);
   m_BTab.clear();
   if (!m_Batch) return FX_OK;
-  for (int k = 0; k < FX_NUM_STAGES; k++) {
-    const int T = m_StageThreads[k] * m_StagePpt[k];  // particles per block
-    if (m_BTab.count(T)) continue;
-    std::vector<int> tab;
-    for (int s = 0; s + 1 < (int)m_PBase.size(); s++) {
-      const int nb = (m_PBase[s + 1] - m_PBase[s] + T - 1) / T;
-      for (int b = 0; b < nb; b++) {
-        tab.push_back(s);
-        tab.push_back(b);
-      }
-    }
-    void* d = nullptr;
-    FX_HIP(hipMalloc(&d, tab.size() * sizeof(int) + 8), "BuildBlockTables");
-    FX_HIP(hipMemcpyHtoD(d, tab.data(), tab.size() * sizeof(int)), "BuildBlockTables");
-    m_BTab[T] = {d, (int)(tab.size() / 2)};
-  }
+  for (int k = 0; k < FX_NUM_STAGES; k++) FX_TRY(BlockTable(m_StageThreads[k] * m_StagePpt[k]));
+  FX_TRY(BlockTable(DensityThreads() / DensityLanes()));
   return FX_OK;
+}
+
+int Particles::BlockTable(int T) {
+  // the table of blocks of T particles
+  if (m_BTab.count(T)) return FX_OK;
+  std::vector<int> tab;
+  for (int s = 0; s + 1 < (int)m_PBase.size(); s++) {
+    const int nb = (m_PBase[s + 1] - m_PBase[s] + T - 1) / T;
+    for (int b = 0; b < nb; b++) {
+      tab.push_back(s);
+      tab.push_back(b);
+    }
+  }
+  void* d = nullptr;
+  FX_HIP(hipMalloc(&d, tab.size() * sizeof(int) + 8), "BuildBlockTables");
+  m_BTab[T] = {d, (int)(tab.size() / 2)};
+  FX_HIP(hipMemcpyHtoD(d, tab.data(), tab.size() * sizeof(int)), "BuildBlockTables");
+  return FX_OK;
+}
+
+bool Particles::WaveDensity() const {
+  // rows of 4 cells and the persistent launches keep the block-wide tiles
+  return m_MaxSrch <= 3 && !(m_Batch && m_Persistent);
+}
+
+int Particles::DensityThreads() const {
+  const int t = m_StageThreads[FX_STAGE_PRESSURE];
+  return t < FX_DENS_THREADS ? t : FX_DENS_THREADS;
+}
+
+int Particles::DensityLanes() const {
+  // Lanes to a particle.  A launch of few waves waits for its longest chain,
+  // which more lanes shorten; one that fills the chip pays for their extra
+  // instructions.  Four lanes were faster than two up to about 85,000
+  // particles (five waves to each of the four SIMDs of a CU) and two faster
+  // than one up to 262,144 (eight, all that are resident at once); the
+  // figures are at the kernel.
+  const int64_t cu = m_NumCU > 0 ? m_NumCU : 1;
+  if ((int64_t)mMaxPoints * 4 <= cu * 20 * 64) return 4;
+  if ((int64_t)mMaxPoints * 2 <= cu * 32 * 64) return 2;
+  return 1;
 }
 
 int Particles::BatchLaunch(int fid, int fid_p, int stage, void* extra0, void* extra1, void* extra2) {
@@ -285,6 +317,21 @@ int Particles::BatchLaunch(int fid, int fid_p, int stage, void* extra0, void* ex
   }
   void* args[4] = {&B, extra0, extra1, extra2};
   return Launch(fid, grid, (unsigned)T, args);
+}
+
+int Particles::LaunchLanes(int fid, int fid_b, int threads, int lanes, unsigned lds) {
+  // a pair stage with `lanes` lanes to a particle, one launch over the scene
+  // or over every scene of a batch
+  const int per = threads / lanes;
+  if (!m_Batch) {
+    void* args[] = {&mNumPoints};
+    return Launch(fid, (unsigned)((mNumPoints + per - 1) / per), (unsigned)threads, args, lds);
+  }
+  const auto it = m_BTab.find(per);
+  if (it == m_BTab.end()) return fx::fail(FX_ESTATE, "batch launch: no block table of %d particles", per);
+  FxBatchArgs B{m_DParams, m_DPBase, m_DCBase, it->second.first, nullptr, it->second.second, 0};
+  void* args[] = {&B, &mNumPoints};
+  return Launch(fid_b, (unsigned)it->second.second, (unsigned)threads, args, lds);
 }
 
 int Particles::SceneRange(int s, int* p0, int* np, int* c0, int* nc) const {
@@ -582,7 +629,10 @@ int Particles::CountingSort() {
 }
 
 int Particles::ComputePressure() {
-  if (m_Batch) {
+  if (WaveDensity()) {
+    const int lanes = DensityLanes(), t = DensityThreads(), v = lanes == 4 ? 2 : lanes - 1;
+    FX_TRY(LaunchLanes(FUNC_PRESS_W + v, FUNC_PRESS_WB + v, t, lanes, FX_DENS_LDS(t)));
+  } else if (m_Batch) {
     FX_TRY(BatchLaunch(FUNC_PRESS_B, FUNC_PRESS_BP, FX_STAGE_PRESSURE, &mNumPoints, nullptr, nullptr));
   } else {
     void* args[] = {&mNumPoints};

@@ -53,7 +53,9 @@
 #define FX_SCAN2_BLOCK 2048   // elements per block (4 per thread)
 #define FX_SCAN2_MAX_BLOCKS 8192
 #define FUNC_SCAN_APPLY 31
-#define FUNC_MAX 32
+#define FUNC_PRESS_W 32    // per-wave density, 1, 2 and 4 lanes to a particle
+#define FUNC_PRESS_WB 35   // the same for a batch
+#define FUNC_MAX 38
 
 #include <map>
 #include <string>
@@ -153,7 +155,7 @@ class Particles {
   hipStream_t Stream() const { return m_Stream; }
 
  private:
-  int Launch(int fid, unsigned blocks, unsigned threads, void** args);
+  int Launch(int fid, unsigned blocks, unsigned threads, void** args, unsigned lds = 0);
   // one thread per particle, with the block size chosen for the stage
   int LaunchP(int fid, int stage, void** args);
   int ScanLevels(void* array1, void* scan1, void* array2, void* scan2, void* array3, void* scan3, int n);
@@ -170,6 +172,11 @@ class Particles {
   // entry, or its persistent variant fid_p (0: none) after resetting the
   // stage's claim counters
   int BatchLaunch(int fid, int fid_p, int stage, void* extra0, void* extra1, void* extra2);
+  int LaunchLanes(int fid, int fid_b, int threads, int lanes, unsigned lds);
+  int DensityLanes() const;
+  int DensityThreads() const;
+  bool WaveDensity() const;
+  int BlockTable(int particles);
   int ResidentBlocks(int fid, int threads, int* blocks);
   int UploadPpt();
   int FinishRestart(int n);
@@ -213,6 +220,7 @@ class Particles {
   hipGraphExec_t m_GraphExec = nullptr;
   bool m_Capturing = false;
   int m_GraphParity = 0;
+  int m_MaxSrch = 0;  // cells a stencil row, the largest of the scenes
   // threads per block of each stage's per-particle kernels (insert, prefix,
   // sort, pressure, force, advance): the sizes fx_autotune keeps choosing on
   // the dam-break and beach scenes at 4M particles
@@ -224,7 +232,7 @@ class Particles {
   int m_NumCU = 0;
   std::map<std::pair<int, int>, int> m_Resident;  // (function, threads) -> resident blocks on the device
 
-  // batch of scenes (m_Batch); a single scene uses the reference-named kernels
+  // batch of scenes (m_Batch); a single scene uses the kernels without Batch in their name
   bool m_Batch = false;
   int m_ScanCells = 0;  // entries of the cell tables: gridTotal+1, or the sum over scenes
   std::vector<FParams_t> m_SceneParams;

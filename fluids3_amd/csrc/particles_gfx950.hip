@@ -1145,6 +1145,380 @@ extern "C" __global__ __launch_bounds__(1024) void computePressureBatchP(BatchAr
   });
 }
 
+// --------------------------------------------------------- density by wave
+//
+// The library's own density stage (stencil rows of 2 or 3 cells): each wave
+// works alone, with G lanes to a particle, on 64 / G consecutive sorted
+// particles.  What the block-wide tiles above cost is waiting: two barriers
+// and two dependent loads per stencil row, nine times, for rows of about 11
+// candidates at rest density, and a block whose particles spread over a
+// sparse layer walks the whole run between its first and last cell.  Here
+// every row's bounds are loaded at once, and the wave stages a layer of the
+// stencil (gridSrch rows), or all rows when they fit, in its own LDS tile
+// with all loads in flight and no barrier.  A layer beyond the tile goes row
+// by row, trimmed to the particle's x-range as above (dense cells), from
+// memory where even one row's run is longer than the tile (sparse layers).
+//
+// G lanes to a particle take candidates s, s + 1, .. of one step each and add
+// their terms in candidate order through DPP broadcasts, so the sums are the
+// same bits for every G.  It costs more instructions per candidate (about 24
+// a wave step of 4 candidates at G = 4, against 15 for one at G = 1) and
+// shortens the chain of a wave, which is what a launch of few waves waits
+// for.  Measured per launch, block tiles / G = 1 / 2 / 4 (us, HIP events
+// around the stage): 16,384 compressed 46 / 28 / 20 / 16; at rest density
+// 65,536 85 / 45 / 33 / 30, 100,000 91 / 49 / 37 / 39, 262,144
+// 99 / 55 / 54 / 71, 400,000 106 / 53 / 60 / 82, 1,000,000
+// 170 / 80 / 112 / 160; the 4M beach from step 20 246 / 185 / 272 / 435 and
+// from step 90 394 / 325 / 475 / 721; the compressed 4M dam break from step 5
+// 917 / 920 / 1500 / 2359, from step 25 1055 / 1050, from step 60
+// 2055 / 1820 (G = 1).  At G = 1 VALU issue (14 instructions a candidate in
+// the unchecked walk, 15 in a staged row) and the LDS reads bound it.
+//
+// Tile: FX_DENS_TILE entries a wave, and FX_DENS_PAD entries after a block's
+// last tile that a lane past its row's end may read and discard: 256-thread
+// blocks of 20 KB, eight to a CU.  Six blocks to a CU (384 entries, a pad of
+// 384) took 207 us on the beach from step 20 and 965 on the compressed dam
+// break, 512 entries 224 and 1095, 256 entries 188 and 959.  Where the lanes'
+// windows lie in a run longer than the tile (compressed cells), the tile
+// slides along the walk; with such rows read from memory, 40 dam-break steps
+// from step 5 took 153.8 instead of 152.0 ms.
+
+// lane K of the particle's G lanes
+template <int G, int K>
+__device__ __forceinline__ float lane_bcast(float v) {
+  constexpr int ctrl = G == 4 ? K * 0x55 : (K == 0 ? 0xA0 : 0xF5);  // quad_perm
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xf, 0xf, true));
+}
+
+// OR over the particle's G lanes
+template <int G>
+__device__ __forceinline__ uint lanes_or(uint v) {
+  if (G >= 2) v |= __builtin_amdgcn_update_dpp(0u, v, 0xB1, 0xf, 0xf, true);  // quad_perm 1,0,3,2
+  if (G >= 4) v |= __builtin_amdgcn_update_dpp(0u, v, 0x4E, 0xf, 0xf, true);  // quad_perm 2,3,0,1
+  return v;
+}
+
+// bit u of v to bit u * G
+template <int G>
+__device__ __forceinline__ uint spread_bits(uint v) {
+  if constexpr (G == 2) {
+    v = (v | v << 8) & 0x00ff00ffu;
+    v = (v | v << 4) & 0x0f0f0f0fu;
+    v = (v | v << 2) & 0x33333333u;
+    v = (v | v << 1) & 0x55555555u;
+  } else if constexpr (G == 4) {
+    v = (v | v << 12) & 0x000f000fu;
+    v = (v | v << 6) & 0x03030303u;
+    v = (v | v << 3) & 0x11111111u;
+  }
+  return v;
+}
+
+// sum + t^3 of the particle's lanes in lane order (tt = t * t)
+template <int G>
+__device__ __forceinline__ float sum_lanes(float tt, float t, float sum) {
+  if constexpr (G == 1) {
+    return fmaf(tt, t, sum);
+  } else if constexpr (G == 2) {
+    sum = fmaf(lane_bcast<2, 0>(tt), lane_bcast<2, 0>(t), sum);
+    return fmaf(lane_bcast<2, 1>(tt), lane_bcast<2, 1>(t), sum);
+  } else {
+    sum = fmaf(lane_bcast<4, 0>(tt), lane_bcast<4, 0>(t), sum);
+    sum = fmaf(lane_bcast<4, 1>(tt), lane_bcast<4, 1>(t), sum);
+    sum = fmaf(lane_bcast<4, 2>(tt), lane_bcast<4, 2>(t), sum);
+    return fmaf(lane_bcast<4, 3>(tt), lane_bcast<4, 3>(t), sum);
+  }
+}
+
+// The density sum of one lane and the bits of the walk's current word, the
+// first candidate highest.
+struct DensAcc {
+  fx_float3 p;
+  float rd2, d2, sum;
+  uint acc;
+};
+
+// One candidate a lane; ok: the lanes that have one.  A lane without a pair
+// adds +0 (sum unchanged).  v_cndmask and v_addc take the wave's pair mask as
+// it is, as in pressure_impl.
+template <int G>
+__device__ __forceinline__ void dens_cand(DensAcc& D, const TileP q, unsigned long long ok) {
+  const float dx = D.p.x - q.x, dy = D.p.y - q.y, dz = D.p.z - q.z;
+  const float dsq = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+  const unsigned long long m = __builtin_amdgcn_ballot_w64(dsq < D.rd2) & __builtin_amdgcn_ballot_w64(dsq > 0.0f) & ok;
+  const float t0 = (D.rd2 - dsq) * D.d2;
+  float t;
+  __asm__("v_cndmask_b32_e64 %0, 0, %1, %2" : "=v"(t) : "v"(t0), "s"(m));
+  unsigned long long carry;
+  uint acc;
+  __asm__("v_addc_co_u32_e64 %0, %1, %2, %2, %3" : "=v"(acc), "=s"(carry) : "v"(D.acc), "s"(m));
+  D.acc = acc;
+  D.sum = sum_lanes<G>(t * t, t, D.sum);
+}
+
+// the word of n steps: bit u * G + sub for this lane's step u, all of the
+// particle's lanes
+template <int G>
+__device__ __forceinline__ uint dens_word(uint acc, int n, int sub) {
+  return lanes_or<G>(spread_bits<G>(__builtin_bitreverse32(acc << (32 - n))) << sub);
+}
+
+template <int G, int SR>
+__device__ __forceinline__ void density_wave(const FParams_t& P, const Span S, int N, float* lds) {
+  constexpr int R = SR * SR;
+  const int lane = (int)(threadIdx.x & 63u), sub = lane & (G - 1);
+  const int i = S.p0 + (S.blk * (int)blockDim.x + (int)threadIdx.x) / G;
+  float* tile = lds + (threadIdx.x >> 6) * (3 * FX_DENS_TILE);
+  const fx_float3* __restrict__ pos = pbuf<const fx_float3>(FPnts, FPOS);
+  const uint* __restrict__ off = pbuf<const uint>(FAccel, AGRIDOFF);
+  uint* __restrict__ bits = pbuf<uint>(FAccel, ANBRBITS);
+  const int gc = i < S.p1 ? pbuf<const int>(FPnts, FGCELL)[i] : FX_GRID_UNDEF;
+  const bool act = gc != FX_GRID_UNDEF;  // the in-range particles are the scene's first
+  const unsigned long long am = __ballot(act);
+  if (am == 0ull) return;
+  const int lastl = 63 - __clzll((long long)am);
+  const int shift = (P.gridRes.z + 1) * P.gridRes.x + 1;
+  const size_t NN = (size_t)N;
+  const int cap = nbr_cap();
+  const bool rec = act && sub == 0;  // the lane that writes the particle's words
+  // Row r: the lane's candidates [jb, jb + len), the wave's run [lo, hi).  A
+  // row ends where the cell after its last one begins.  Lanes past the last
+  // particle load nothing and read what lane 0 reads.
+  int jb[R], len[R], lo[R], hi[R];
+  DensAcc D;
+  D.p = fx_float3{0.0f, 0.0f, 0.0f};
+  D.rd2 = P.rd2;
+  D.d2 = P.d2;
+  D.sum = 0.0f;
+  D.acc = 0u;
+#pragma unroll
+  for (int r = 0; r < R; r++) jb[r] = len[r] = 0;
+  if (act) {
+    D.p = ld3(pos, (size_t)i);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int c0 = gc + P.gridAdj[r * SR] - shift;
+      jb[r] = (int)off[c0];
+      len[r] = (int)off[c0 + SR];
+    }
+  }
+  int total = 0, longest = 0;
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    lo[r] = __builtin_amdgcn_readlane(jb[r], 0);
+    hi[r] = __builtin_amdgcn_readlane(len[r], lastl);
+    len[r] -= jb[r];
+    jb[r] = act ? jb[r] : lo[r];
+    total += hi[r] - lo[r];
+    longest = max(longest, len[r]);
+  }
+  longest = wave_max(longest);
+  // n tile entries, entry k the particle at(k); four loads in flight
+  auto stage = [&](int n, auto at) {
+    for (int k0 = 0; k0 < n; k0 += 256) {
+      fx_float3 q[4];
+#pragma unroll
+      for (int v = 0; v < 4; v++) q[v] = ld3(pos, (size_t)at(min(k0 + 64 * v + lane, n - 1)));
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int k = k0 + 64 * v + lane;
+        if (k < n) tile_put(tile, k, q[v]);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  };
+  // entry k of the rows [r0, r1) staged one after another
+  auto entry = [&](int r0, int r1, int k) {
+    int q = lo[r0], e = 0;
+#pragma unroll
+    for (int r = r0 + 1; r < r1; r++) {
+      e += hi[r - 1] - lo[r - 1];
+      q = k >= e ? lo[r] - e : q;
+    }
+    return q + k;
+  };
+  // a staged row: the lane's candidate s is tile entry a + s, bit s % 32 of
+  // word W + s / 32
+  auto staged_row = [&](int W, int a, int L, int lm) {
+    for (int s0 = 0; s0 < lm; s0 += 32) {
+      const int n = (min(32, lm - s0) + G - 1) / G;  // steps
+      const int left = L - s0 - sub;                 // step u is this lane's while u * G < left
+      D.acc = 0u;
+      int u = 0;
+      for (; u + 4 <= n; u += 4) {
+        TileP q[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) q[v] = tile_get(tile, a + s0 + (u + v) * G + sub);
+#pragma unroll
+        for (int v = 0; v < 4; v++) dens_cand<G>(D, q[v], __builtin_amdgcn_ballot_w64((u + v) * G < left));
+      }
+      for (; u < n; u++)
+        dens_cand<G>(D, tile_get(tile, a + s0 + u * G + sub), __builtin_amdgcn_ballot_w64(u * G < left));
+      const uint word = dens_word<G>(D.acc, n, sub);
+      const int w = W + (s0 >> 5);
+      if (rec && s0 < L && w < cap) bits[(size_t)w * NN + i] = word;
+    }
+  };
+  // a row on its own: the lane walks candidates [ts, te) (see "Row trimming"),
+  // those every lane has unchecked; its words carry the phase ts % 32
+  const uint* __restrict__ cnt = pbuf<const uint>(FAccel, AGRIDCNT);
+  const uint* __restrict__ sstart = pbuf<const uint>(FAccel, ASLABSTART);
+  int slo = 0, shi = FX_SLABS;
+  if (total > FX_DENS_TILE) {
+    const float rlim = __fsqrt_rn(D.rd2) * (1.0f + 0x1p-20f);
+    const float Rg = rlim * P.gridDelta.x + FX_TRIM_MARGIN + (float)P.gridRes.x * 0x1p-20f;
+    const float gp = (D.p.x - P.gridMin.x) * P.gridDelta.x;
+    if (act) trim_slabs(gp, (int)gp, SR, Rg, slo, shi);
+  }
+  auto long_row = [&](int W, int r, int jbr, int L0, int lor, int n) {
+    const int nw = (L0 + 31) >> 5;
+    int ts = 0, te = L0;
+    if (act && sstart != nullptr && L0 > FX_RANK_WAVE) {
+      const int c0 = gc + P.gridAdj[r * SR] - shift, c2 = c0 + SR - 1;
+      const int n0 = (int)cnt[c0], n2 = (int)cnt[c2];
+      if (n0 > FX_RANK_WAVE && n0 <= FX_RANK_CAP) ts = slab_start(sstart, c0, n0, slo);
+      if (n2 > FX_RANK_WAVE && n2 <= FX_RANK_CAP) te = max(ts, te - n2 + slab_start(sstart, c2, n2, shi));
+    }
+    auto put = [&](int w, uint v) {
+      if (rec && W + w < cap) bits[(size_t)(W + w) * NN + i] = v;
+    };
+    const int L = te - ts, ph = ts & 31;
+    const int lm = wave_max(L), lmin = wave_min(act ? L : INT_MAX);
+    int a0 = jbr - lor + ts;  // the lane's first candidate in the row's run
+    const int amin = wave_min(act ? a0 : INT_MAX), spread = wave_max(act ? a0 : 0) - amin;
+    a0 = act ? a0 : amin;
+    int w = ts >> 5;
+    uint carry = 0u;
+    for (int k = 0; k < w; k++) put(k, 0u);
+    // steps [sb, se) of the walk, candidate s at fetch(a0 + s), which holds
+    // entries up to `last`
+    auto part = [&](int sb, int se, int last, auto fetch) {
+      for (int s0 = sb; s0 < se; s0 += 32) {
+        const int ns = (min(32, se - s0) + G - 1) / G;
+        const int nu = max(0, min(ns, (lmin - s0) / G));  // steps with a candidate in every lane
+        D.acc = 0u;
+        int u = 0;
+        for (; u + 4 <= nu; u += 4) {
+          TileP q[4];
+#pragma unroll
+          for (int v = 0; v < 4; v++) q[v] = fetch(a0 + s0 + (u + v) * G + sub);
+#pragma unroll
+          for (int v = 0; v < 4; v++) dens_cand<G>(D, q[v], ~0ull);
+        }
+        for (; u < ns; u++) {
+          const int s = s0 + u * G + sub;
+          dens_cand<G>(D, fetch(min(a0 + s, last)), __builtin_amdgcn_ballot_w64(s < L));
+        }
+        const uint chunk = dens_word<G>(D.acc, ns, sub);
+        if (w < nw) put(w, carry | (chunk << ph));
+        carry = ph ? chunk >> (32 - ph) : 0u;
+        w++;
+      }
+    };
+    // The lanes' windows start within `spread` entries of each other, so a
+    // tile from the first of them serves as many steps as it has entries
+    // beyond that; it then slides on.
+    const int steps = (FX_DENS_TILE - spread) & ~31;
+    if (steps > 0) {
+      for (int sb = 0; sb < lm; sb += steps) {
+        const int base = amin + sb, m = min(n - base, FX_DENS_TILE);
+        stage(m, [&](int k) { return lor + base + k; });
+        part(sb, min(lm, sb + steps), base + m - 1, [&](int k) { return tile_get(tile, k - base); });
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+      }
+    } else {
+      part(0, lm, n - 1, [&](int k) {
+        const fx_float3 q = ld3(pos, (size_t)(lor + k));
+        return TileP{q.x, q.y, q.z};
+      });
+    }
+    if (w < nw) put(w, carry);
+    for (int k = w + 1; k < nw; k++) put(k, 0u);
+  };
+  // reading past a row's end stays within the pad: rows of at most PAD - G
+  const bool all = total <= FX_DENS_TILE && longest <= FX_DENS_PAD - G;
+  int W = 0, t0 = 0;  // the row's first word and tile entry
+#pragma unroll
+  for (int r0 = 0; r0 < R; r0 += SR) {  // a layer of the stencil
+    int n = 0;
+#pragma unroll
+    for (int r = r0; r < r0 + SR; r++) n += hi[r] - lo[r];
+    if (all || (n <= FX_DENS_TILE && longest <= FX_DENS_PAD - G)) {
+      if (!all) {
+        t0 = 0;
+        stage(n, [&](int k) { return entry(r0, r0 + SR, k); });
+      } else if (r0 == 0) {
+        stage(total, [&](int k) { return entry(0, R, k); });
+      }
+#pragma unroll
+      for (int r = r0; r < r0 + SR; r++) {
+        staged_row(W, t0 + jb[r] - lo[r], len[r], wave_max(len[r]));
+        t0 += hi[r] - lo[r];
+        W += (len[r] + 31) >> 5;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    } else {
+      // one copy of the row's code: the bounds of the layer's rows move down
+      int j[SR], m[SR], f[SR], e[SR];
+#pragma unroll
+      for (int k = 0; k < SR; k++) {
+        j[k] = jb[r0 + k];
+        m[k] = len[r0 + k];
+        f[k] = lo[r0 + k];
+        e[k] = hi[r0 + k];
+      }
+#pragma clang loop unroll(disable)
+      for (int k = 0; k < SR; k++) {
+        long_row(W, r0 + k, j[0], m[0], f[0], e[0] - f[0]);
+        W += (m[0] + 31) >> 5;
+#pragma unroll
+        for (int q = 0; q < SR - 1; q++) {
+          j[q] = j[q + 1];
+          m[q] = m[q + 1];
+          f[q] = f[q + 1];
+          e[q] = e[q + 1];
+        }
+      }
+    }
+  }
+  if (!act) return;
+  float rho = D.sum * P.pmass * P.poly6kern;
+  if (rho == 0.0f) rho = 1.0f;
+  float4* fr = pbuf<float4>(FAccel, AFREC);
+  if (sub == 0) {
+    pbuf<float>(FPnts, FPRESS)[i] = rho;
+    fr[2 * (size_t)i] = make_float4(D.p.x, D.p.y, D.p.z, rho);
+  }
+  if (sub == G - 1) {
+    const fx_float3 v = ld3nt(pbuf<const fx_float3>(FPnts, FVEVAL), (size_t)i);
+    fr[2 * (size_t)i + 1] = make_float4(v.x, v.y, v.z, 0.0f);
+  }
+}
+
+extern __shared__ __align__(16) float dens_lds[];  // FX_DENS_LDS(threads) bytes
+
+template <int G>
+__device__ __forceinline__ void density_wave_any(const FParams_t& P, const Span S, int N) {
+  if (P.gridSrch == 3)
+    density_wave<G, 3>(P, S, N, dens_lds);
+  else
+    density_wave<G, 2>(P, S, N, dens_lds);
+}
+
+#define FX_DENSITY_WAVE(G)                                                                                    \
+  extern "C" __global__ __launch_bounds__(FX_DENS_THREADS) void computePressureWave##G(int pnum) {            \
+    density_wave_any<G>(*cparams(&FParams), Span{0, pnum, 0, xcd_block()}, pnum);                             \
+  }                                                                                                           \
+  extern "C" __global__ __launch_bounds__(FX_DENS_THREADS) void computePressureWaveBatch##G(BatchArgs B,      \
+                                                                                          int ntotal) {       \
+    const FParams_t* P;                                                                                       \
+    const Span S = batch_span(B, xcd_block(), P);                                                             \
+    density_wave_any<G>(*P, S, ntotal);                                                                       \
+  }
+FX_DENSITY_WAVE(1)
+FX_DENSITY_WAVE(2)
+FX_DENSITY_WAVE(4)
+
 // ------------------------------------------------------------------- force
 
 // Force (particles.cu:188-225): for 0 < d2 < rd2, r = sqrt(d2 * d2s),

@@ -74,6 +74,12 @@ extern "C" {
 #define ASLABSTART 15 /* per cell c and x slab k: members of c in slabs below k, uint32 at [c * FX_SLABS + k] */
 #define FX_NUM_ABUF 16
 #define FX_NBR_WORDS 256 /* bitmask words per particle (8192 candidates) */
+/* launches of the per-wave density kernels: threads per block at most, tile
+ * entries (12 bytes) of a wave, entries after a block's last tile */
+#define FX_DENS_THREADS 512
+#define FX_DENS_TILE 384
+#define FX_DENS_PAD 128
+#define FX_DENS_LDS(threads) (12 * ((threads) / 64 * FX_DENS_TILE + FX_DENS_PAD))
 #define FX_SLABS 16      /* x slabs per cell: the in-cell order of the ranked sort */
 #define FX_MEMBER_BITS 28 /* AGRID member entries: index in the low 28 bits, x slab above */
 
