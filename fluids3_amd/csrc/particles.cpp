@@ -24,7 +24,8 @@ static const char* kKernelNames[FUNC_MAX] = {
     "insertParticlesBatchP", "countingSortIndexBatchP", "countingSortFullBatchP", "computePressureBatchP",
     "computeForceBatchP", "advanceParticlesBatchP", "fxScanSums", "fxScanApply",
     "computePressureWave1", "computePressureWave2", "computePressureWave4",
-    "computePressureWaveBatch1", "computePressureWaveBatch2", "computePressureWaveBatch4"};
+    "computePressureWaveBatch1", "computePressureWaveBatch2", "computePressureWaveBatch4",
+    "computeForceWave",  "computeForceWaveBatch"};
 
 Particles::Particles() { memset(&m_Params, 0, sizeof(m_Params)); }
 
@@ -248,7 +249,8 @@ int Particles::BuildBlockTables() {
   m_BTab.clear();
   if (!m_Batch) return FX_OK;
   for (int k = 0; k < FX_NUM_STAGES; k++) FX_TRY(BlockTable(m_StageThreads[k] * m_StagePpt[k]));
-  FX_TRY(BlockTable(DensityThreads() / DensityLanes()));
+  FX_TRY(BlockTable(StageThreads(FX_STAGE_PRESSURE, FX_DENS_THREADS) / DensityLanes()));
+  FX_TRY(BlockTable(StageThreads(FX_STAGE_FORCE, FX_FORCE_THREADS)));
   return FX_OK;
 }
 
@@ -270,14 +272,14 @@ int Particles::BlockTable(int T) {
   return FX_OK;
 }
 
-bool Particles::WaveDensity() const {
-  // rows of 4 cells and the persistent launches keep the block-wide tiles
+bool Particles::WaveStages() const {
+  // the per-wave density and force; rows of 4 cells and the persistent
+  // launches keep the block-wide tiles and the earlier queue
   return m_MaxSrch <= 3 && !(m_Batch && m_Persistent);
 }
 
-int Particles::DensityThreads() const {
-  const int t = m_StageThreads[FX_STAGE_PRESSURE];
-  return t < FX_DENS_THREADS ? t : FX_DENS_THREADS;
+int Particles::StageThreads(int stage, int most) const {
+  return m_StageThreads[stage] < most ? m_StageThreads[stage] : most;
 }
 
 int Particles::DensityLanes() const {
@@ -629,8 +631,8 @@ int Particles::CountingSort() {
 }
 
 int Particles::ComputePressure() {
-  if (WaveDensity()) {
-    const int lanes = DensityLanes(), t = DensityThreads(), v = lanes == 4 ? 2 : lanes - 1;
+  if (WaveStages()) {
+    const int lanes = DensityLanes(), t = StageThreads(FX_STAGE_PRESSURE, FX_DENS_THREADS), v = lanes == 4 ? 2 : lanes - 1;
     FX_TRY(LaunchLanes(FUNC_PRESS_W + v, FUNC_PRESS_WB + v, t, lanes, FX_DENS_LDS(t)));
   } else if (m_Batch) {
     FX_TRY(BatchLaunch(FUNC_PRESS_B, FUNC_PRESS_BP, FX_STAGE_PRESSURE, &mNumPoints, nullptr, nullptr));
@@ -643,7 +645,10 @@ int Particles::ComputePressure() {
 }
 
 int Particles::ComputeForce() {
-  if (m_Batch) {
+  if (WaveStages()) {
+    const int t = StageThreads(FX_STAGE_FORCE, FX_FORCE_THREADS);
+    FX_TRY(LaunchLanes(FUNC_FORCE_W, FUNC_FORCE_WB, t, 1, FX_FORCE_LDS(t)));
+  } else if (m_Batch) {
     FX_TRY(BatchLaunch(FUNC_FORCE_B, FUNC_FORCE_BP, FX_STAGE_FORCE, &mNumPoints, nullptr, nullptr));
   } else {
     void* args[] = {&mNumPoints};

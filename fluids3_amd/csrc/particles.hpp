@@ -55,7 +55,9 @@
 #define FUNC_SCAN_APPLY 31
 #define FUNC_PRESS_W 32    // per-wave density, 1, 2 and 4 lanes to a particle
 #define FUNC_PRESS_WB 35   // the same for a batch
-#define FUNC_MAX 38
+#define FUNC_FORCE_W 38    // per-wave force
+#define FUNC_FORCE_WB 39
+#define FUNC_MAX 40
 
 #include <map>
 #include <string>
@@ -174,8 +176,8 @@ class Particles {
   int BatchLaunch(int fid, int fid_p, int stage, void* extra0, void* extra1, void* extra2);
   int LaunchLanes(int fid, int fid_b, int threads, int lanes, unsigned lds);
   int DensityLanes() const;
-  int DensityThreads() const;
-  bool WaveDensity() const;
+  int StageThreads(int stage, int most) const;
+  bool WaveStages() const;
   int BlockTable(int particles);
   int ResidentBlocks(int fid, int threads, int* blocks);
   int UploadPpt();

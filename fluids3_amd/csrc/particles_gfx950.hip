@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "fluidsx_params.h"
+#include "fx_near.hpp"
 #include "fx_trig.hpp"
 
 typedef unsigned int uint;
@@ -1555,18 +1556,24 @@ struct PairTerm {
   float A, B, dx, dy, dz, ux, uy, uz;
 };
 
-__device__ __forceinline__ PairTerm pair_term(const FParams_t& P, const ForceI& I, const float4 a,
-                                              const float4 v) {
+// Near: square root and reciprocal by near_sqrt and near_rcp, their arguments
+// ORed into chk (the term holds when chk < FX_NEAR_SPAN).
+template <bool Near>
+__device__ __forceinline__ PairTerm pair_term(const FParams_t& P, const ForceI& I, const float4 a, const float4 v,
+                                              uint& chk) {
   PairTerm q;
   q.dx = I.px - a.x;
   q.dy = I.py - a.y;
   q.dz = I.pz - a.z;
   const float dsq = fmaf(q.dz, q.dz, fmaf(q.dy, q.dy, q.dx * q.dx));
-  const float rr = sqrtf(dsq * P.d2);
+  const float r2 = dsq * P.d2;
+  const float rr = Near ? near_sqrt(r2) : sqrtf(r2);
   const float c = P.psmoothradius - rr;
   const float dj = a.w;
   const float pj = (dj - P.prest_dens) * P.pintstiff;
-  const float inv = 1.0f / (rr * (I.di * dj));
+  const float den = rr * (I.di * dj);
+  const float inv = Near ? near_rcp(den) : 1.0f / den;
+  if (Near) chk |= near_bits(r2) | near_bits(den);
   const float kp = (P.sim_scale * -0.5f) * P.spikykern;
   q.A = (kp * (c * c)) * (I.pi + pj) * inv;
   q.B = (P.vterm * c) * rr * inv;
@@ -1593,7 +1600,8 @@ __device__ __forceinline__ void pair_add_if(ForceI& I, const PairTerm& q, bool o
 }
 
 __device__ __forceinline__ void force_pair(const FParams_t& P, ForceI& I, const float4 a, const float4 v) {
-  pair_add(I, pair_term(P, I, a, v));
+  uint chk = 0u;
+  pair_add(I, pair_term<false>(P, I, a, v, chk));
 }
 
 __device__ __forceinline__ bool is_pair(const FParams_t& P, const ForceI& I, const float4 a) {
@@ -1799,17 +1807,19 @@ __device__ __forceinline__ void force_walk_q(const FParams_t& P, ForceI& I, cons
       uint j[FW_STEP];
       bool ok[FW_STEP];
       PairTerm q[FW_STEP];
+      uint chk = 0u;
 #pragma unroll
       for (int u = 0; u < FW_STEP; u++) ok[u] = take(j[u]);
 #pragma unroll
-      for (int u = 0; u < FW_STEP; u++) q[u] = pair_term(P, I, srcA[S * (size_t)j[u]], srcV[S * (size_t)j[u]]);
+      for (int u = 0; u < FW_STEP; u++)
+        q[u] = pair_term<false>(P, I, srcA[S * (size_t)j[u]], srcV[S * (size_t)j[u]], chk);
 #pragma unroll
       for (int u = 0; u < FW_STEP; u++) pair_add_if(I, q[u], ok[u]);
     }
     for (; e < f; e++) {
-      uint j;
+      uint j, chk = 0u;
       const bool ok = take(j);
-      pair_add_if(I, pair_term(P, I, srcA[S * (size_t)j], srcV[S * (size_t)j]), ok);
+      pair_add_if(I, pair_term<false>(P, I, srcA[S * (size_t)j], srcV[S * (size_t)j], chk), ok);
     }
     qn = max(qn - f, 0);
   };
@@ -1967,6 +1977,279 @@ extern "C" __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu
     const Span S = batch_span(B, b, P);
     force_q(*P, S, ntotal, lq);
   });
+}
+
+// ----------------------------------------------------------- force by wave
+//
+// The library's own force stage (stencil rows of 2 or 3 cells): the word
+// queue above with three costs taken out.
+//
+// Gathers.  A wave's 64 scattered 16-byte loads take 37 cycles of a CU's
+// texture path whatever their width, 21 when neighbouring lanes read the two
+// halves of one record (16 when four lanes share a 128-byte line; measured on
+// records in L1).  So lanes 2k and 2k + 1 read both halves of the even lane's
+// record together, then both halves of the odd lane's, and exchange what is
+// the other's: seven v_cndmask with a DPP source a pair, written as asm (the
+// compiler makes a move and a select of each).
+//
+// Queue.  All words but the current one lie in LDS, and the two that follow
+// it are read a step ahead, so that a lane that finishes a word waits for
+// nothing; the queue above read the next word when it was needed, inside a
+// branch, up to three times a step.
+//
+// Terms.  Square root and reciprocal by near_sqrt and near_rcp (8
+// instructions instead of 27), with one check for the FQ_STEP terms of a
+// step; a step with an argument outside their range is evaluated again with
+// the IEEE sequences.  The bits are the same.
+//
+// Force per launch, queue above / here (us, HIP events around the stage):
+// the compressed 4M dam break from step 5 1950 / 1640, from step 60
+// 4800 / 4110; the 4M beach from step 20 285 / 260, from step 90 765 / 687;
+// at rest density 1,000,000 at step 40 88 / 77, at step 140 218 / 184,
+// 262,144 at step 90 92 / 78, 65,536 at step 40 44 / 34.  FQ_STEP 2 / 3 / 4 /
+// 5 gave 1708 / 1632 / 1640 / 1727, 4586 / 4287 / 4160 / 4255 and
+// 290 / 267 / 261 / 284 us on the first three; 8 instead of 16 queued words
+// 1857, 4830 and 284 (at FQ_STEP 3).  117 VGPRs, four waves a SIMD; held at
+// 96 it spills (2250 us).  VALU issue bounds it (about 52 instructions a
+// pair and lane) with the gathers' latency beside it.
+#define FQ_K 16   // queued words a lane (FX_FORCE_LDS); a power of two
+#define FQ_STEP 4 // pairs a lane and step
+
+template <int SR>
+__device__ __forceinline__ void force_wave(const FParams_t& P, const Span S, int N, uint* lds) {
+  constexpr int R = SR * SR, MASK = FQ_K * 64 - 1;
+  static_assert(R <= FQ_K, "a word of every row fits the queue");
+  const int lane = (int)(threadIdx.x & 63u);
+  const bool odd = (lane & 1) != 0;
+  const int i = S.p0 + S.blk * (int)blockDim.x + (int)threadIdx.x;
+  uint* qw = lds + (threadIdx.x >> 6) * (2 * FQ_K * 64) + lane;  // words, 64 apart
+  uint* qb = qw + FQ_K * 64;                                      // and where they begin
+  const uint* __restrict__ off = pbuf<const uint>(FAccel, AGRIDOFF);
+  const uint* __restrict__ cell = pbuf<const uint>(FAccel, AGRIDCNT);
+  const uint* __restrict__ bits = pbuf<const uint>(FAccel, ANBRBITS);
+  const float4* __restrict__ fr = pbuf<const float4>(FAccel, AFREC);
+  const float4* __restrict__ half = fr + (odd ? 1 : 0);  // the half of a record this lane reads
+  const int gc = i < S.p1 ? pbuf<const int>(FPnts, FGCELL)[i] : FX_GRID_UNDEF;
+  const bool act = gc != FX_GRID_UNDEF;
+  if (__ballot(act) == 0ull) return;
+  const int shift = (P.gridRes.z + 1) * P.gridRes.x + 1;
+  ForceI I;
+  I.px = I.py = I.pz = I.vx = I.vy = I.vz = 0.0f;
+  I.di = 1.0f;
+  I.pi = 0.0f;
+  I.fx = I.fy = I.fz = 0.0f;
+  // row r: candidates from jb[r], words [E_[r - 1], E_[r]) of the bitmask
+  int jb[R], E_[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) jb[r] = E_[r] = 0;
+  if (act) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int c0 = gc + P.gridAdj[r * SR] - shift;
+      jb[r] = (int)off[c0];
+      E_[r] = (int)off[c0 + SR];
+    }
+    const float4 a = fr[2 * (size_t)i], v = fr[2 * (size_t)i + 1];
+    I.px = a.x; I.py = a.y; I.pz = a.z;
+    I.vx = v.x; I.vy = v.y; I.vz = v.z;
+    I.di = a.w;
+    I.pi = (I.di - P.prest_dens) * P.pintstiff;
+  }
+  int nwords = 0, longest = 0;
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const int len = E_[r] - jb[r];
+    longest = max(longest, len);
+    nwords += (len + 31) >> 5;
+    E_[r] = nwords;
+  }
+  if (act && nwords > nbr_cap()) {  // no recorded bits: test every candidate
+    const int base = stencil_base(P, gc);
+    for (int r = 0; r < R; r++) {
+      int b, e;
+      row_range(P, base, r, off, cell, b, e);
+      for (int j = b; j < e; j++) {
+        const float4 a = fr[2 * (size_t)j];
+        if (is_pair(P, I, a)) force_pair(P, I, a, fr[2 * (size_t)j + 1]);
+      }
+    }
+    nwords = 0;
+#pragma unroll
+    for (int r = 0; r < R; r++) E_[r] = 0;
+  }
+  const size_t NN = (size_t)N;
+  // the current word and what its bit 0 stands for, in half records; the
+  // queue's first two (0 where it holds fewer)
+  uint cur = 0u, curb = 0u, n1 = 0u, n1b = 0u, n2 = 0u, n2b = 0u;
+  int head = 0, cnt = 0;  // of the queue, n1 and n2 included
+  int qn = 0;             // pairs held
+  auto ahead = [&]() {
+    const int h2 = (head + 64) & MASK;
+    n1 = qw[head];
+    n1b = qb[head];
+    n2 = qw[h2];
+    n2b = qb[h2];
+    n1 = cnt > 0 ? n1 : 0u;
+    n2 = cnt > 1 ? n2 : 0u;
+  };
+  // FQ_STEP pairs from every lane (a lane that has none left evaluates record
+  // 0 and discards it), each lane's in candidate order
+  auto step = [&]() {
+    uint j[FQ_STEP];
+    bool ok[FQ_STEP];
+    const int have = min(cnt, 2);
+#pragma unroll
+    for (int u = 0; u < FQ_STEP; u++) {
+      ok[u] = cur != 0u;
+      j[u] = ok[u] ? curb + 2u * (uint)__builtin_ctz(cur) : 0u;
+      const uint rest = cur & (cur - 1u);
+      const bool next = rest == 0u;
+      cur = next ? n1 : rest;
+      curb = next ? n1b : curb;
+      n1 = next ? n2 : n1;
+      n1b = next ? n2b : n1b;
+      n2 = next ? 0u : n2;
+      qn -= ok[u] ? 1 : 0;
+    }
+    const int used = have - (n1 != 0u ? 1 : 0) - (n2 != 0u ? 1 : 0);
+    cnt -= used;
+    head = (head + 64 * used) & MASK;
+    ahead();
+    float4 e[FQ_STEP], o[FQ_STEP];  // this lane's half of the even lane's record, and of the odd lane's
+#pragma unroll
+    for (int u = 0; u < FQ_STEP; u++) {
+      const uint jx = __builtin_amdgcn_update_dpp(0u, j[u], 0xB1, 0xf, 0xf, true);  // quad_perm 1,0,3,2
+      e[u] = half[odd ? jx : j[u]];
+      o[u] = half[odd ? j[u] : jx];
+    }
+    PairTerm q[FQ_STEP];
+    float4 a[FQ_STEP];
+    uint chk = 0u;
+#pragma unroll
+    for (int u = 0; u < FQ_STEP; u++) {
+      // a, the (pos, rho) half: an even lane's e, an odd lane takes the even
+      // lane's o.  o becomes the (veval, 0) half: an odd lane's own, an even
+      // lane takes the odd lane's e.  Every lane of the wave runs this; a DPP
+      // source needs two cycles after a VALU write of it.
+      __asm__("s_nop 1\n\ts_mov_b64 vcc, %8\n\t"
+              "v_cndmask_b32_dpp %0, %4, %9, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+              "v_cndmask_b32_dpp %1, %5, %10, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+              "v_cndmask_b32_dpp %2, %6, %11, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+              "v_cndmask_b32_dpp %3, %7, %12, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+              : "=&v"(a[u].x), "=&v"(a[u].y), "=&v"(a[u].z), "=&v"(a[u].w)
+              : "v"(o[u].x), "v"(o[u].y), "v"(o[u].z), "v"(o[u].w), "s"(0x5555555555555555ull), "v"(e[u].x),
+                "v"(e[u].y), "v"(e[u].z), "v"(e[u].w)
+              : "vcc");
+      __asm__("s_nop 1\n\ts_mov_b64 vcc, %6\n\t"
+              "v_cndmask_b32_dpp %0, %3, %0, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+              "v_cndmask_b32_dpp %1, %4, %1, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+              "v_cndmask_b32_dpp %2, %5, %2, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+              : "+v"(o[u].x), "+v"(o[u].y), "+v"(o[u].z)
+              : "v"(e[u].x), "v"(e[u].y), "v"(e[u].z), "s"(0xAAAAAAAAAAAAAAAAull)
+              : "vcc");
+      q[u] = pair_term<true>(P, I, a[u], o[u], chk);
+    }
+    if (__any(chk >= FX_NEAR_SPAN)) {
+#pragma unroll
+      for (int u = 0; u < FQ_STEP; u++) q[u] = pair_term<false>(P, I, a[u], o[u], chk);
+    }
+    bool every = true;
+#pragma unroll
+    for (int u = 0; u < FQ_STEP; u++) every = every && ok[u];
+    if (__all(every)) {
+#pragma unroll
+      for (int u = 0; u < FQ_STEP; u++) pair_add(I, q[u]);
+    } else {
+#pragma unroll
+      for (int u = 0; u < FQ_STEP; u++) pair_add_if(I, q[u], ok[u]);
+    }
+  };
+  // The bitmask is read once, as a stream: non-temporal loads, as above.
+  if (wave_max(longest) <= 32) {
+    // a word a row: the queue holds them all
+    uint w[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int f = r == 0 ? 0 : E_[r - 1];
+      w[r] = f < E_[r] ? __builtin_nontemporal_load(&bits[(size_t)f * NN + i]) : 0u;
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {  // a zero word is written over by the next
+      qw[64 * cnt] = w[r];
+      qb[64 * cnt] = 2u * (uint)jb[r];
+      cnt += w[r] != 0u ? 1 : 0;
+      qn += __popc(w[r]);
+    }
+  } else {
+    const int maxf = wave_max(nwords);
+    uint nx[FW_AHEAD];
+#pragma unroll
+    for (int k = 0; k < FW_AHEAD; k++) nx[k] = k < nwords ? __builtin_nontemporal_load(&bits[(size_t)k * NN + i]) : 0u;
+    for (int f0 = 0; f0 < maxf; f0 += FW_AHEAD) {
+      uint cw[FW_AHEAD];
+#pragma unroll
+      for (int k = 0; k < FW_AHEAD; k++) {
+        cw[k] = nx[k];
+        const int fn = f0 + FW_AHEAD + k;
+        nx[k] = fn < nwords ? __builtin_nontemporal_load(&bits[(size_t)fn * NN + i]) : 0u;
+      }
+#pragma unroll
+      for (int k = 0; k < FW_AHEAD; k++) {
+        const int f = f0 + k;
+        if (f >= maxf) break;
+        const uint word = cw[k];
+        int base = jb[0], first = 0;  // of the row that holds word f
+#pragma unroll
+        for (int r = 1; r < R; r++) {
+          const bool in = f >= E_[r - 1];
+          base = in ? jb[r] : base;
+          first = in ? E_[r - 1] : first;
+        }
+        const bool full = word != 0u && cnt == FQ_K;
+        if (__any(full)) {
+          // free a slot: the full lanes finish their current word, every lane
+          // gives as many pairs as the shortest queue holds
+          ahead();
+          int f1 = max(wave_max(full ? __popc(cur) + 1 : 0), wave_min(nwords > 0 ? qn : INT_MAX));
+          do {
+            step();
+            f1 -= FQ_STEP;
+          } while (f1 > 0 || __any(word != 0u && cnt == FQ_K));
+        }
+        if (word != 0u) {
+          const int t = (head + 64 * cnt) & MASK;
+          qw[t] = word;
+          qb[t] = 2u * (uint)(base + ((f - first) << 5));
+          cnt++;
+          qn += __popc(word);
+        }
+      }
+    }
+  }
+  ahead();
+  while (__any(qn > 0)) step();
+  if (act) st3(pbuf<fx_float3>(FPnts, FFORCE), (size_t)i, I.fx, I.fy, I.fz);
+}
+
+extern __shared__ uint force_lds[];  // FX_FORCE_LDS(threads) bytes
+
+__device__ __forceinline__ void force_wave_any(const FParams_t& P, const Span S, int N) {
+  if (P.gridSrch == 3)
+    force_wave<3>(P, S, N, force_lds);
+  else
+    force_wave<2>(P, S, N, force_lds);
+}
+
+// Bounds of 1024 threads, twice what is launched, keep the compiler's schedule
+// at four waves a SIMD: 280 instead of 260 us on the beach with 512.
+extern "C" __global__ __launch_bounds__(1024) void computeForceWave(int pnum) {
+  force_wave_any(*cparams(&FParams), Span{0, pnum, 0, xcd_block()}, pnum);
+}
+
+extern "C" __global__ __launch_bounds__(1024) void computeForceWaveBatch(BatchArgs B, int ntotal) {
+  const FParams_t* P;
+  const Span S = batch_span(B, xcd_block(), P);
+  force_wave_any(*P, S, ntotal);
 }
 
 // ------------------------------------------------------ neighbour statistics

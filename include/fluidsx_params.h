@@ -80,6 +80,9 @@ extern "C" {
 #define FX_DENS_TILE 384
 #define FX_DENS_PAD 128
 #define FX_DENS_LDS(threads) (12 * ((threads) / 64 * FX_DENS_TILE + FX_DENS_PAD))
+/* and of the per-wave force kernels: 16 queued (word, base) pairs a thread */
+#define FX_FORCE_THREADS 512
+#define FX_FORCE_LDS(threads) (128 * (threads))
 #define FX_SLABS 16      /* x slabs per cell: the in-cell order of the ranked sort */
 #define FX_MEMBER_BITS 28 /* AGRID member entries: index in the low 28 bits, x slab above */
 
