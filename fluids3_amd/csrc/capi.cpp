@@ -149,8 +149,7 @@ int fx_stage(fx_system* s, int32_t stage) {
 int fx_run(fx_system* s, int32_t nsteps) {
   FX_CHECK_SYS(s);
   if (nsteps < 0) return fx::fail(FX_EINVAL, "fx_run: nsteps < 0");
-  for (int k = 0; k < nsteps; k++) FX_TRY(s->p.Run());
-  return FX_OK;
+  return s->p.Run(nsteps);
 }
 
 int fx_synchronize(fx_system* s) {

@@ -25,7 +25,7 @@ static const char* kKernelNames[FUNC_MAX] = {
     "computeForceBatchP", "advanceParticlesBatchP", "fxScanSums", "fxScanApply",
     "computePressureWave1", "computePressureWave2", "computePressureWave4",
     "computePressureWaveBatch1", "computePressureWaveBatch2", "computePressureWaveBatch4",
-    "computeForceWave",  "computeForceWaveBatch"};
+    "computeForceWave",  "computeForceWaveBatch", "advanceInsert", "advanceInsertBatch"};
 
 Particles::Particles() { memset(&m_Params, 0, sizeof(m_Params)); }
 
@@ -321,18 +321,18 @@ int Particles::BatchLaunch(int fid, int fid_p, int stage, void* extra0, void* ex
   return Launch(fid, grid, (unsigned)T, args);
 }
 
-int Particles::LaunchLanes(int fid, int fid_b, int threads, int lanes, unsigned lds) {
+int Particles::LaunchLanes(int fid, int fid_b, int threads, int lanes, unsigned lds, void* extra0, void* extra1) {
   // a pair stage with `lanes` lanes to a particle, one launch over the scene
   // or over every scene of a batch
   const int per = threads / lanes;
   if (!m_Batch) {
-    void* args[] = {&mNumPoints};
+    void* args[] = {&mNumPoints, extra0, extra1};
     return Launch(fid, (unsigned)((mNumPoints + per - 1) / per), (unsigned)threads, args, lds);
   }
   const auto it = m_BTab.find(per);
   if (it == m_BTab.end()) return fx::fail(FX_ESTATE, "batch launch: no block table of %d particles", per);
   FxBatchArgs B{m_DParams, m_DPBase, m_DCBase, it->second.first, nullptr, it->second.second, 0};
-  void* args[] = {&B, &mNumPoints};
+  void* args[] = {&B, &mNumPoints, extra0, extra1};
   return Launch(fid_b, (unsigned)it->second.second, (unsigned)threads, args, lds);
 }
 
@@ -525,10 +525,14 @@ int Particles::PrefixScanParticles() {
   // auxiliary level of each, which holds one entry per 1024 elements); the
   // reference's three-level prefixSum/prefixFixup for a scan beyond
   // FX_SCAN2_MAX_BLOCKS blocks.
-  FX_TRY(ScanTwoLaunch(m_Accel.gpu(AGRIDCNT), m_Accel.gpu(AGRIDOFF), m_Accel.gpu(AAUXARRAY1), m_ScanCells,
-                       m_Accel.gpu(ATAILFLAG), m_Accel.gpu(ATAILSCAN), m_Accel.gpu(ATAILAUX1), mNumPoints));
+  FX_TRY(ScanGrid(false));
   m_Done = FX_STAGE_PREFIX;
   return FX_OK;
+}
+
+int Particles::ScanGrid(bool exchange) {
+  return ScanTwoLaunch(m_Accel.gpu(AGRIDCNT), m_Accel.gpu(AGRIDOFF), m_Accel.gpu(AAUXARRAY1), m_ScanCells,
+                       m_Accel.gpu(ATAILFLAG), m_Accel.gpu(ATAILSCAN), m_Accel.gpu(ATAILAUX1), mNumPoints, exchange);
 }
 
 namespace {
@@ -540,12 +544,23 @@ struct ScanJob {
   int n;
   int nb;
 };
+// FxExchange of the code object
+struct Exchange {
+  void* bank;
+  void* pnts;
+  void* tmp;
+  void* clock;
+  float dt;
+  int parity;
+};
 struct ScanJobs {
   ScanJob j[2];
+  Exchange ex;
 };
 }  // namespace
 
-int Particles::ScanTwoLaunch(void* in, void* out, void* sums, int n, void* in2, void* out2, void* sums2, int n2) {
+int Particles::ScanTwoLaunch(void* in, void* out, void* sums, int n, void* in2, void* out2, void* sums2, int n2,
+                             bool exchange) {
   const int nb = (n + FX_SCAN2_BLOCK - 1) / FX_SCAN2_BLOCK;
   const int nb2 = (n2 + FX_SCAN2_BLOCK - 1) / FX_SCAN2_BLOCK;
   if (nb > FX_SCAN2_MAX_BLOCKS || nb2 > FX_SCAN2_MAX_BLOCKS) {
@@ -560,9 +575,13 @@ int Particles::ScanTwoLaunch(void* in, void* out, void* sums, int n, void* in2, 
                         m_Accel.gpu(ATAILAUXS2), m);
     };
     FX_TRY(one(in, out, sums, n));
-    return n2 > 0 ? one(in2, out2, sums2, n2) : FX_OK;
+    if (n2 > 0) FX_TRY(one(in2, out2, sums2, n2));
+    return exchange ? PublishTables() : FX_OK;
   }
-  ScanJobs J = {{{in, out, sums, n, nb}, {in2, out2, sums2, n2, nb2}}};
+  ScanJobs J = {{{in, out, sums, n, nb}, {in2, out2, sums2, n2, nb2}}, {}};
+  if (exchange)
+    J.ex = {m_Tables, m_Points.SymbolAddress(), m_PointsTemp.SymbolAddress(), m_Capturing ? (void*)m_Clock : nullptr,
+            m_Params.dt, m_Parity};
   if (nb + nb2 == 0) return FX_OK;
   void* a[] = {&J};
   FX_TRY(Launch(FUNC_SCAN_SUMS, (unsigned)(nb + nb2), FX_SCAN2_THREADS, a));
@@ -596,13 +615,9 @@ int Particles::PublishTables() {
   // FPnts <- table of the set m_Points now holds, FPntTmp <- the other one;
   // in a captured step the same launch moves the step clock (the advance of
   // this step reads clock[0])
-  void* bank = m_Tables;
-  void* pnts = m_Points.SymbolAddress();
-  void* tmp = m_PointsTemp.SymbolAddress();
-  void* clk = m_Capturing ? (void*)m_Clock : nullptr;
-  float dt = m_Params.dt;
-  int parity = m_Parity;
-  void* args[] = {&bank, &parity, &pnts, &tmp, &clk, &dt};
+  Exchange ex = {m_Tables, m_Points.SymbolAddress(), m_PointsTemp.SymbolAddress(),
+                 m_Capturing ? (void*)m_Clock : nullptr, m_Params.dt, m_Parity};
+  void* args[] = {&ex};
   return Launch(FUNC_PUBLISH, 1, 64, args);
 }
 
@@ -618,6 +633,10 @@ int Particles::CountingSort() {
   FX_TRY(m_Points.SwapGPU(&m_PointsTemp));
   m_Parity ^= 1;
   FX_TRY(PublishTables());
+  return SortKernels();
+}
+
+int Particles::SortKernels() {
   if (m_Batch) {
     FX_TRY(BatchLaunch(FUNC_SORT_INDEX_B, FUNC_SORT_INDEX_BP, FX_STAGE_SORT, nullptr, nullptr, nullptr));
     FX_TRY(BatchLaunch(FUNC_SORT_FULL_B, FUNC_SORT_FULL_BP, FX_STAGE_SORT, nullptr, nullptr, nullptr));
@@ -644,10 +663,11 @@ int Particles::ComputePressure() {
   return FX_OK;
 }
 
-int Particles::ComputeForce() {
+int Particles::ComputeForce(bool clear) {
   if (WaveStages()) {
     const int t = StageThreads(FX_STAGE_FORCE, FX_FORCE_THREADS);
-    FX_TRY(LaunchLanes(FUNC_FORCE_W, FUNC_FORCE_WB, t, 1, FX_FORCE_LDS(t)));
+    void* cnt = clear ? m_Accel.gpu(AGRIDCNT) : nullptr;  // counts cleared for the next step's insert
+    FX_TRY(LaunchLanes(FUNC_FORCE_W, FUNC_FORCE_WB, t, 1, FX_FORCE_LDS(t), &cnt, &m_ScanCells));
   } else if (m_Batch) {
     FX_TRY(BatchLaunch(FUNC_FORCE_B, FUNC_FORCE_BP, FX_STAGE_FORCE, &mNumPoints, nullptr, nullptr));
   } else {
@@ -713,16 +733,43 @@ int Particles::Stage(int stage) {
   }
 }
 
-int Particles::Run() {
-  if (mNumPoints == 0) return fx::fail(FX_ESTATE, "Run: call Restart first");
-  FX_TRY(InsertParticles());
-  FX_TRY(PrefixScanParticles());
-  FX_TRY(CountingSort());
+// Whether a step's advance may also make the next step's insert: one particle
+// per thread in both, and the per-wave stages, whose force clears the counts.
+bool Particles::JoinedSteps() const {
+  return WaveStages() && m_StagePpt[FX_STAGE_INSERT] == 1 && m_StagePpt[FX_STAGE_ADVANCE] == 1;
+}
+
+// One step of several that run straight through.  first: no step before it
+// made its insert; last: it leaves the counts, cells and ranks of its own
+// sort, as a step alone does.
+int Particles::Step(bool first, bool last) {
+  const bool joined = JoinedSteps();
+  if (first || !joined) FX_TRY(InsertParticles());
+  FX_TRY(m_Points.SwapGPU(&m_PointsTemp));
+  m_Parity ^= 1;
+  FX_TRY(ScanGrid(true));
+  FX_TRY(SortKernels());
   FX_TRY(ComputePressure());
-  FX_TRY(ComputeForce());
-  FX_TRY(Advance());
-  AdvanceTime();
+  FX_TRY(ComputeForce(joined && !last));
+  FX_TRY(joined && !last ? AdvanceInsert() : Advance());
   m_Done = FX_STAGE_ADVANCE;
+  return FX_OK;
+}
+
+int Particles::AdvanceInsert() {
+  float dt = m_Params.dt, ss = m_Params.sim_scale, time = m_Params.time;
+  void* clk = m_Capturing ? (void*)m_Clock : nullptr;
+  if (m_Batch) return BatchLaunch(FUNC_ADVANCE_INSERT_B, 0, FX_STAGE_INSERT, &clk, &time, nullptr);
+  void* args[] = {&clk, &time, &dt, &ss, &mNumPoints};
+  return LaunchP(FUNC_ADVANCE_INSERT, FX_STAGE_INSERT, args);
+}
+
+int Particles::Run(int nsteps) {
+  if (mNumPoints == 0) return fx::fail(FX_ESTATE, "Run: call Restart first");
+  for (int s = 0; s < nsteps; s++) {
+    FX_TRY(Step(s == 0, s + 1 == nsteps));
+    AdvanceTime();
+  }
   return FX_OK;
 }
 
@@ -743,14 +790,7 @@ int Particles::CaptureGraph() {
   FX_HIP(hipStreamBeginCapture(m_Stream, hipStreamCaptureModeThreadLocal), "CaptureGraph");
   m_Capturing = true;
   int st = FX_OK;
-  for (int s = 0; s < 2 && st == FX_OK; s++) {
-    st = InsertParticles();
-    if (st == FX_OK) st = PrefixScanParticles();
-    if (st == FX_OK) st = CountingSort();
-    if (st == FX_OK) st = ComputePressure();
-    if (st == FX_OK) st = ComputeForce();
-    if (st == FX_OK) st = Advance();
-  }
+  for (int s = 0; s < 2 && st == FX_OK; s++) st = Step(s == 0, s == 1);
   m_Capturing = false;
   hipGraph_t g = nullptr;
   hipError_t e = hipStreamEndCapture(m_Stream, &g);
@@ -1110,7 +1150,7 @@ int Particles::TimeSteps(int nsteps, bool use_graph, double* ms_total) {
       }
       if (st == FX_OK && (nsteps & 1)) st = Run();
     } else {
-      for (int k = 0; k < nsteps && st == FX_OK; k++) st = Run();
+      st = Run(nsteps);
     }
   }
   if (st == FX_OK && hipEventRecord(b, m_Stream) != hipSuccess) st = fx::fail(FX_EHIP, "time_steps: record");

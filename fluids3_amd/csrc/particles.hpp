@@ -57,7 +57,9 @@
 #define FUNC_PRESS_WB 35   // the same for a batch
 #define FUNC_FORCE_W 38    // per-wave force
 #define FUNC_FORCE_WB 39
-#define FUNC_MAX 40
+#define FUNC_ADVANCE_INSERT 40  // a step's advance and the next one's insert
+#define FUNC_ADVANCE_INSERT_B 41
+#define FUNC_MAX 42
 
 #include <map>
 #include <string>
@@ -106,12 +108,12 @@ class Particles {
   bool Persistent() const { return m_Persistent; }
 
   // the step (particles.cpp:382-400)
-  int Run();
+  int Run(int nsteps = 1);
   int InsertParticles();
   int PrefixScanParticles();
   int CountingSort();
   int ComputePressure();
-  int ComputeForce();
+  int ComputeForce(bool clear = false);  // clear: zero the cell counts for an insert that follows (WaveStages only)
   int Advance();
   void AdvanceTime();
   int Stage(int stage);
@@ -165,8 +167,13 @@ class Particles {
   // uint per block of 2048 elements
   // exclusive scans of up to two arrays (n2 = 0: one) in two launches
   int ScanTwoLaunch(void* in, void* out, void* sums, int n, void* in2 = nullptr, void* out2 = nullptr,
-                    void* sums2 = nullptr, int n2 = 0);
+                    void* sums2 = nullptr, int n2 = 0, bool exchange = false);
+  int ScanGrid(bool exchange);
+  int SortKernels();
   int PublishTables();
+  bool JoinedSteps() const;
+  int Step(bool first, bool last);
+  int AdvanceInsert();
   int SetDeviceClock();
   void ReleaseGraph();
   int BuildBlockTables();
@@ -174,7 +181,8 @@ class Particles {
   // entry, or its persistent variant fid_p (0: none) after resetting the
   // stage's claim counters
   int BatchLaunch(int fid, int fid_p, int stage, void* extra0, void* extra1, void* extra2);
-  int LaunchLanes(int fid, int fid_b, int threads, int lanes, unsigned lds);
+  int LaunchLanes(int fid, int fid_b, int threads, int lanes, unsigned lds, void* extra0 = nullptr,
+                  void* extra1 = nullptr);
   int DensityLanes() const;
   int StageThreads(int stage, int most) const;
   bool WaveStages() const;

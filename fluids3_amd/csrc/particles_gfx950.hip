@@ -297,12 +297,12 @@ extern "C" __global__ void fxMark(int tag) {}
 // of atomics on that one address.  `tl` is the block's LDS (two sets of 17
 // words, alternating between calls so that one call's reads cannot meet
 // the next call's writes).
-__device__ __forceinline__ void insert_impl(const FParams_t& P, const Span S, bool tail, uint (*tl)[17]) {
+__device__ __forceinline__ void insert_at(const FParams_t& P, const Span S, const fx_float3 p, bool tail,
+                                          uint (*tl)[17]) {
   const int i = S.p0 + S.blk * (int)blockDim.x + (int)threadIdx.x;
   bool active = i < S.p1;  // below: particles that take a count slot
   int gs = 0;
   if (active) {
-    const fx_float3 p = pbuf<const fx_float3>(FPnts, FPOS)[i];
     const float gx = (p.x - P.gridMin.x) * P.gridDelta.x;
     const float gy = (p.y - P.gridMin.y) * P.gridDelta.y;
     const float gz = (p.z - P.gridMin.z) * P.gridDelta.z;
@@ -365,6 +365,13 @@ __device__ __forceinline__ void insert_impl(const FParams_t& P, const Span S, bo
     mine = tm;
   }
   if (active) pbuf<int>(FPnts, FGNDX)[i] = (int)(base + lanes_below(mine));
+}
+
+__device__ __forceinline__ void insert_impl(const FParams_t& P, const Span S, bool tail, uint (*tl)[17]) {
+  const int i = S.p0 + S.blk * (int)blockDim.x + (int)threadIdx.x;
+  fx_float3 p = fx_float3{0.0f, 0.0f, 0.0f};
+  if (i < S.p1) p = ld3(pbuf<const fx_float3>(FPnts, FPOS), (size_t)i);
+  insert_at(P, S, p, tail, tl);
 }
 
 // The streaming kernels keep a straight-line body for one particle per
@@ -490,8 +497,38 @@ struct FxScanJob {
   int n;
   int nb;  // blocks: ceil(n / FXS_BLOCK)
 };
+// The set exchange of the counting sort: FPnts and FPntTmp receive the two
+// 128-byte tables of bank[parity] and bank[parity ^ 1] (64 threads).  In a
+// captured step it also moves the step clock: clock[1] holds the time of the
+// step about to run, which becomes clock[0] (read by the advance of this
+// step) while clock[1] moves on by dt.  No exchange where bank is null.
+struct FxExchange {
+  const uint* bank;
+  uint* pnts;
+  uint* tmp;
+  float* clock;
+  float dt;
+  int parity;
+};
+
+__device__ __forceinline__ void exchange_tables(const FxExchange& E) {
+  const int t = (int)threadIdx.x;
+  constexpr int W = (int)(sizeof(cuDataX) / sizeof(uint));
+  static_assert(2 * W <= 64, "one thread per word of the two tables");
+  if (t < W) E.pnts[t] = E.bank[E.parity * W + t];
+  else if (t < 2 * W) E.tmp[t - W] = E.bank[(E.parity ^ 1) * W + t - W];
+  if (E.clock != nullptr && t == 0) {
+    const float now = E.clock[1];
+    E.clock[0] = now;
+    E.clock[1] = now + E.dt;
+  }
+}
+
+// (fxScanApply also makes the exchange when a step runs straight through: the
+// scans read neither table.)
 struct FxScanJobs {
   FxScanJob j[2];
+  FxExchange ex;
 };
 
 __device__ __forceinline__ const FxScanJob& fxs_job(const FxScanJobs& J, int& b) {
@@ -512,6 +549,7 @@ extern "C" __global__ __launch_bounds__(FXS_THREADS) void fxScanSums(FxScanJobs 
 
 extern "C" __global__ __launch_bounds__(FXS_THREADS) void fxScanApply(FxScanJobs J) {
   __shared__ uint lds[FXS_THREADS / 64];
+  if (blockIdx.x == 0 && J.ex.bank != nullptr) exchange_tables(J.ex);
   int b;
   const FxScanJob& S = fxs_job(J, b);
   const uint* __restrict__ in = S.in;
@@ -2233,6 +2271,15 @@ __device__ __forceinline__ void force_wave(const FParams_t& P, const Span S, int
 
 extern __shared__ uint force_lds[];  // FX_FORCE_LDS(threads) bytes
 
+// Clears n counts, spread over the launch: no stage after the density reads
+// them, and the advance of this step also makes the next step's insert.
+// After the pairs: before them it cost the batch kernel five registers and
+// 2 % of its time.
+__device__ __forceinline__ void clear_counts(uint* __restrict__ p, int n) {
+  if (p == nullptr) return;
+  for (int k = (int)(blockIdx.x * blockDim.x + threadIdx.x); k < n; k += (int)(gridDim.x * blockDim.x)) p[k] = 0u;
+}
+
 __device__ __forceinline__ void force_wave_any(const FParams_t& P, const Span S, int N) {
   if (P.gridSrch == 3)
     force_wave<3>(P, S, N, force_lds);
@@ -2242,14 +2289,17 @@ __device__ __forceinline__ void force_wave_any(const FParams_t& P, const Span S,
 
 // Bounds of 1024 threads, twice what is launched, keep the compiler's schedule
 // at four waves a SIMD: 280 instead of 260 us on the beach with 512.
-extern "C" __global__ __launch_bounds__(1024) void computeForceWave(int pnum) {
+extern "C" __global__ __launch_bounds__(1024) void computeForceWave(int pnum, uint* clear, int nclear) {
   force_wave_any(*cparams(&FParams), Span{0, pnum, 0, xcd_block()}, pnum);
+  clear_counts(clear, nclear);
 }
 
-extern "C" __global__ __launch_bounds__(1024) void computeForceWaveBatch(BatchArgs B, int ntotal) {
+extern "C" __global__ __launch_bounds__(1024) void computeForceWaveBatch(BatchArgs B, int ntotal, uint* clear,
+                                                                                int nclear) {
   const FParams_t* P;
   const Span S = batch_span(B, xcd_block(), P);
   force_wave_any(*P, S, ntotal);
+  clear_counts(clear, nclear);
 }
 
 // ------------------------------------------------------ neighbour statistics
@@ -2427,15 +2477,15 @@ extern "C" __global__ void emitParticles(float frame, int emit, int numPnts) {
 // (Y-min with slope and friction, Y-max with friction, X-min moving wall whose
 // stiffness term is scaled by 'wall', X-max, Z-min, Z-max), gravity, the
 // acceleration limit, the velocity limit applied to the old velocity, and the
-// leapfrog update.  GRID_UNDEF particles are parked at (-1000)^3 with zero
-// velocity.
-__device__ __forceinline__ void advance_one(const FParams_t& P, int i, float time, float dt, float ss) {
+// leapfrog update; returns the new position.  GRID_UNDEF particles are parked
+// at (-1000)^3 with zero velocity.
+__device__ __forceinline__ fx_float3 advance_one(const FParams_t& P, int i, float time, float dt, float ss) {
   fx_float3* __restrict__ posb = pbuf<fx_float3>(FPnts, FPOS);
   fx_float3* __restrict__ velb = pbuf<fx_float3>(FPnts, FVEL);
   if (pbuf<const int>(FPnts, FGCELL)[i] == FX_GRID_UNDEF) {
     posb[i] = fx_float3{-1000.0f, -1000.0f, -1000.0f};
     velb[i] = fx_float3{0.0f, 0.0f, 0.0f};
-    return;
+    return fx_float3{-1000.0f, -1000.0f, -1000.0f};
   }
   fx_float3* __restrict__ vevb = pbuf<fx_float3>(FPnts, FVEVAL);
   const fx_float3 pos = posb[i];
@@ -2525,7 +2575,9 @@ __device__ __forceinline__ void advance_one(const FParams_t& P, int i, float tim
   vevb[i] = fx_float3{(vel.x + vnx) * 0.5f, (vel.y + vny) * 0.5f, (vel.z + vnz) * 0.5f};
   velb[i] = fx_float3{vnx, vny, vnz};
   const float dts = dt / ss;
-  posb[i] = fx_float3{pos.x + vnx * dts, pos.y + vny * dts, pos.z + vnz * dts};
+  const float x = pos.x + vnx * dts, y = pos.y + vny * dts, z = pos.z + vnz * dts;
+  posb[i] = fx_float3{x, y, z};
+  return fx_float3{x, y, z};
 }
 
 extern "C" __global__ void advanceParticles(float time, float dt, float ss, int numPnts) {
@@ -2558,24 +2610,8 @@ extern "C" __global__ void advanceParticlesClock(const float* clock, float dt, f
   }
 }
 
-// The set exchange of the counting sort (one launch, 64 threads): FPnts and
-// FPntTmp receive the two 128-byte tables of bank[parity] and
-// bank[parity ^ 1].  In a captured step it also moves the step clock: clock[1]
-// holds the time of the step about to run, which becomes clock[0] (read by
-// the advance of this step) while clock[1] moves on by dt.
-extern "C" __global__ void fxPublishTables(const uint* __restrict__ bank, int parity, uint* __restrict__ pnts,
-                                           uint* __restrict__ tmp, float* __restrict__ clock, float dt) {
-  const int t = (int)threadIdx.x;
-  constexpr int W = (int)(sizeof(cuDataX) / sizeof(uint));
-  static_assert(2 * W <= 64, "one thread per word of the two tables");
-  if (t < W) pnts[t] = bank[parity * W + t];
-  else if (t < 2 * W) tmp[t - W] = bank[(parity ^ 1) * W + t - W];
-  if (clock != nullptr && t == 0) {
-    const float now = clock[1];
-    clock[0] = now;
-    clock[1] = now + dt;
-  }
-}
+// The set exchange as a launch of its own (64 threads).
+extern "C" __global__ void fxPublishTables(FxExchange E) { exchange_tables(E); }
 
 // Batch integrator: the time comes from clock[0] when clock is given, else
 // from the argument; dt and the scale from each scene's parameters.
@@ -2587,6 +2623,34 @@ __device__ __forceinline__ void advance_entry(const BatchArgs& B, int b, const f
     const int i = S.p0 + (S.blk * ppt + k) * (int)blockDim.x + (int)threadIdx.x;
     if (i < S.p1) advance_one(*P, i, clock != nullptr ? clock[0] : time, P->dt, P->sim_scale);
   }
+}
+
+// The advance of a step and the insert of the next in one pass, for steps that
+// run straight through: the position goes from one to the other in
+// registers, and the launch that is saved costs a small scene some 4 us (each
+// waits for the one before it and for its writes).  The counts were cleared
+// by the force stage.  4M particles on the beach: 75 us for 54 + 52 + 11 of
+// advance, insert and clearing.  Runs with these and the exchange merged:
+// 54.2 instead of 58.7 us a step at 16,384 particles, 156 instead of 165 at
+// 262,144, 1099 instead of 1133 at the beach.
+extern "C" __global__ void advanceInsert(const float* clock, float time, float dt, float ss, int numPnts) {
+  __shared__ uint tl[2][17];
+  const FParams_t& P = *cparams(&FParams);
+  const Span S{0, numPnts, 0, (int)blockIdx.x};
+  const int i = S.blk * (int)blockDim.x + (int)threadIdx.x;
+  fx_float3 x = fx_float3{0.0f, 0.0f, 0.0f};
+  if (i < numPnts) x = advance_one(P, i, clock != nullptr ? clock[0] : time, dt, ss);
+  insert_at(P, S, x, true, tl);
+}
+
+extern "C" __global__ void advanceInsertBatch(BatchArgs B, const float* clock, float time) {
+  __shared__ uint tl[2][17];
+  const FParams_t* P;
+  const Span S = batch_span(B, blockIdx.x, P);
+  const int i = S.p0 + S.blk * (int)blockDim.x + (int)threadIdx.x;
+  fx_float3 x = fx_float3{0.0f, 0.0f, 0.0f};
+  if (i < S.p1) x = advance_one(*P, i, clock != nullptr ? clock[0] : time, P->dt, P->sim_scale);
+  insert_at(*P, S, x, true, tl);
 }
 
 extern "C" __global__ void advanceParticlesBatch(BatchArgs B, const float* clock, float time) {

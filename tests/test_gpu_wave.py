@@ -108,3 +108,40 @@ def test_stencils_in_a_batch(ps, gd):
             want = one.state()
         for k in ("press", "force", "pos", "vel", "veval"):
             assert bits_equal(got[k][p0:p0 + n], want[k]), (s, k)
+
+
+# Steps that run straight through share a pass between one step's advance and
+# the next one's insert: the same state, tables and ranks as single steps, in
+# one scene (with particles that leave the grid), in a batch and replayed.
+@pytest.mark.parametrize("n", [1, 63, 65, 257, 5003])
+@pytest.mark.parametrize("batch", [False, True])
+def test_joined_steps(ps, n, batch):
+    def restart():
+        if batch:
+            ps.RestartBatch([scenes.scaled_dam_break(n), scenes.scaled_dam_break(64), scenes.scaled_dam_break(n + 7)])
+        else:
+            ps.Restart(scenes.scaled_dam_break(n))
+        total = ps.NumPoints()
+        pos = ps.state()["pos"]
+        pos[:: 9] += 500.0
+        ps.Commit(abi.FPOS, pos)
+        ps.Commit(abi.FVEL, swirl(total, total))
+
+    states = []
+    for steps in ([1] * 5, [5], [2, 3], "graph"):
+        restart()
+        if steps == "graph":
+            ps.LaunchGraph(2)
+            ps.Run(1)
+        else:
+            for k in steps:
+                ps.Run(k)
+        states.append(ps.state())
+    for s in states[1:]:
+        for k in ("gcell", "gndx", "id", "cnt", "off"):
+            assert_int_equal(k, s[k], states[0][k])
+        m = valid_mask(states[0])
+        for k in ("press", "force"):
+            assert bits_equal(s[k][m], states[0][k][m]), k
+        for k in ("pos", "vel", "veval"):
+            assert bits_equal(s[k], states[0][k]), k
