@@ -17,7 +17,7 @@
 // step's slot order to the one before it.  For the length of a rollout the
 // particles are also numbered by their slot at its start (see adjFrameIn).
 // Memory: (segments
-// + 1) x 44 B x N of checkpoints plus every x (60 B x N + 8 B x cells +
+// + 1) x 44 B x N of checkpoints plus every x (60 B x N + 4 B x cells +
 // W x 4 B x N of neighbour bitmask, W sized from the densest stencil) of tape, twice when there is
 // more than one segment and the second buffer fits in 60 % of the free
 // device memory.
@@ -47,7 +47,6 @@ struct CkptPtr {
 struct TapeSrc {
   const void* v3[4];
   const void* s1[3];
-  const void* cnt;
   const void* off;
 };
 const int kAdjThreads = 64;   // ADJ_THREADS: one wave per block
@@ -65,7 +64,6 @@ struct AdjArgs {
   const void* rho;
   const void* id;
   const void* gcell;
-  const void* cnt;
   const void* off;
   const void* target;
   void* gx;
@@ -152,7 +150,7 @@ int Particles::AdjConfigure(const char* path, int nsteps, int every) {
   FX_HIP(hipStreamSynchronize(m_Stream), "adjoint");
   AdjRelease();
   const int n = mNumPoints;
-  const size_t tape_step = kTapeBytes * (size_t)n + 8 * (size_t)m_ScanCells;
+  const size_t tape_step = kTapeBytes * (size_t)n + 4 * (size_t)m_ScanCells;
   // Bitmask words per particle a tape slot holds: twice the densest stencil
   // of the current state (counts and offsets from an insert and scan, which
   // reorder nothing), at least 32 and at most FX_NBR_WORDS, a multiple of 4;
@@ -311,6 +309,9 @@ int Particles::AdjSetTarget(const float* target, int64_t count) {
   return FX_OK;
 }
 
+// bytes of a recorded step's tape slot
+size_t Particles::TapeStep() const { return kTapeBytes * (size_t)m_AdjN + 4 * (size_t)m_AdjCells; }
+
 int Particles::AdjLaunch(int fid, void* args, hipStream_t st) {
   if (m_AdjBlocks == 0) return FX_OK;
   void* a[] = {args};
@@ -340,37 +341,47 @@ int Particles::AdjRestoreCheckpoint(int k) {
   return FX_OK;
 }
 
-// One step (Particles::Run order); with record_slot >= 0 the step's sorted
-// state after the force stage goes to that tape slot.
-int Particles::AdjStep(int record_slot) {
-  FX_TRY(InsertParticles());
-  FX_TRY(PrefixScanParticles());
-  FX_TRY(CountingSort());
+// One step (Particles::Run order; first and last as in Particles::Step); with
+// record_slot >= 0 the step's sorted state after the force stage goes to that
+// tape slot.
+int Particles::AdjStep(int record_slot, bool first, bool last) {
+  const bool joined = JoinedSteps(), rec = record_slot >= 0, wave = WaveStages();
+  FX_TRY(SortStep(first || !joined));
   char* tabs = static_cast<char*>(m_AdjTabs);
-  if (record_slot >= 0) {  // the density kernel writes this step's bitmask into the tape, m_AdjWords a particle
+  const size_t n = (size_t)m_AdjN;
+  NbrBits bits;  // a recorded step's bitmask is written into the tape, m_AdjWords a particle
+  if (rec && wave) {
+    bits = {m_AdjBits + sizeof(uint32_t) * (size_t)m_AdjWords * n * (size_t)record_slot, m_AdjWords};
+  } else if (rec) {
     FX_HIP(hipMemcpyAsync(m_NbrWordsSym, m_AdjWordCaps + 1, sizeof(int), hipMemcpyDeviceToDevice, m_Stream), "tape");
     FX_HIP(hipMemcpyAsync(m_Accel.SymbolAddress(), tabs + sizeof(cuDataX) * (size_t)(record_slot + 1),
                           sizeof(cuDataX), hipMemcpyDeviceToDevice, m_Stream), "tape");
   }
-  FX_TRY(ComputePressure());
-  FX_TRY(ComputeForce());
-  if (record_slot >= 0) {
+  FX_TRY(ComputePressure(bits));
+  FX_TRY(ComputeForce(joined && !last, bits));
+  if (rec && !wave) {
     FX_HIP(hipMemcpyAsync(m_Accel.SymbolAddress(), tabs, sizeof(cuDataX), hipMemcpyDeviceToDevice, m_Stream),
            "tape");
     FX_HIP(hipMemcpyAsync(m_NbrWordsSym, m_AdjWordCaps, sizeof(int), hipMemcpyDeviceToDevice, m_Stream), "tape");
-    // pos, vel, veval, force, rho, id, gcell, then the cell counts and offsets: one kernel
-    const size_t n = (size_t)m_AdjN;
-    char* t = m_AdjTape + (kTapeBytes * n + 8 * (size_t)m_AdjCells) * (size_t)record_slot;
-    TapeSrc src = {{m_Points.gpu(FPOS), m_Points.gpu(FVEL), m_Points.gpu(FVEVAL), m_Points.gpu(FFORCE)},
-                   {m_Points.gpu(FPRESS), m_AdjSrc, m_Points.gpu(FGCELL)},
-                   m_Accel.gpu(AGRIDCNT),
-                   m_Accel.gpu(AGRIDOFF)};
-    int nn = m_AdjN, cells = m_AdjCells;
-    void* a[] = {&src, &t, &nn, &cells};
-    FX_TRY(launch_n(m_AdjFunc[ADJ_TAPE], kAdjNames[ADJ_TAPE], m_Stream, nn > cells ? nn : cells, a));
-    m_AdjTapeTime[record_slot] = m_Params.time;
   }
-  FX_TRY(Advance());
+  char* t = m_AdjTape + TapeStep() * (size_t)(rec ? record_slot : 0);
+  if (rec) m_AdjTapeTime[record_slot] = m_Params.time;
+  if (joined && !last) {
+    TapeSlot slot = {t, m_AdjSrc, m_AdjN, m_AdjCells};
+    FX_TRY(AdvanceInsert(rec ? &slot : nullptr));
+  } else {
+    if (rec) {
+      // pos, vel, veval, force, rho, permutation, gcell, then the cell offsets: one kernel
+      TapeSrc src = {{m_Points.gpu(FPOS), m_Points.gpu(FVEL), m_Points.gpu(FVEVAL), m_Points.gpu(FFORCE)},
+                     {m_Points.gpu(FPRESS), m_AdjSrc, m_Points.gpu(FGCELL)},
+                     m_Accel.gpu(AGRIDOFF)};
+      int nn = m_AdjN, cells = m_AdjCells;
+      void* a[] = {&src, &t, &nn, &cells};
+      FX_TRY(launch_n(m_AdjFunc[ADJ_TAPE], kAdjNames[ADJ_TAPE], m_Stream, nn > cells ? nn : cells, a));
+    }
+    FX_TRY(Advance());
+  }
+  m_Done = FX_STAGE_ADVANCE;
   AdvanceTime();
   return FX_OK;
 }
@@ -409,7 +420,8 @@ int Particles::AdjForward(double* loss, double* ms) {
   for (int t = 0; t < m_AdjSteps; t++) {
     const int seg = t / m_AdjEvery;
     if (t % m_AdjEvery == 0) FX_TRY(AdjSaveCheckpoint(seg));
-    FX_TRY(AdjStep(seg >= first_rec ? (seg % m_AdjBufs) * m_AdjTapeSteps + t - seg * m_AdjEvery : -1));
+    FX_TRY(AdjStep(seg >= first_rec ? (seg % m_AdjBufs) * m_AdjTapeSteps + t - seg * m_AdjEvery : -1, t == 0,
+                   t + 1 == m_AdjSteps));
   }
   for (int sg = first_rec < 0 ? 0 : first_rec; sg <= last; sg++) m_AdjBufSeg[sg % m_AdjBufs] = sg;
   FX_TRY(AdjSortSrc(false));
@@ -468,7 +480,7 @@ int Particles::AdjRecompute(int seg) {
   const int s0 = seg * m_AdjEvery;
   const int s1 = (s0 + m_AdjEvery < m_AdjSteps) ? s0 + m_AdjEvery : m_AdjSteps;
   m_AdjBufSeg[b] = -1;
-  for (int t = s0; t < s1; t++) FX_TRY(AdjStep(b * m_AdjTapeSteps + t - s0));
+  for (int t = s0; t < s1; t++) FX_TRY(AdjStep(b * m_AdjTapeSteps + t - s0, t == s0, t + 1 == s1));
   FX_HIP(hipEventRecord(m_AdjEv[b], m_Stream), "adjoint");
   m_AdjBufSeg[b] = seg;
   return FX_OK;
@@ -486,7 +498,7 @@ int Particles::AdjBackward(float* gpos, float* gvel, float* gveval, double* gvis
   }
   const size_t n = (size_t)m_AdjN;
   float* V = m_AdjVec;
-  const size_t tape_step = kTapeBytes * n + 8 * (size_t)m_AdjCells;
+  const size_t tape_step = TapeStep();
   // The adjoint kernels run on their own stream; the system stream
   // recomputes segment s-1 into the other tape buffer meanwhile.  Events:
   // [b] buffer b holds its segment, [2 + b] the adjoint reading buffer b is
@@ -526,8 +538,7 @@ int Particles::AdjBackward(float* gpos, float* gvel, float* gveval, double* gvis
       A.rho = T + 48 * n;
       A.id = T + 52 * n;
       A.gcell = T + 56 * n;
-      A.cnt = T + 60 * n;
-      A.off = T + 60 * n + 4 * (size_t)m_AdjCells;
+      A.off = T + 60 * n;
       A.target = V + 22 * n;
       A.gx = set[cur];
       A.gv = set[cur] + 3 * n;

@@ -71,7 +71,6 @@ struct AdjArgs {
   const float* rho;
   const uint* id;  // adjLoss: the final state's ids; the step kernels: the step's sort permutation src
   const int* gcell;
-  const uint* cnt;
   const uint* off;
   const fx_float3* target;  // by id (loss only)
   // adjoint state of the step's outputs (its sorted order) ...
@@ -206,13 +205,11 @@ extern "C" __global__ void adjUnframe(const fx_float3* g, fx_float3* out, const 
 
 // ------------------------------------------------------------------- tape
 // One recorded step's tape slot, written in one pass: pos, vel, veval, force
-// (12 B each), rho, id, gcell (4 B each) of the n particles, then the cell
-// counts and offsets of the cells-entry table, each array contiguous in that
-// order.  Thread a copies particle a and table entry a.
+// (12 B each), rho, id, gcell (4 B each) of the n particles, then the offsets
+// of the cells-entry table, each array contiguous in that order.  Thread a copies particle a and table entry a.
 struct TapeSrc {
   const fx_float3* v3[4];  // pos, vel, veval, force
   const uint* s1[3];       // rho (as bits), id, gcell
-  const uint* cnt;
   const uint* off;
 };
 
@@ -244,10 +241,7 @@ extern "C" __global__ void adjTapeRecord(TapeSrc S, char* dst, int n, int cells)
     for (int k = 0; k < 3; k++) reinterpret_cast<uint*>(dst + 48 * N + 4 * N * k)[a] = w[k];
   }
   if (a < cells) {
-    const uint c = S.cnt[a], o = S.off[a];
-    uint* t = reinterpret_cast<uint*>(dst + 60 * N);
-    t[a] = c;
-    t[(size_t)cells + a] = o;
+    reinterpret_cast<uint*>(dst + 60 * N)[a] = S.off[a];
   }
 }
 
@@ -453,19 +447,18 @@ __device__ __forceinline__ int wave_min_i(int v) {
 // Row r of the stencil at base: candidates [jb, je).  A row ends where the
 // cell after its last one begins (an in-range particle's row is followed by
 // a cell of the same grid row), so two loads, not three.
-__device__ __forceinline__ void row_of(const FParams_t& P, int base, int r, const uint* off, const uint* cnt,
-                                       int& jb, int& je) {
+__device__ __forceinline__ void row_of(const FParams_t& P, int base, int r, const uint* off, int& jb, int& je) {
   const int srch = P.gridSrch;
   const int c0 = base + P.gridAdj[r * srch];
   jb = (int)off[c0];
   je = (int)off[c0 + srch];
 }
 
-__device__ __forceinline__ int words_of(const FParams_t& P, int base, const uint* off, const uint* cnt) {
+__device__ __forceinline__ int words_of(const FParams_t& P, int base, const uint* off) {
   int w = 0;
   for (int r = 0; r < P.gridSrch * P.gridSrch; r++) {
     int jb, je;
-    row_of(P, base, r, off, cnt, jb, je);
+    row_of(P, base, r, off, jb, je);
     w += (je - jb + 31) >> 5;
   }
   return w;
@@ -495,7 +488,7 @@ __device__ __forceinline__ void ring_walk(const FParams_t& P, const AdjArgs& A, 
   };
   for (int r = 0; r < srch * srch; r++) {
     int jb = 0, je = 0;
-    if (use) row_of(P, base, r, A.off, A.cnt, jb, je);
+    if (use) row_of(P, base, r, A.off, jb, je);
     const int nw = (je - jb + 31) >> 5;
     const int maxw = min(wave_max_i(nw), A.ncap);
     for (int w = 0; w < maxw; w++) {
@@ -558,7 +551,7 @@ __device__ __forceinline__ bool queue_walk(const FParams_t& P, const AdjArgs& A,
 #pragma unroll
   for (int r = 0; r < R; r++) {
     int jb = 0, je = 0;
-    if (use) row_of(P, base, r, A.off, A.cnt, jb, je);
+    if (use) row_of(P, base, r, A.off, jb, je);
     G[r] = jb - (nwords << 5);
     nwords += (je - jb + 31) >> 5;
     E_[r] = nwords;
@@ -662,7 +655,7 @@ __device__ __forceinline__ bool pair_walk(const FParams_t& P, const AdjArgs& A, 
                                           uint* lq, Op& op) {
   if (P.gridSrch == 3) return queue_walk<3, K>(P, A, i, base, use, lq, op);
   if (P.gridSrch == 2) return queue_walk<2, K>(P, A, i, base, use, lq, op);
-  const bool over = use && words_of(P, base, A.off, A.cnt) > A.ncap;
+  const bool over = use && words_of(P, base, A.off) > A.ncap;
   ring_walk(P, A, i, base, use && !over, lq, op);
   return over;
 }
@@ -766,7 +759,7 @@ extern "C" __global__ void __launch_bounds__(ADJ_THREADS) AW_FORCE_ATTR adjForce
     const float rd2 = P.rd2;
     for (int r = 0; r < P.gridSrch * P.gridSrch; r++) {
       int jb, je;
-      row_of(P, base, r, A.off, A.cnt, jb, je);
+      row_of(P, base, r, A.off, jb, je);
       for (int j = jb; j < je; j++) {
         const float4 a = A.arec[3 * (size_t)j];
         const float dx = F.px - a.x, dy = F.py - a.y, dz = F.pz - a.z;
@@ -842,7 +835,7 @@ extern "C" __global__ void __launch_bounds__(ADJ_THREADS) adjDensity(AdjArgs A) 
   if (ovf) {  // no recorded bits: the candidates in place
     for (int r = 0; r < P.gridSrch * P.gridSrch; r++) {
       int jb, je;
-      row_of(P, base, r, A.off, A.cnt, jb, je);
+      row_of(P, base, r, A.off, jb, je);
       for (int j = jb; j < je; j++) {
         const float4 a = A.drec[j];
         const float dx = D.px - a.x, dy = D.py - a.y, dz = D.pz - a.z;

@@ -25,7 +25,8 @@ static const char* kKernelNames[FUNC_MAX] = {
     "computeForceBatchP", "advanceParticlesBatchP", "fxScanSums", "fxScanApply",
     "computePressureWave1", "computePressureWave2", "computePressureWave4",
     "computePressureWaveBatch1", "computePressureWaveBatch2", "computePressureWaveBatch4",
-    "computeForceWave",  "computeForceWaveBatch", "advanceInsert", "advanceInsertBatch"};
+    "computeForceWave",  "computeForceWaveBatch", "advanceInsert", "advanceInsertBatch",
+    "advanceInsertTape", "advanceInsertTapeBatch"};
 
 Particles::Particles() { memset(&m_Params, 0, sizeof(m_Params)); }
 
@@ -321,18 +322,20 @@ int Particles::BatchLaunch(int fid, int fid_p, int stage, void* extra0, void* ex
   return Launch(fid, grid, (unsigned)T, args);
 }
 
-int Particles::LaunchLanes(int fid, int fid_b, int threads, int lanes, unsigned lds, void* extra0, void* extra1) {
+int Particles::LaunchLanes(int fid, int fid_b, int threads, int lanes, unsigned lds, NbrBits b,
+                           void* extra0, void* extra1) {
   // a pair stage with `lanes` lanes to a particle, one launch over the scene
   // or over every scene of a batch
+  if (b.words == nullptr) b = {m_Accel.gpu(ANBRBITS), FX_NBR_WORDS};
   const int per = threads / lanes;
   if (!m_Batch) {
-    void* args[] = {&mNumPoints, extra0, extra1};
+    void* args[] = {&mNumPoints, &b.words, &b.cap, extra0, extra1};
     return Launch(fid, (unsigned)((mNumPoints + per - 1) / per), (unsigned)threads, args, lds);
   }
   const auto it = m_BTab.find(per);
   if (it == m_BTab.end()) return fx::fail(FX_ESTATE, "batch launch: no block table of %d particles", per);
   FxBatchArgs B{m_DParams, m_DPBase, m_DCBase, it->second.first, nullptr, it->second.second, 0};
-  void* args[] = {&B, &mNumPoints, extra0, extra1};
+  void* args[] = {&B, &mNumPoints, &b.words, &b.cap, extra0, extra1};
   return Launch(fid_b, (unsigned)it->second.second, (unsigned)threads, args, lds);
 }
 
@@ -649,10 +652,10 @@ int Particles::SortKernels() {
   return FX_OK;
 }
 
-int Particles::ComputePressure() {
+int Particles::ComputePressure(NbrBits bits) {
   if (WaveStages()) {
     const int lanes = DensityLanes(), t = StageThreads(FX_STAGE_PRESSURE, FX_DENS_THREADS), v = lanes == 4 ? 2 : lanes - 1;
-    FX_TRY(LaunchLanes(FUNC_PRESS_W + v, FUNC_PRESS_WB + v, t, lanes, FX_DENS_LDS(t)));
+    FX_TRY(LaunchLanes(FUNC_PRESS_W + v, FUNC_PRESS_WB + v, t, lanes, FX_DENS_LDS(t), bits));
   } else if (m_Batch) {
     FX_TRY(BatchLaunch(FUNC_PRESS_B, FUNC_PRESS_BP, FX_STAGE_PRESSURE, &mNumPoints, nullptr, nullptr));
   } else {
@@ -663,11 +666,11 @@ int Particles::ComputePressure() {
   return FX_OK;
 }
 
-int Particles::ComputeForce(bool clear) {
+int Particles::ComputeForce(bool clear, NbrBits bits) {
   if (WaveStages()) {
     const int t = StageThreads(FX_STAGE_FORCE, FX_FORCE_THREADS);
     void* cnt = clear ? m_Accel.gpu(AGRIDCNT) : nullptr;  // counts cleared for the next step's insert
-    FX_TRY(LaunchLanes(FUNC_FORCE_W, FUNC_FORCE_WB, t, 1, FX_FORCE_LDS(t), &cnt, &m_ScanCells));
+    FX_TRY(LaunchLanes(FUNC_FORCE_W, FUNC_FORCE_WB, t, 1, FX_FORCE_LDS(t), bits, &cnt, &m_ScanCells));
   } else if (m_Batch) {
     FX_TRY(BatchLaunch(FUNC_FORCE_B, FUNC_FORCE_BP, FX_STAGE_FORCE, &mNumPoints, nullptr, nullptr));
   } else {
@@ -744,11 +747,7 @@ bool Particles::JoinedSteps() const {
 // sort, as a step alone does.
 int Particles::Step(bool first, bool last) {
   const bool joined = JoinedSteps();
-  if (first || !joined) FX_TRY(InsertParticles());
-  FX_TRY(m_Points.SwapGPU(&m_PointsTemp));
-  m_Parity ^= 1;
-  FX_TRY(ScanGrid(true));
-  FX_TRY(SortKernels());
+  FX_TRY(SortStep(first || !joined));
   FX_TRY(ComputePressure());
   FX_TRY(ComputeForce(joined && !last));
   FX_TRY(joined && !last ? AdvanceInsert() : Advance());
@@ -756,9 +755,23 @@ int Particles::Step(bool first, bool last) {
   return FX_OK;
 }
 
-int Particles::AdvanceInsert() {
+// A step's insert (unless the step before it made it) to its sort.
+int Particles::SortStep(bool insert) {
+  if (insert) FX_TRY(InsertParticles());
+  FX_TRY(m_Points.SwapGPU(&m_PointsTemp));
+  m_Parity ^= 1;
+  FX_TRY(ScanGrid(true));
+  return SortKernels();
+}
+
+int Particles::AdvanceInsert(TapeSlot* tape) {
   float dt = m_Params.dt, ss = m_Params.sim_scale, time = m_Params.time;
   void* clk = m_Capturing ? (void*)m_Clock : nullptr;
+  if (tape != nullptr) {
+    if (m_Batch) return BatchLaunch(FUNC_ADVANCE_TAPE_B, 0, FX_STAGE_INSERT, &time, tape, nullptr);
+    void* args[] = {&time, &dt, &ss, &mNumPoints, tape};
+    return LaunchP(FUNC_ADVANCE_TAPE, FX_STAGE_INSERT, args);
+  }
   if (m_Batch) return BatchLaunch(FUNC_ADVANCE_INSERT_B, 0, FX_STAGE_INSERT, &clk, &time, nullptr);
   void* args[] = {&clk, &time, &dt, &ss, &mNumPoints};
   return LaunchP(FUNC_ADVANCE_INSERT, FX_STAGE_INSERT, args);

@@ -59,7 +59,9 @@
 #define FUNC_FORCE_WB 39
 #define FUNC_ADVANCE_INSERT 40  // a step's advance and the next one's insert
 #define FUNC_ADVANCE_INSERT_B 41
-#define FUNC_MAX 42
+#define FUNC_ADVANCE_TAPE 42    // the same, recording the step on a rollout's tape
+#define FUNC_ADVANCE_TAPE_B 43
+#define FUNC_MAX 44
 
 #include <map>
 #include <string>
@@ -74,6 +76,21 @@ struct FxBatchArgs {
   void* queue;  // claim counters of a persistent launch, else null
   int nitems;   // block-table entries
   int pad;
+};
+
+// Where the per-wave pair stages keep the neighbour bitmask, and how many
+// words a particle may record there; null: the system's own buffer.
+struct NbrBits {
+  void* words = nullptr;
+  int cap = 0;
+};
+
+// TapeDst of the kernel file: a recorded step's tape slot.
+struct TapeSlot {
+  void* dst;
+  const void* src;
+  int n;
+  int cells;
 };
 
 class Particles {
@@ -112,8 +129,9 @@ class Particles {
   int InsertParticles();
   int PrefixScanParticles();
   int CountingSort();
-  int ComputePressure();
-  int ComputeForce(bool clear = false);  // clear: zero the cell counts for an insert that follows (WaveStages only)
+  int ComputePressure(NbrBits bits = NbrBits());
+  // clear: zero the cell counts for an insert that follows (WaveStages only)
+  int ComputeForce(bool clear = false, NbrBits bits = NbrBits());
   int Advance();
   void AdvanceTime();
   int Stage(int stage);
@@ -173,7 +191,8 @@ class Particles {
   int PublishTables();
   bool JoinedSteps() const;
   int Step(bool first, bool last);
-  int AdvanceInsert();
+  int SortStep(bool insert);
+  int AdvanceInsert(TapeSlot* tape = nullptr);
   int SetDeviceClock();
   void ReleaseGraph();
   int BuildBlockTables();
@@ -181,8 +200,8 @@ class Particles {
   // entry, or its persistent variant fid_p (0: none) after resetting the
   // stage's claim counters
   int BatchLaunch(int fid, int fid_p, int stage, void* extra0, void* extra1, void* extra2);
-  int LaunchLanes(int fid, int fid_b, int threads, int lanes, unsigned lds, void* extra0 = nullptr,
-                  void* extra1 = nullptr);
+  int LaunchLanes(int fid, int fid_b, int threads, int lanes, unsigned lds, NbrBits bits,
+                  void* extra0 = nullptr, void* extra1 = nullptr);
   int DensityLanes() const;
   int StageThreads(int stage, int most) const;
   bool WaveStages() const;
@@ -193,7 +212,8 @@ class Particles {
   // adjoint helpers
   void AdjRelease();
   int AdjTables();
-  int AdjStep(int record_slot);
+  size_t TapeStep() const;
+  int AdjStep(int record_slot, bool first, bool last);
   int AdjCheckpointCopy(int k, int save);
   int AdjSaveCheckpoint(int k);
   int AdjRestoreCheckpoint(int k);
@@ -267,7 +287,7 @@ class Particles {
   std::vector<float> m_AdjCkptTime;      // checkpoint k = state before step k*every
   std::vector<float> m_AdjTapeTime;      // time of each recorded step of the segment
   char* m_AdjCkpt = nullptr;             // (segs+1) x 44 B x N
-  char* m_AdjTape = nullptr;             // every x (60 B x N + 8 B x cells)
+  char* m_AdjTape = nullptr;             // every x (60 B x N + 4 B x cells)
   char* m_AdjBits = nullptr;             // every x m_AdjWords x 4 B x N: each recorded step's bitmask
   int m_AdjWords = FX_NBR_WORDS;         // bitmask words a tape slot holds per particle
   int* m_AdjWordCaps = nullptr;          // device {FX_NBR_WORDS, m_AdjWords}: values copied into FNbrWords

@@ -1303,14 +1303,14 @@ __device__ __forceinline__ uint dens_word(uint acc, int n, int sub) {
 }
 
 template <int G, int SR>
-__device__ __forceinline__ void density_wave(const FParams_t& P, const Span S, int N, float* lds) {
+__device__ __forceinline__ void density_wave(const FParams_t& P, const Span S, int N, uint* __restrict__ bits, int cap,
+                                             float* lds) {
   constexpr int R = SR * SR;
   const int lane = (int)(threadIdx.x & 63u), sub = lane & (G - 1);
   const int i = S.p0 + (S.blk * (int)blockDim.x + (int)threadIdx.x) / G;
   float* tile = lds + (threadIdx.x >> 6) * (3 * FX_DENS_TILE);
   const fx_float3* __restrict__ pos = pbuf<const fx_float3>(FPnts, FPOS);
   const uint* __restrict__ off = pbuf<const uint>(FAccel, AGRIDOFF);
-  uint* __restrict__ bits = pbuf<uint>(FAccel, ANBRBITS);
   const int gc = i < S.p1 ? pbuf<const int>(FPnts, FGCELL)[i] : FX_GRID_UNDEF;
   const bool act = gc != FX_GRID_UNDEF;  // the in-range particles are the scene's first
   const unsigned long long am = __ballot(act);
@@ -1318,7 +1318,6 @@ __device__ __forceinline__ void density_wave(const FParams_t& P, const Span S, i
   const int lastl = 63 - __clzll((long long)am);
   const int shift = (P.gridRes.z + 1) * P.gridRes.x + 1;
   const size_t NN = (size_t)N;
-  const int cap = nbr_cap();
   const bool rec = act && sub == 0;  // the lane that writes the particle's words
   // Row r: the lane's candidates [jb, jb + len), the wave's run [lo, hi).  A
   // row ends where the cell after its last one begins.  Lanes past the last
@@ -1537,22 +1536,24 @@ __device__ __forceinline__ void density_wave(const FParams_t& P, const Span S, i
 extern __shared__ __align__(16) float dens_lds[];  // FX_DENS_LDS(threads) bytes
 
 template <int G>
-__device__ __forceinline__ void density_wave_any(const FParams_t& P, const Span S, int N) {
+__device__ __forceinline__ void density_wave_any(const FParams_t& P, const Span S, int N, uint* bits, int cap) {
   if (P.gridSrch == 3)
-    density_wave<G, 3>(P, S, N, dens_lds);
+    density_wave<G, 3>(P, S, N, bits, cap, dens_lds);
   else
-    density_wave<G, 2>(P, S, N, dens_lds);
+    density_wave<G, 2>(P, S, N, bits, cap, dens_lds);
 }
 
+// bits: cap words of bitmask a particle (the system's buffer, or a rollout's tape)
 #define FX_DENSITY_WAVE(G)                                                                                    \
-  extern "C" __global__ __launch_bounds__(FX_DENS_THREADS) void computePressureWave##G(int pnum) {            \
-    density_wave_any<G>(*cparams(&FParams), Span{0, pnum, 0, xcd_block()}, pnum);                             \
+  extern "C" __global__ __launch_bounds__(FX_DENS_THREADS) void computePressureWave##G(int pnum, uint* bits,  \
+                                                                                     int cap) {               \
+    density_wave_any<G>(*cparams(&FParams), Span{0, pnum, 0, xcd_block()}, pnum, bits, cap);                  \
   }                                                                                                           \
-  extern "C" __global__ __launch_bounds__(FX_DENS_THREADS) void computePressureWaveBatch##G(BatchArgs B,      \
-                                                                                          int ntotal) {       \
+  extern "C" __global__ __launch_bounds__(FX_DENS_THREADS) void computePressureWaveBatch##G(                  \
+      BatchArgs B, int ntotal, uint* bits, int cap) {                                                         \
     const FParams_t* P;                                                                                       \
     const Span S = batch_span(B, xcd_block(), P);                                                             \
-    density_wave_any<G>(*P, S, ntotal);                                                                       \
+    density_wave_any<G>(*P, S, ntotal, bits, cap);                                                            \
   }
 FX_DENSITY_WAVE(1)
 FX_DENSITY_WAVE(2)
@@ -2054,7 +2055,8 @@ extern "C" __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu
 #define FQ_STEP 4 // pairs a lane and step
 
 template <int SR>
-__device__ __forceinline__ void force_wave(const FParams_t& P, const Span S, int N, uint* lds) {
+__device__ __forceinline__ void force_wave(const FParams_t& P, const Span S, int N, const uint* __restrict__ bits,
+                                           int cap, uint* lds) {
   constexpr int R = SR * SR, MASK = FQ_K * 64 - 1;
   static_assert(R <= FQ_K, "a word of every row fits the queue");
   const int lane = (int)(threadIdx.x & 63u);
@@ -2064,7 +2066,6 @@ __device__ __forceinline__ void force_wave(const FParams_t& P, const Span S, int
   uint* qb = qw + FQ_K * 64;                                      // and where they begin
   const uint* __restrict__ off = pbuf<const uint>(FAccel, AGRIDOFF);
   const uint* __restrict__ cell = pbuf<const uint>(FAccel, AGRIDCNT);
-  const uint* __restrict__ bits = pbuf<const uint>(FAccel, ANBRBITS);
   const float4* __restrict__ fr = pbuf<const float4>(FAccel, AFREC);
   const float4* __restrict__ half = fr + (odd ? 1 : 0);  // the half of a record this lane reads
   const int gc = i < S.p1 ? pbuf<const int>(FPnts, FGCELL)[i] : FX_GRID_UNDEF;
@@ -2101,7 +2102,7 @@ __device__ __forceinline__ void force_wave(const FParams_t& P, const Span S, int
     nwords += (len + 31) >> 5;
     E_[r] = nwords;
   }
-  if (act && nwords > nbr_cap()) {  // no recorded bits: test every candidate
+  if (act && nwords > cap) {  // no recorded bits: test every candidate
     const int base = stencil_base(P, gc);
     for (int r = 0; r < R; r++) {
       int b, e;
@@ -2280,25 +2281,26 @@ __device__ __forceinline__ void clear_counts(uint* __restrict__ p, int n) {
   for (int k = (int)(blockIdx.x * blockDim.x + threadIdx.x); k < n; k += (int)(gridDim.x * blockDim.x)) p[k] = 0u;
 }
 
-__device__ __forceinline__ void force_wave_any(const FParams_t& P, const Span S, int N) {
+__device__ __forceinline__ void force_wave_any(const FParams_t& P, const Span S, int N, const uint* bits, int cap) {
   if (P.gridSrch == 3)
-    force_wave<3>(P, S, N, force_lds);
+    force_wave<3>(P, S, N, bits, cap, force_lds);
   else
-    force_wave<2>(P, S, N, force_lds);
+    force_wave<2>(P, S, N, bits, cap, force_lds);
 }
 
 // Bounds of 1024 threads, twice what is launched, keep the compiler's schedule
 // at four waves a SIMD: 280 instead of 260 us on the beach with 512.
-extern "C" __global__ __launch_bounds__(1024) void computeForceWave(int pnum, uint* clear, int nclear) {
-  force_wave_any(*cparams(&FParams), Span{0, pnum, 0, xcd_block()}, pnum);
+extern "C" __global__ __launch_bounds__(1024) void computeForceWave(int pnum, const uint* bits, int cap,
+                                                                           uint* clear, int nclear) {
+  force_wave_any(*cparams(&FParams), Span{0, pnum, 0, xcd_block()}, pnum, bits, cap);
   clear_counts(clear, nclear);
 }
 
-extern "C" __global__ __launch_bounds__(1024) void computeForceWaveBatch(BatchArgs B, int ntotal, uint* clear,
-                                                                                int nclear) {
+extern "C" __global__ __launch_bounds__(1024) void computeForceWaveBatch(BatchArgs B, int ntotal, const uint* bits,
+                                                                                int cap, uint* clear, int nclear) {
   const FParams_t* P;
   const Span S = batch_span(B, xcd_block(), P);
-  force_wave_any(*P, S, ntotal);
+  force_wave_any(*P, S, ntotal, bits, cap);
   clear_counts(clear, nclear);
 }
 
@@ -2650,6 +2652,64 @@ extern "C" __global__ void advanceInsertBatch(BatchArgs B, const float* clock, f
   const int i = S.p0 + S.blk * (int)blockDim.x + (int)threadIdx.x;
   fx_float3 x = fx_float3{0.0f, 0.0f, 0.0f};
   if (i < S.p1) x = advance_one(*P, i, clock != nullptr ? clock[0] : time, P->dt, P->sim_scale);
+  insert_at(*P, S, x, true, tl);
+}
+
+// The same in a recorded step of a rollout, whose particles (as they are
+// before the advance) and cell offsets also go to the tape, in the layout of
+// adjTapeRecord: pos, vel, veval, force (12 B each), rho, the sort's
+// permutation, cell (4 B each), then the offsets.  The pass reads most of it
+// already.  A rollout of 262,144 particles and its gradients take 12.1 instead
+// of 13.3 ms with this and the bitmask's place passed to the pair stages (it
+// was set by four copies a recorded step before), 12 scenes' 31.7 instead of
+// 32.8, one of 2,000 particles 0.57 instead of 0.61.
+struct TapeDst {
+  char* dst;
+  const uint* src;  // the sort's permutation
+  int n;
+  int cells;
+};
+
+__device__ __forceinline__ void tape_store(const TapeDst& T, int i, int end) {
+  const size_t N = (size_t)T.n;
+  if (i < end) {
+    const fx_float3 x = ld3(pbuf<const fx_float3>(FPnts, FPOS), (size_t)i);
+    const fx_float3 v = ld3(pbuf<const fx_float3>(FPnts, FVEL), (size_t)i);
+    const fx_float3 e = ld3(pbuf<const fx_float3>(FPnts, FVEVAL), (size_t)i);
+    const fx_float3 f = ld3(pbuf<const fx_float3>(FPnts, FFORCE), (size_t)i);
+    st3(reinterpret_cast<fx_float3*>(T.dst), (size_t)i, x.x, x.y, x.z);
+    st3(reinterpret_cast<fx_float3*>(T.dst + 12 * N), (size_t)i, v.x, v.y, v.z);
+    st3(reinterpret_cast<fx_float3*>(T.dst + 24 * N), (size_t)i, e.x, e.y, e.z);
+    st3(reinterpret_cast<fx_float3*>(T.dst + 36 * N), (size_t)i, f.x, f.y, f.z);
+    uint* w = reinterpret_cast<uint*>(T.dst + 48 * N);
+    w[i] = __float_as_uint(pbuf<const float>(FPnts, FPRESS)[i]);
+    w[N + i] = T.src[i];
+    w[2 * N + i] = pbuf<const uint>(FPnts, FGCELL)[i];
+  }
+  const uint* __restrict__ off = pbuf<const uint>(FAccel, AGRIDOFF);
+  uint* o = reinterpret_cast<uint*>(T.dst + 60 * N);
+  for (int k = (int)(blockIdx.x * blockDim.x + threadIdx.x); k < T.cells; k += (int)(gridDim.x * blockDim.x)) o[k] = off[k];
+}
+
+extern "C" __global__ void advanceInsertTape(float time, float dt, float ss, int numPnts, TapeDst T) {
+  __shared__ uint tl[2][17];
+  const FParams_t& P = *cparams(&FParams);
+  const Span S{0, numPnts, 0, (int)blockIdx.x};
+  const int i = S.blk * (int)blockDim.x + (int)threadIdx.x;
+  tape_store(T, i, numPnts);
+  fx_float3 x = fx_float3{0.0f, 0.0f, 0.0f};
+  if (i < numPnts) x = advance_one(P, i, time, dt, ss);
+  insert_at(P, S, x, true, tl);
+}
+
+extern "C" __global__ void advanceInsertTapeBatch(BatchArgs B, float time, TapeDst T) {
+  __shared__ uint tl[2][17];
+  const FParams_t* P;
+  const Span S = batch_span(B, blockIdx.x, P);
+  const int i = S.p0 + S.blk * (int)blockDim.x + (int)threadIdx.x;
+  tape_store(T, i, S.p1);
+  fx_float3 x = fx_float3{0.0f, 0.0f, 0.0f};
+  if (i < S.p1) x = advance_one(*P, i, time, P->dt, P->sim_scale);
   insert_at(*P, S, x, true, tl);
 }
 
