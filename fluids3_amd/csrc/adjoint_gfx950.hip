@@ -38,9 +38,12 @@
 #include <climits>
 
 #include "fluidsx_params.h"
+#include "fx_near.hpp"
 #include "fx_trig.hpp"
 
 typedef unsigned int uint;
+
+#include "fx_walk.hpp"
 
 #define ADJ_THREADS 64   // one wave per block
 #define RED_THREADS 256
@@ -421,28 +424,19 @@ extern "C" __global__ void __launch_bounds__(ADJ_THREADS) adjAdvance(AdjArgs A) 
   A.ges[s] = fx_float3{ex, ey, ez};
 }
 
-// ------------------------------------------------------- neighbour rings
+// -------------------------------------------------------- neighbour walks
 //
 // The recorded forward step's density kernel left, per particle, one bit per
 // stencil candidate (set for the in-radius pairs; row r occupies a
 // word-aligned run of ceil(len/32) words at [w * N + i]).  Both pair kernels
-// below turn those bits into neighbour indices in a per-lane ring in LDS and
-// evaluate queued pairs in wave-wide batches (every lane takes as many pairs
-// as the shortest active queue holds), so the pair arithmetic runs with
-// nearly all lanes busy and no candidate is tested twice.  Each lane visits
-// its pairs in candidate order (the order of the CPU oracle's loops).  One
-// wave per block; a particle whose candidates needed more than ncap
-// words has no bits and tests its candidates in place.
+// below take their pairs from those bits: with fx_walk.hpp's queue of words
+// for stencil rows of 2 and 3 cells; for rows of 4 by turning the bits into
+// neighbour indices in a per-lane ring in LDS, evaluated in wave-wide batches
+// (every lane takes as many pairs as the shortest active queue holds).  Each
+// lane visits its pairs in candidate order (the order of the CPU oracle's
+// loops).  One wave per block; a particle whose candidates needed more than
+// ncap words has no bits and tests its candidates in place.
 #define AQ_SLOTS 1024  // ring slots per block: 16 per lane
-
-__device__ __forceinline__ int wave_max_i(int v) {
-  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-  return v;
-}
-__device__ __forceinline__ int wave_min_i(int v) {
-  for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
-  return v;
-}
 
 // Row r of the stencil at base: candidates [jb, je).  A row ends where the
 // cell after its last one begins (an in-range particle's row is followed by
@@ -490,7 +484,7 @@ __device__ __forceinline__ void ring_walk(const FParams_t& P, const AdjArgs& A, 
     int jb = 0, je = 0;
     if (use) row_of(P, base, r, A.off, jb, je);
     const int nw = (je - jb + 31) >> 5;
-    const int maxw = min(wave_max_i(nw), A.ncap);
+    const int maxw = min(wave_max(nw), A.ncap);
     for (int w = 0; w < maxw; w++) {
       uint word = 0;
       if (w < nw) word = A.bits[(size_t)(W + w) * NN + i];
@@ -498,8 +492,8 @@ __device__ __forceinline__ void ring_walk(const FParams_t& P, const AdjArgs& A, 
         uint m = (word >> h) & 0xffffu;
         const int pc = __popc(m);
         if (__any(qn + pc > fqn)) {
-          const int need = wave_max_i(qn + pc - fqn);
-          drain(min(max(need, wave_min_i(use ? qn : 0x7fffffff)), fqn));
+          const int need = wave_max(qn + pc - fqn);
+          drain(min(max(need, wave_min(use ? qn : 0x7fffffff)), fqn));
         }
         int tail = head + qn;
         if (tail >= fqn) tail -= fqn;
@@ -514,155 +508,71 @@ __device__ __forceinline__ void ring_walk(const FParams_t& P, const AdjArgs& A, 
     }
     W += nw;
   }
-  drain(min(wave_max_i(qn), fqn));
+  drain(min(wave_max(qn), fqn));
 }
 
-// Walks the lane's recorded pairs through a word queue: each lane reads its
-// bitmask words as one stream (row r's words follow row r-1's) and queues
-// every non-zero word whole, with the record index of its bit 0 -- two words
-// in registers, up to AW_QWORDS more in LDS; the wave then takes the same
-// number of pairs from every lane (as many as the shortest queue holds, more
-// only when a queue must make room), AW_STEP per step, each lane's in candidate
-// order.  Same contract as ring_walk; for stencil rows of SR cells, K LDS
-// words per lane (8 K bytes per block).
-#ifndef AW_QF
-#define AW_QF 8   // LDS words per lane in the force adjoint
-#endif
-#ifndef AW_QD
-#define AW_QD 8   // and in the density adjoint
-#endif
-#ifndef AW_STEP
-#define AW_STEP 3  // pairs taken per drain step
-#endif
-#ifndef AW_FORCE_ATTR
-#define AW_FORCE_ATTR
-#endif
-
-template <int SR, int K, class Op>
-__device__ __forceinline__ bool queue_walk(const FParams_t& P, const AdjArgs& A, int i, int base, bool use,
-                                           uint* lq, Op& op) {
+// Walks the recorded pairs of a wave's particles (i and its cell gc a lane,
+// act where it has one) with word_walk, for stencil rows of SR cells.  Same
+// contract as ring_walk; returns whether the lane's rows need more bitmask
+// words than a tape slot holds (then it recorded no bits, and nothing was
+// walked for it).
+template <int SR, class Op>
+__device__ __forceinline__ bool row_walk(const FParams_t& P, const AdjArgs& A, int i, int base, bool act, uint* lq,
+                                         Op& op) {
   constexpr int R = SR * SR;
-  const int t = threadIdx.x;
-  const size_t NN = (size_t)A.nbits;
-  // row r covers words [W_r, W_{r+1}) of the lane's bitmask; E_[r] = W_{r+1},
-  // and the record of word f, bit b is G[r] + 32 f + b
-  int E_[R], G[R];
-  int nwords = 0;
+  int jb[R], E_[R];  // row r: candidates from jb[r], words [E_[r - 1], E_[r]) of the bitmask
+#pragma unroll
+  for (int r = 0; r < R; r++) jb[r] = E_[r] = 0;
+  if (act) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int c0 = base + P.gridAdj[r * SR];
+      jb[r] = (int)A.off[c0];
+      E_[r] = (int)A.off[c0 + SR];
+    }
+  }
+  int nwords = 0, longest = 0;
 #pragma unroll
   for (int r = 0; r < R; r++) {
-    int jb = 0, je = 0;
-    if (use) row_of(P, base, r, A.off, jb, je);
-    G[r] = jb - (nwords << 5);
-    nwords += (je - jb + 31) >> 5;
+    const int len = E_[r] - jb[r];
+    longest = max(longest, len);
+    nwords += (len + 31) >> 5;
     E_[r] = nwords;
   }
-  // a lane whose rows need more words than a tape slot holds recorded none
-  // of them: it walks nothing here
-  const bool over = use && nwords > A.ncap;
+  const bool over = act && nwords > A.ncap;
   if (over) {
     nwords = 0;
 #pragma unroll
-    for (int r = 0; r < R; r++) E_[r] = G[r] = 0;
+    for (int r = 0; r < R; r++) E_[r] = 0;
   }
-  use = use && !over;
-  uint* Qw = lq;
-  uint* Qb = lq + K * 64;
-  uint cur = 0u, nxt = 0u;
-  int curb = 0, nxtb = 0, qh = 0, qc = 0, qn = 0;
-  auto take = [&](uint& j) -> bool {
-    const bool ok = cur != 0u;
-    j = ok ? (uint)(curb + __builtin_ctz(cur)) : 0u;
-    cur &= cur - 1u;
-    if (ok && cur == 0u) {
-      cur = nxt;
-      curb = nxtb;
-      nxt = 0u;
-      if (qc > 0) {
-        nxt = Qw[qh * 64 + t];
-        nxtb = (int)Qb[qh * 64 + t];
-        qh = (qh + 1 == K) ? 0 : qh + 1;
-        qc--;
-      }
-    }
-    return ok;
-  };
-  auto drain = [&](int f) {
-    int e = 0;
-    for (; e + AW_STEP <= f; e += AW_STEP) {
-      uint j[AW_STEP];
-      bool ok[AW_STEP];
-      typename Op::Rec rc[AW_STEP];
-#pragma unroll
-      for (int u = 0; u < AW_STEP; u++) ok[u] = take(j[u]);
-#pragma unroll
-      for (int u = 0; u < AW_STEP; u++) rc[u] = op.load(j[u]);  // every gather of the step first
-#pragma unroll
-      for (int u = 0; u < AW_STEP; u++) op.apply(rc[u], ok[u]);
-    }
-    for (; e < f; e++) {
-      uint j;
-      const bool ok = take(j);
-      op.eval(j, ok);
-    }
-    qn = max(qn - f, 0);
-  };
-  const int maxf = wave_max_i(nwords);
-  for (int f = 0; f < maxf; f++) {
-    const uint word = f < nwords ? A.bits[(size_t)f * NN + i] : 0u;
-    if (word != 0u) {
-      while (f >= E_[0]) {  // move to the row holding word f
-#pragma unroll
-        for (int r = 0; r < R - 1; r++) {
-          E_[r] = E_[r + 1];
-          G[r] = G[r + 1];
-        }
-        E_[R - 1] = INT_MAX;
-      }
-    }
-    const int held = (cur != 0u ? 1 : 0) + (nxt != 0u ? 1 : 0) + qc;
-    const bool full = word != 0u && held == K + 2;
-    if (__any(full)) {  // free a word slot: the full lanes finish their current word
-      const int need = wave_max_i(full ? __popc(cur) : 0);
-      drain(max(need, wave_min_i(use ? qn : 0x7fffffff)));
-    }
-    if (word != 0u) {
-      const int wb = G[0] + (f << 5);
-      if (cur == 0u) {
-        cur = word;
-        curb = wb;
-      } else if (nxt == 0u) {
-        nxt = word;
-        nxtb = wb;
-      } else {
-        int tl = qh + qc;
-        if (tl >= K) tl -= K;
-        Qw[tl * 64 + t] = word;
-        Qb[tl * 64 + t] = (uint)wb;
-        qc++;
-      }
-      qn += __popc(word);
-    }
-  }
-  drain(wave_max_i(qn));
+  word_walk<R, Op::MUL, Op::STEP>(A.bits, (size_t)A.nbits, i, nwords, longest, jb, E_, lq + threadIdx.x,
+                                  [&](const uint (&j)[Op::STEP], const bool (&ok)[Op::STEP])
+                                      __attribute__((always_inline)) { op.step(j, ok); });
   return over;
 }
 
 // Stencil rows of 2 or 3 cells through the word queue, 4 through the ring.
-// Returns whether the lane's rows need more bitmask words than a tape slot
-// holds (then it recorded no bits, and nothing was walked for it).
-template <int K, class Op>
-__device__ __forceinline__ bool pair_walk(const FParams_t& P, const AdjArgs& A, int i, int base, bool use,
+template <class Op>
+__device__ __forceinline__ bool pair_walk(const FParams_t& P, const AdjArgs& A, int i, int base, bool act,
                                           uint* lq, Op& op) {
-  if (P.gridSrch == 3) return queue_walk<3, K>(P, A, i, base, use, lq, op);
-  if (P.gridSrch == 2) return queue_walk<2, K>(P, A, i, base, use, lq, op);
-  const bool over = use && words_of(P, base, A.off) > A.ncap;
-  ring_walk(P, A, i, base, use && !over, lq, op);
+  if (P.gridSrch == 3) return row_walk<3>(P, A, i, base, act, lq, op);
+  if (P.gridSrch == 2) return row_walk<2>(P, A, i, base, act, lq, op);
+  const bool over = act && words_of(P, base, A.off) > A.ncap;
+  ring_walk(P, A, i, base, act && !over, lq, op);
   return over;
 }
+
+// LDS of a block (one wave): the word queue, or the ring
+#define ADJ_LDS_WORDS (2 * FX_WALK_K * 64 > AQ_SLOTS ? 2 * FX_WALK_K * 64 : AQ_SLOTS)
 
 // ------------------------------------------------------------------ force
 
 // Pair term of the force adjoint; same expression tree as the CPU oracle.
+// About 85 instructions a pair, and the walk's 30: VALU issue bounds it.  The
+// gathers (three 16-byte records a pair, two of them read by neighbouring
+// lanes together) and the roots are the forward force's.  Per launch, with a
+// queue that read its words when it needed them, plain gathers and IEEE roots
+// before / now: 262,144 particles 49 / 41 us, 12 scenes 158 / 146.
 struct ForceAdj {
   const FParams_t* P;
   const float4* rec;  // (pos, rho), (veval, 0), (gF, 0) per slot
@@ -670,23 +580,72 @@ struct ForceAdj {
   float kp, stiff, vterm, lap, h, rest, d2;
   float gpx, gpy, gpz, gex, gey, gez, gr, ak, av;
 
-  // the pair's records (load), then its terms added in order (apply)
+  static constexpr uint MUL = 3;  // records of a slot
+  static constexpr int STEP = 4;  // 2, 3 and 4 measure the same at 262,144 particles, 13.1 / 12.3 / 12.0 us at 2,000
   struct Rec {
     float4 a, v, q;
   };
-  __device__ __forceinline__ Rec load(uint j) const {
-    return Rec{rec[3 * (size_t)j], rec[3 * (size_t)j + 1], rec[3 * (size_t)j + 2]};
+  // 1 / (r rho_i rho_j) and r; Near: by near_sqrt and near_rcp, chk >= FX_NEAR_SPAN where they may not be exact
+  template <bool Near>
+  __device__ __forceinline__ void roots(const float4& a, float& rr, float& inv, uint& chk) const {
+    const float dx = px - a.x, dy = py - a.y, dz = pz - a.z;
+    const float r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx)) * d2;
+    rr = Near ? near_sqrt(r2) : sqrtf(r2);
+    const float den = rr * (di * a.w);
+    inv = Near ? near_rcp(den) : 1.0f / den;
+    if (Near) chk |= near_bits(r2) | near_bits(den);
   }
-  __device__ __forceinline__ void eval(uint j, bool ok) { apply(load(j), ok); }
-  __device__ __forceinline__ void apply(const Rec& r, bool ok) {
+  __device__ __forceinline__ void eval(uint j, bool ok) {
+    const Rec r{rec[3 * (size_t)j], rec[3 * (size_t)j + 1], rec[3 * (size_t)j + 2]};
+    float rr, inv;
+    uint chk;
+    roots<false>(r.a, rr, inv, chk);
+    apply<true>(r, rr, inv, ok);
+  }
+  // STEP pairs, each lane's in order; neighbouring lanes read the first two
+  // records of a slot together (see the forward force)
+  __device__ __forceinline__ void step(const uint (&j)[STEP], const bool (&ok)[STEP]) {
+    const bool odd = (threadIdx.x & 1u) != 0u;
+    const float4* __restrict__ half = rec + (odd ? 1 : 0);
+    float4 e[STEP];
+    Rec r[STEP];
+#pragma unroll
+    for (int u = 0; u < STEP; u++) {
+      const uint jx = lane_other(j[u]);
+      e[u] = half[odd ? jx : j[u]];
+      r[u].v = half[odd ? j[u] : jx];
+      r[u].q = rec[j[u] + 2u];
+    }
+    float rr[STEP], inv[STEP];
+    uint chk = 0u;
+#pragma unroll
+    for (int u = 0; u < STEP; u++) {
+      swap_halves(e[u], r[u].v, r[u].a);
+      roots<true>(r[u].a, rr[u], inv[u], chk);
+    }
+    if (__any(chk >= FX_NEAR_SPAN)) {
+#pragma unroll
+      for (int u = 0; u < STEP; u++) roots<false>(r[u].a, rr[u], inv[u], chk);
+    }
+    bool every = true;
+#pragma unroll
+    for (int u = 0; u < STEP; u++) every = every && ok[u];
+    if (__all(every)) {
+#pragma unroll
+      for (int u = 0; u < STEP; u++) apply<false>(r[u], rr[u], inv[u], true);
+    } else {
+#pragma unroll
+      for (int u = 0; u < STEP; u++) apply<true>(r[u], rr[u], inv[u], ok[u]);
+    }
+  }
+  // adds the pair's terms (where ok, if Pad)
+  template <bool Pad>
+  __device__ __forceinline__ void apply(const Rec& r, float rr, float inv, bool ok) {
     const float4 a = r.a, v = r.v, q = r.q;
     const float dx = px - a.x, dy = py - a.y, dz = pz - a.z;
-    const float dsq = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-    const float rr = sqrtf(dsq * d2);
     const float c = h - rr;
     const float dj = a.w;
     const float pj = (dj - rest) * stiff;
-    const float inv = 1.0f / (rr * (di * dj));
     const float invd = inv * rr;
     const float ir = inv * (di * dj);
     const float kc2i = (kp * (c * c)) * inv;
@@ -711,7 +670,7 @@ struct ForceAdj {
     const float n_gr = fmaf(kc2i * stiff, su, gr) - fmaf(Ac, su, Bc * sv) * idi;
     const float n_ak = fmaf(kc2i * (qi + (dj - rest)), ui, ak);
     const float n_av = fmaf((lap * c) * invd, wi, av);
-    if (ok) {
+    if (!Pad || ok) {
       gpx = n_gpx; gpy = n_gpy; gpz = n_gpz;
       gex = n_gex; gey = n_gey; gez = n_gez;
       gr = n_gr; ak = n_ak; av = n_av;
@@ -719,8 +678,8 @@ struct ForceAdj {
   }
 };
 
-extern "C" __global__ void __launch_bounds__(ADJ_THREADS) AW_FORCE_ATTR adjForce(AdjArgs A) {
-  __shared__ uint fq[(2 * AW_QF * 64 > AQ_SLOTS) ? 2 * AW_QF * 64 : AQ_SLOTS];
+extern "C" __global__ void __launch_bounds__(ADJ_THREADS) adjForce(AdjArgs A) {
+  __shared__ uint fq[ADJ_LDS_WORDS];
   const Slot S = slot_of(A);
   const FParams_t& P = *S.P;
   const int i = S.i;
@@ -754,7 +713,7 @@ extern "C" __global__ void __launch_bounds__(ADJ_THREADS) AW_FORCE_ATTR adjForce
   }
   // a particle without recorded bits tests its candidates in place, in the
   // same candidate order (after the walk, which took none of its pairs)
-  const bool ovf = pair_walk<AW_QF>(P, A, i, base, act, fq, F);
+  const bool ovf = pair_walk(P, A, i, base, act, fq, F);
   if (ovf) {
     const float rd2 = P.rd2;
     for (int r = 0; r < P.gridSrch * P.gridSrch; r++) {
@@ -788,18 +747,26 @@ extern "C" __global__ void __launch_bounds__(ADJ_THREADS) AW_FORCE_ATTR adjForce
 
 // ---------------------------------------------------------------- density
 
+// Pair term of the density adjoint: about 15 instructions a pair beside the
+// walk's 20, and one 16-byte gather; the gathers in flight bound it, hence
+// eight to a step.  Per launch before / now (the queue as above): 262,144
+// particles 28 / 18 us, 12 scenes 70 / 63.
 struct DensityAdj {
   const float4* rec;  // (pos, grho) per slot
   float px, py, pz, gi, d2, rd2, k6;
   float gpx, gpy, gpz;
 
-  struct Rec {
-    float4 a;
-  };
-  __device__ __forceinline__ Rec load(uint j) const { return Rec{rec[j]}; }
-  __device__ __forceinline__ void eval(uint j, bool ok) { apply(load(j), ok); }
-  __device__ __forceinline__ void apply(const Rec& r, bool ok) {
-    const float4 a = r.a;
+  static constexpr uint MUL = 1;
+  static constexpr int STEP = 8;  // 4 / 6 / 8: 18.7 / 18.3 / 18.1 us at 262,144 particles, 68 / 64 / 63 for 12 scenes
+  __device__ __forceinline__ void eval(uint j, bool ok) { apply(rec[j], ok); }
+  __device__ __forceinline__ void step(const uint (&j)[STEP], const bool (&ok)[STEP]) {
+    float4 a[STEP];
+#pragma unroll
+    for (int u = 0; u < STEP; u++) a[u] = rec[j[u]];
+#pragma unroll
+    for (int u = 0; u < STEP; u++) apply(a[u], ok[u]);
+  }
+  __device__ __forceinline__ void apply(const float4& a, bool ok) {
     const float dx = px - a.x, dy = py - a.y, dz = pz - a.z;
     const float dsq = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
     const float t = (rd2 - dsq) * d2;
@@ -812,7 +779,7 @@ struct DensityAdj {
 };
 
 extern "C" __global__ void __launch_bounds__(ADJ_THREADS) adjDensity(AdjArgs A) {
-  __shared__ uint fq[(2 * AW_QD * 64 > AQ_SLOTS) ? 2 * AW_QD * 64 : AQ_SLOTS];
+  __shared__ uint fq[ADJ_LDS_WORDS];
   const Slot S = slot_of(A);
   const FParams_t& P = *S.P;
   const int i = S.i;
@@ -831,7 +798,7 @@ extern "C" __global__ void __launch_bounds__(ADJ_THREADS) adjDensity(AdjArgs A) 
     D.px = a.x; D.py = a.y; D.pz = a.z;
     D.gi = a.w;
   }
-  const bool ovf = pair_walk<AW_QD>(P, A, i, base, act, fq, D);
+  const bool ovf = pair_walk(P, A, i, base, act, fq, D);
   if (ovf) {  // no recorded bits: the candidates in place
     for (int r = 0; r < P.gridSrch * P.gridSrch; r++) {
       int jb, je;

@@ -23,6 +23,7 @@
 
 #include "fluidsx_params.h"
 #include "fx_near.hpp"
+#include "fx_walk.hpp"
 #include "fx_trig.hpp"
 
 typedef unsigned int uint;
@@ -136,27 +137,6 @@ __device__ __forceinline__ uint wave_inclusive_scan(uint v) {
   v += t;
   return v;
 }
-
-// Wave-wide max / min with the same DPP pattern; lane 63 ends up with the
-// reduction of all 64 lanes and is read back as a scalar.
-template <bool kMax>
-__device__ __forceinline__ int wave_reduce(int v) {
-  const int id = kMax ? INT_MIN : INT_MAX;
-  int t;
-#define FX_RED_STEP(ctrl, rmask)                                    \
-  t = __builtin_amdgcn_update_dpp(id, v, ctrl, rmask, 0xf, false); \
-  v = kMax ? max(v, t) : min(v, t);
-  FX_RED_STEP(0x111, 0xf)  // row_shr:1
-  FX_RED_STEP(0x112, 0xf)  // row_shr:2
-  FX_RED_STEP(0x114, 0xf)  // row_shr:4
-  FX_RED_STEP(0x118, 0xf)  // row_shr:8
-  FX_RED_STEP(0x142, 0xa)  // row_bcast:15
-  FX_RED_STEP(0x143, 0xc)  // row_bcast:31
-#undef FX_RED_STEP
-  return __builtin_amdgcn_readlane(v, 63);
-}
-__device__ __forceinline__ int wave_max(int v) { return wave_reduce<true>(v); }
-__device__ __forceinline__ int wave_min(int v) { return wave_reduce<false>(v); }
 
 // Block barrier that orders LDS accesses only: global loads and atomics
 // already in flight stay in flight across it (a __syncthreads() would first
@@ -2051,19 +2031,16 @@ extern "C" __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu
 // 1857, 4830 and 284 (at FQ_STEP 3).  117 VGPRs, four waves a SIMD; held at
 // 96 it spills (2250 us).  VALU issue bounds it (about 52 instructions a
 // pair and lane) with the gathers' latency beside it.
-#define FQ_K 16   // queued words a lane (FX_FORCE_LDS); a power of two
 #define FQ_STEP 4 // pairs a lane and step
 
 template <int SR>
 __device__ __forceinline__ void force_wave(const FParams_t& P, const Span S, int N, const uint* __restrict__ bits,
                                            int cap, uint* lds) {
-  constexpr int R = SR * SR, MASK = FQ_K * 64 - 1;
-  static_assert(R <= FQ_K, "a word of every row fits the queue");
+  constexpr int R = SR * SR;
   const int lane = (int)(threadIdx.x & 63u);
   const bool odd = (lane & 1) != 0;
   const int i = S.p0 + S.blk * (int)blockDim.x + (int)threadIdx.x;
-  uint* qw = lds + (threadIdx.x >> 6) * (2 * FQ_K * 64) + lane;  // words, 64 apart
-  uint* qb = qw + FQ_K * 64;                                      // and where they begin
+  uint* q = lds + (threadIdx.x >> 6) * (2 * FX_WALK_K * 64) + lane;
   const uint* __restrict__ off = pbuf<const uint>(FAccel, AGRIDOFF);
   const uint* __restrict__ cell = pbuf<const uint>(FAccel, AGRIDCNT);
   const float4* __restrict__ fr = pbuf<const float4>(FAccel, AFREC);
@@ -2116,157 +2093,37 @@ __device__ __forceinline__ void force_wave(const FParams_t& P, const Span S, int
 #pragma unroll
     for (int r = 0; r < R; r++) E_[r] = 0;
   }
-  const size_t NN = (size_t)N;
-  // the current word and what its bit 0 stands for, in half records; the
-  // queue's first two (0 where it holds fewer)
-  uint cur = 0u, curb = 0u, n1 = 0u, n1b = 0u, n2 = 0u, n2b = 0u;
-  int head = 0, cnt = 0;  // of the queue, n1 and n2 included
-  int qn = 0;             // pairs held
-  auto ahead = [&]() {
-    const int h2 = (head + 64) & MASK;
-    n1 = qw[head];
-    n1b = qb[head];
-    n2 = qw[h2];
-    n2b = qb[h2];
-    n1 = cnt > 0 ? n1 : 0u;
-    n2 = cnt > 1 ? n2 : 0u;
-  };
-  // FQ_STEP pairs from every lane (a lane that has none left evaluates record
-  // 0 and discards it), each lane's in candidate order
-  auto step = [&]() {
-    uint j[FQ_STEP];
-    bool ok[FQ_STEP];
-    const int have = min(cnt, 2);
-#pragma unroll
-    for (int u = 0; u < FQ_STEP; u++) {
-      ok[u] = cur != 0u;
-      j[u] = ok[u] ? curb + 2u * (uint)__builtin_ctz(cur) : 0u;
-      const uint rest = cur & (cur - 1u);
-      const bool next = rest == 0u;
-      cur = next ? n1 : rest;
-      curb = next ? n1b : curb;
-      n1 = next ? n2 : n1;
-      n1b = next ? n2b : n1b;
-      n2 = next ? 0u : n2;
-      qn -= ok[u] ? 1 : 0;
-    }
-    const int used = have - (n1 != 0u ? 1 : 0) - (n2 != 0u ? 1 : 0);
-    cnt -= used;
-    head = (head + 64 * used) & MASK;
-    ahead();
+  word_walk<R, 2, FQ_STEP>(bits, (size_t)N, i, nwords, longest, jb, E_, q, [&](const uint (&j)[FQ_STEP], const bool (&ok)[FQ_STEP]) __attribute__((always_inline)) {
     float4 e[FQ_STEP], o[FQ_STEP];  // this lane's half of the even lane's record, and of the odd lane's
 #pragma unroll
     for (int u = 0; u < FQ_STEP; u++) {
-      const uint jx = __builtin_amdgcn_update_dpp(0u, j[u], 0xB1, 0xf, 0xf, true);  // quad_perm 1,0,3,2
+      const uint jx = lane_other(j[u]);
       e[u] = half[odd ? jx : j[u]];
       o[u] = half[odd ? j[u] : jx];
     }
-    PairTerm q[FQ_STEP];
+    PairTerm t[FQ_STEP];
     float4 a[FQ_STEP];
     uint chk = 0u;
 #pragma unroll
     for (int u = 0; u < FQ_STEP; u++) {
-      // a, the (pos, rho) half: an even lane's e, an odd lane takes the even
-      // lane's o.  o becomes the (veval, 0) half: an odd lane's own, an even
-      // lane takes the odd lane's e.  Every lane of the wave runs this; a DPP
-      // source needs two cycles after a VALU write of it.
-      __asm__("s_nop 1\n\ts_mov_b64 vcc, %8\n\t"
-              "v_cndmask_b32_dpp %0, %4, %9, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-              "v_cndmask_b32_dpp %1, %5, %10, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-              "v_cndmask_b32_dpp %2, %6, %11, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-              "v_cndmask_b32_dpp %3, %7, %12, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
-              : "=&v"(a[u].x), "=&v"(a[u].y), "=&v"(a[u].z), "=&v"(a[u].w)
-              : "v"(o[u].x), "v"(o[u].y), "v"(o[u].z), "v"(o[u].w), "s"(0x5555555555555555ull), "v"(e[u].x),
-                "v"(e[u].y), "v"(e[u].z), "v"(e[u].w)
-              : "vcc");
-      __asm__("s_nop 1\n\ts_mov_b64 vcc, %6\n\t"
-              "v_cndmask_b32_dpp %0, %3, %0, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-              "v_cndmask_b32_dpp %1, %4, %1, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-              "v_cndmask_b32_dpp %2, %5, %2, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
-              : "+v"(o[u].x), "+v"(o[u].y), "+v"(o[u].z)
-              : "v"(e[u].x), "v"(e[u].y), "v"(e[u].z), "s"(0xAAAAAAAAAAAAAAAAull)
-              : "vcc");
-      q[u] = pair_term<true>(P, I, a[u], o[u], chk);
+      swap_halves(e[u], o[u], a[u]);
+      t[u] = pair_term<true>(P, I, a[u], o[u], chk);
     }
     if (__any(chk >= FX_NEAR_SPAN)) {
 #pragma unroll
-      for (int u = 0; u < FQ_STEP; u++) q[u] = pair_term<false>(P, I, a[u], o[u], chk);
+      for (int u = 0; u < FQ_STEP; u++) t[u] = pair_term<false>(P, I, a[u], o[u], chk);
     }
     bool every = true;
 #pragma unroll
     for (int u = 0; u < FQ_STEP; u++) every = every && ok[u];
     if (__all(every)) {
 #pragma unroll
-      for (int u = 0; u < FQ_STEP; u++) pair_add(I, q[u]);
+      for (int u = 0; u < FQ_STEP; u++) pair_add(I, t[u]);
     } else {
 #pragma unroll
-      for (int u = 0; u < FQ_STEP; u++) pair_add_if(I, q[u], ok[u]);
+      for (int u = 0; u < FQ_STEP; u++) pair_add_if(I, t[u], ok[u]);
     }
-  };
-  // The bitmask is read once, as a stream: non-temporal loads, as above.
-  if (wave_max(longest) <= 32) {
-    // a word a row: the queue holds them all
-    uint w[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int f = r == 0 ? 0 : E_[r - 1];
-      w[r] = f < E_[r] ? __builtin_nontemporal_load(&bits[(size_t)f * NN + i]) : 0u;
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++) {  // a zero word is written over by the next
-      qw[64 * cnt] = w[r];
-      qb[64 * cnt] = 2u * (uint)jb[r];
-      cnt += w[r] != 0u ? 1 : 0;
-      qn += __popc(w[r]);
-    }
-  } else {
-    const int maxf = wave_max(nwords);
-    uint nx[FW_AHEAD];
-#pragma unroll
-    for (int k = 0; k < FW_AHEAD; k++) nx[k] = k < nwords ? __builtin_nontemporal_load(&bits[(size_t)k * NN + i]) : 0u;
-    for (int f0 = 0; f0 < maxf; f0 += FW_AHEAD) {
-      uint cw[FW_AHEAD];
-#pragma unroll
-      for (int k = 0; k < FW_AHEAD; k++) {
-        cw[k] = nx[k];
-        const int fn = f0 + FW_AHEAD + k;
-        nx[k] = fn < nwords ? __builtin_nontemporal_load(&bits[(size_t)fn * NN + i]) : 0u;
-      }
-#pragma unroll
-      for (int k = 0; k < FW_AHEAD; k++) {
-        const int f = f0 + k;
-        if (f >= maxf) break;
-        const uint word = cw[k];
-        int base = jb[0], first = 0;  // of the row that holds word f
-#pragma unroll
-        for (int r = 1; r < R; r++) {
-          const bool in = f >= E_[r - 1];
-          base = in ? jb[r] : base;
-          first = in ? E_[r - 1] : first;
-        }
-        const bool full = word != 0u && cnt == FQ_K;
-        if (__any(full)) {
-          // free a slot: the full lanes finish their current word, every lane
-          // gives as many pairs as the shortest queue holds
-          ahead();
-          int f1 = max(wave_max(full ? __popc(cur) + 1 : 0), wave_min(nwords > 0 ? qn : INT_MAX));
-          do {
-            step();
-            f1 -= FQ_STEP;
-          } while (f1 > 0 || __any(word != 0u && cnt == FQ_K));
-        }
-        if (word != 0u) {
-          const int t = (head + 64 * cnt) & MASK;
-          qw[t] = word;
-          qb[t] = 2u * (uint)(base + ((f - first) << 5));
-          cnt++;
-          qn += __popc(word);
-        }
-      }
-    }
-  }
-  ahead();
-  while (__any(qn > 0)) step();
+  });
   if (act) st3(pbuf<fx_float3>(FPnts, FFORCE), (size_t)i, I.fx, I.fy, I.fz);
 }
 

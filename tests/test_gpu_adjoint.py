@@ -370,3 +370,36 @@ def test_adjoint_dambreak_262k_full_size(ps):
         errs.append(e)
     assert len(errs) == 6
     assert max(errs) <= 1e-4
+
+
+def close_pair(pos):
+    """Two particles whose r^2 lies below the range of the pair terms' short square root (2^-79)."""
+    pos[0] = (0.0, 20.0, 0.0)
+    pos[1] = (6e-11, 20.0, 0.0)
+    return pos
+
+
+# one lane, both sides of a wave, rows of several words (beyond the queue's 16
+# a lane), and a pair whose roots the short sequences do not take
+@pytest.mark.parametrize("n,side", [(1, 5.0), (63, 5.0), (65, 5.0), (4000, 10.0), (2500, 20.0)])
+def test_adjoint_pair_walk(ps, n, side):
+    sc = scenes.dambreak_16k(n)
+    rng = np.random.default_rng(n)
+    pos = (rng.uniform(0, 1, (n, 3)) * side + [-side / 2, 20 - side / 2, -side / 2]).astype(np.float32)
+    if n > 1:
+        pos = close_pair(pos)
+    T = 2
+    target = (pos + rng.uniform(-0.1, 0.1, (n, 3))).astype(np.float32)
+    ps.Restart(sc)
+    ps.Commit(abi.FPOS, pos)
+    ps.AdjointConfigure(T, 1)
+    ps.AdjointSetTarget(target)
+    loss, _ = ps.AdjointForward()
+    g = ps.AdjointBackward()
+    P = derive_params(sc)
+    _, clr = fill_points(sc)
+    r = oracle.grad(P, {"pos": pos, "clr": clr}, T, target, fp64=False, threads=THREADS)
+    for k in ("gpos", "gvel", "gveval"):
+        assert np.isfinite(r[k]).all()
+        assert bits_equal(g[k], r[k]), (k, np.abs(g[k] - r[k]).max())
+    assert loss[0] == pytest.approx(r["loss"], rel=1e-9)
