@@ -525,9 +525,9 @@ int Particles::PrefixScanParticles() {
   // particles.cpp:774-815, over gridTotal+1 counts; then the out-of-range
   // flags, whose exclusive scan ranks the tail bucket in particle order.
   // Both scans in two launches (block totals first, into the first
-  // auxiliary level of each, which holds one entry per 1024 elements); the
-  // reference's three-level prefixSum/prefixFixup for a scan beyond
-  // FX_SCAN2_MAX_BLOCKS blocks.
+  // auxiliary level of each, which holds one entry per 1024 elements), one
+  // where they are short; the reference's three-level prefixSum/prefixFixup
+  // for a scan beyond FX_SCAN2_MAX_BLOCKS blocks.
   FX_TRY(ScanGrid(false));
   m_Done = FX_STAGE_PREFIX;
   return FX_OK;
@@ -587,7 +587,10 @@ int Particles::ScanTwoLaunch(void* in, void* out, void* sums, int n, void* in2, 
             m_Params.dt, m_Parity};
   if (nb + nb2 == 0) return FX_OK;
   void* a[] = {&J};
-  FX_TRY(Launch(FUNC_SCAN_SUMS, (unsigned)(nb + nb2), FX_SCAN2_THREADS, a));
+  if (nb > FX_SCAN1_MAX_BLOCKS || nb2 > FX_SCAN1_MAX_BLOCKS)
+    FX_TRY(Launch(FUNC_SCAN_SUMS, (unsigned)(nb + nb2), FX_SCAN2_THREADS, a));
+  else
+    J.j[0].sums = J.j[1].sums = nullptr;
   return Launch(FUNC_SCAN_APPLY, (unsigned)(nb + nb2), FX_SCAN2_THREADS, a);
 }
 

@@ -52,6 +52,12 @@
 #define FX_SCAN2_THREADS 512  // threads per block of fxScanSums / fxScanApply
 #define FX_SCAN2_BLOCK 2048   // elements per block (4 per thread)
 #define FX_SCAN2_MAX_BLOCKS 8192
+// Up to this many blocks fxScanApply alone: its last block reads everything
+// before its own elements (8 KB a block), cheaper than the launch of
+// fxScanSums while they are few.  Prefix stage, two launches / one (us, HIP
+// events around it): 9.6 / 7.3 at 3 to 13 blocks, 9.8 / 9.3 at 40 (the same
+// within a captured step), 10.0 / 12.0 at 75.
+#define FX_SCAN1_MAX_BLOCKS 24
 #define FUNC_SCAN_APPLY 31
 #define FUNC_PRESS_W 32    // per-wave density, 1, 2 and 4 lanes to a particle
 #define FUNC_PRESS_WB 35   // the same for a batch

@@ -441,7 +441,8 @@ extern "C" __global__ __launch_bounds__(SCAN_BLOCKSIZE) void prefixFixup(
 // every block of FXS_BLOCK elements; in fxScanApply block b adds up the
 // totals of the blocks before it (a few thousand at most, read once per
 // block) and scans its own elements on top.  Exclusive, uint32: the same
-// results as the reference-named kernels.
+// results as the reference-named kernels.  Where sums is null there is no
+// first launch: a block adds up the elements before its own itself.
 #define FXS_THREADS 512
 #define FXS_PER 4
 #define FXS_BLOCK (FXS_THREADS * FXS_PER)
@@ -473,7 +474,7 @@ __device__ __forceinline__ uint fxs_block_sum(uint v, uint* lds) {
 struct FxScanJob {
   const uint* in;
   uint* out;
-  uint* sums;  // one total per block of FXS_BLOCK elements
+  uint* sums;  // one total per block of FXS_BLOCK elements, or null
   int n;
   int nb;  // blocks: ceil(n / FXS_BLOCK)
 };
@@ -536,7 +537,18 @@ extern "C" __global__ __launch_bounds__(FXS_THREADS) void fxScanApply(FxScanJobs
   uint* __restrict__ out = S.out;
   const int n = S.n;
   uint pre = 0u;
-  for (int j = (int)threadIdx.x; j < b; j += FXS_THREADS) pre += S.sums[j];
+  if (S.sums != nullptr) {
+    for (int j = (int)threadIdx.x; j < b; j += FXS_THREADS) pre += S.sums[j];
+  } else {
+    const uint4* __restrict__ in4 = reinterpret_cast<const uint4*>(in) + threadIdx.x;
+    for (int j0 = 0; j0 < b; j0 += 16) {  // 16 loads in flight
+      uint4 w[16];
+#pragma unroll
+      for (int k = 0; k < 16; k++) w[k] = in4[(size_t)(j0 + k < b ? j0 + k : 0) * FXS_THREADS];
+#pragma unroll
+      for (int k = 0; k < 16; k++) pre += j0 + k < b ? w[k].x + w[k].y + w[k].z + w[k].w : 0u;
+    }
+  }
   pre = fxs_block_sum(pre, lds);
   const int i = b * FXS_BLOCK + (int)threadIdx.x * FXS_PER;
   const uint4 v = fxs_load(in, i, n);

@@ -113,7 +113,7 @@ def test_stencils_in_a_batch(ps, gd):
 # Steps that run straight through share a pass between one step's advance and
 # the next one's insert: the same state, tables and ranks as single steps, in
 # one scene (with particles that leave the grid), in a batch and replayed.
-@pytest.mark.parametrize("n", [1, 63, 65, 257, 5003])
+@pytest.mark.parametrize("n", [1, 63, 65, 257, 5003, 60001])
 @pytest.mark.parametrize("batch", [False, True])
 def test_joined_steps(ps, n, batch):
     def restart():
@@ -145,3 +145,12 @@ def test_joined_steps(ps, n, batch):
             assert bits_equal(s[k][m], states[0][k][m]), k
         for k in ("pos", "vel", "veval"):
             assert bits_equal(s[k], states[0][k]), k
+
+
+# particles and cell tables on both sides of the block counts (24 blocks of
+# 2,048 entries) up to which one launch scans them
+@pytest.mark.parametrize("n,half", [(2047, 30), (2049, 30), (49152, 30), (49153, 30), (2047, 67), (2047, 68)])
+def test_scan_launches(ps, n, half):
+    sc = scenes.dambreak_16k(n)
+    sc.bound_min.x, sc.bound_max.x = -half, half
+    one_step_bitexact(ps, sc, vel=swirl(n, 9))
