@@ -991,11 +991,15 @@ int Particles::SampleParticles(float* brick, const int* res, const float* bmin, 
   fx_int3 r = {res[0], res[1], res[2]};
   fx_float3 lo = {bmin[0], bmin[1], bmin[2]}, hi = {bmax[0], bmax[1], bmax[2]};
   int n = mNumPoints;
-  void* args[] = {&d, &r, &lo, &hi, &n, &scalar};
+  // exp(-r^2 / h2) as a power of two: its exponent per world d^2, in two floats
+  const float h2 = 2.0f * m_Params.r2 / 8.0f;
+  const double k = -(double)m_Params.d2 / (double)h2 * 1.4426950408889634;
+  float khi = (float)k, klo = (float)(k - (double)khi);
+  void* args[] = {&d, &r, &lo, &hi, &n, &scalar, &khi, &klo};
   const unsigned bx = 8, by = 8, bz = 4;
   hipError_t e = hipModuleLaunchKernel(m_Func[FUNC_SAMPLE], (unsigned)((res[0] + bx - 1) / bx),
-                                       (unsigned)((res[1] + by - 1) / by), (unsigned)((res[2] + bz - 1) / bz), bx, by,
-                                       bz, 0, m_Stream, args, nullptr);
+                                       (unsigned)((res[1] + by - 1) / by), (unsigned)((res[2] + bz - 1) / bz), 256, 1,
+                                       1, 0, m_Stream, args, nullptr);
   if (e == hipSuccess) e = hipStreamSynchronize(m_Stream);
   if (e == hipSuccess) e = hipMemcpyDtoH(brick, d, nv * sizeof(float));
   (void)hipFree(d);

@@ -203,3 +203,23 @@ def test_scene_file_scene_steps_like_the_oracle():
     valid = ref["gcell"] != abi.GRID_UNDEF
     for k in ("press", "force"):
         assert bits_equal(g[k][valid], ref[k][valid]), k
+
+
+# bricks that fill no block (8 x 8 x 4 voxels), and stencil rows of 2, 3 and 4 cells
+@pytest.mark.parametrize("res", [(1, 1, 1), (7, 9, 5), (33, 8, 4)])
+@pytest.mark.parametrize("gd", [1.0, 1.5, 2.5])
+def test_sample_particles_shapes(ps, res, gd):
+    from oracle import oracle
+    from parity import rel_err
+
+    sc = scenes.dambreak_16k(4000)
+    sc.grid_density = gd
+    ps.Restart(sc)
+    ps.Run(2)
+    st = ps.state()
+    p = ps.params
+    lo, hi = (-25.0, 0.0, -25.0), (25.0, 30.0, 25.0)
+    g = ps.SampleParticles(res, lo, hi, 0.5)
+    r = oracle.sample(p, st, res, lo, hi, 0.5)
+    assert np.array_equal(g == 0, r == 0)
+    assert rel_err(g, r) <= 1e-5  # as the test above: powers in 32 bits on both sides
