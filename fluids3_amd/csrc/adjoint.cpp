@@ -290,23 +290,17 @@ int Particles::AdjConfigure(const char* path, int nsteps, int every) {
 int Particles::AdjTables() {
   if (m_AdjN == 0 || m_AdjN != mNumPoints || m_AdjCells != m_ScanCells || m_AdjScenes != NumScenes())
     return fx::fail(FX_ESTATE, "adjoint: configure after Restart (the particle or cell count changed)");
-  if (m_Batch) {
-    FX_HIP(hipMemcpyHtoD(m_AdjParams, m_SceneParams.data(), sizeof(FParams_t) * m_SceneParams.size()),
-           "adjoint");
-  } else {
-    FX_HIP(hipMemcpyHtoD(m_AdjParams, &m_Params, sizeof(FParams_t)), "adjoint");
-  }
-  return FX_OK;
+  if (m_Batch)
+    return m_Staging.up(m_AdjParams, m_SceneParams.data(), sizeof(FParams_t) * m_SceneParams.size(), "adjoint");
+  return m_Staging.up(m_AdjParams, &m_Params, sizeof(FParams_t), "adjoint");
 }
 
 int Particles::AdjSetTarget(const float* target, int64_t count) {
   if (m_AdjN == 0) return fx::fail(FX_ESTATE, "adjoint: call fx_adjoint_configure first");
   if (target == nullptr || count != (int64_t)m_AdjN)
     return fx::fail(FX_EINVAL, "adjoint: the target holds one position per particle (%d)", m_AdjN);
-  FX_HIP(hipStreamSynchronize(m_Stream), "adjoint");
-  FX_HIP(hipMemcpyHtoD(m_AdjVec + (size_t)m_AdjN * 19, const_cast<float*>(target), sizeof(float) * 3 * (size_t)count),
-         "adjoint: target upload");
-  return FX_OK;
+  return m_Staging.up(m_AdjVec + (size_t)m_AdjN * 19, target, sizeof(float) * 3 * (size_t)count,
+                      "adjoint: target upload");
 }
 
 // bytes of a recorded step's tape slot
@@ -454,9 +448,7 @@ int Particles::AdjForward(double* loss, double* ms) {
   }
   if (ms) FX_HIP(hipEventRecord(e1.e, m_Stream), "adjoint");
   std::vector<double> acc(3 * (size_t)m_AdjScenes);
-  FX_HIP(hipMemcpyAsync(acc.data(), m_AdjAccum, acc.size() * sizeof(double), hipMemcpyDeviceToHost, m_Stream),
-         "adjoint");
-  FX_HIP(hipStreamSynchronize(m_Stream), "adjoint");
+  FX_TRY(m_Staging.down(acc.data(), m_AdjAccum, acc.size() * sizeof(double), "adjoint"));
   for (int s = 0; s < m_AdjScenes; s++) {
     const int ns = m_PBase[s + 1] - m_PBase[s];
     if (loss) loss[s] = ns > 0 ? acc[3 * s] / (double)ns : 0.0;
@@ -594,13 +586,11 @@ int Particles::AdjBackward(float* gpos, float* gvel, float* gveval, double* gvis
            "adjReduce");
   }
   if (ms) FX_HIP(hipEventRecord(e1.e, m_Stream), "adjoint");
-  if (!first)
-    FX_HIP(hipMemcpyAsync(acc.data(), m_AdjAccum, acc.size() * sizeof(double), hipMemcpyDeviceToHost, m_Stream),
-           "adjoint");
+  if (!first) FX_TRY(m_Staging.down(acc.data(), m_AdjAccum, acc.size() * sizeof(double), "adjoint"));
   const size_t vb = sizeof(float) * 3 * n;
-  if (gpos) FX_HIP(hipMemcpyAsync(gpos, V + 9 * n, vb, hipMemcpyDeviceToHost, m_Stream), "adjoint");
-  if (gvel) FX_HIP(hipMemcpyAsync(gvel, V + 12 * n, vb, hipMemcpyDeviceToHost, m_Stream), "adjoint");
-  if (gveval) FX_HIP(hipMemcpyAsync(gveval, V + 15 * n, vb, hipMemcpyDeviceToHost, m_Stream), "adjoint");
+  if (gpos) FX_TRY(m_Staging.down(gpos, V + 9 * n, vb, "adjoint"));
+  if (gvel) FX_TRY(m_Staging.down(gvel, V + 12 * n, vb, "adjoint"));
+  if (gveval) FX_TRY(m_Staging.down(gveval, V + 15 * n, vb, "adjoint"));
   FX_HIP(hipStreamSynchronize(m_Stream), "adjoint");
   for (int s = 0; s < m_AdjScenes; s++) {
     if (gk) gk[s] = acc[3 * s + 1];

@@ -42,6 +42,7 @@ static void free_batch(void*& a, void*& b, void*& c, std::map<int, std::pair<voi
 }
 
 Particles::~Particles() {
+  if (m_Stream) (void)hipStreamSynchronize(m_Stream);  // queued copies read the staging memory
   ReleaseGraph();
   AdjRelease();
   for (hipEvent_t& e : m_AdjEv)
@@ -56,6 +57,7 @@ Particles::~Particles() {
   if (m_Clock) (void)hipFree(m_Clock);
   if (m_Stats) (void)hipFree(m_Stats);
   if (m_WorkQ) (void)hipFree(m_WorkQ);
+  if (m_Brick) (void)hipFree(m_Brick);
   if (m_Stream) (void)hipStreamDestroy(m_Stream);
   if (m_Module) (void)hipModuleUnload(m_Module);
 }
@@ -87,6 +89,7 @@ int Particles::Initialize(const char* path) {
   int capv = FX_CAP_TAIL | FX_CAP_RANKED;
   FX_HIP(hipMemcpyHtoD(caps, &capv, sizeof(int)), "Initialize");
   FX_HIP(hipStreamCreate(&m_Stream), "Initialize");
+  FX_TRY(m_Staging.create(m_Stream));
   FX_HIP(hipMalloc(&m_Tables, 2 * sizeof(cuDataX)), "Initialize");
   FX_HIP(hipMalloc((void**)&m_Clock, 2 * sizeof(float)), "Initialize");
   FX_HIP(hipMalloc(&m_Stats, 2 * sizeof(unsigned long long)), "Initialize");
@@ -629,8 +632,7 @@ int Particles::PublishTables() {
 
 int Particles::SetDeviceClock() {
   // clock[1] is the time of the next step a captured graph runs
-  FX_HIP(hipMemcpyHtoD(m_Clock + 1, &m_Params.time, sizeof(float)), "device clock");
-  return FX_OK;
+  return m_Staging.up(m_Clock + 1, &m_Params.time, sizeof(float), "device clock");
 }
 
 int Particles::CountingSort() {
@@ -831,7 +833,6 @@ int Particles::LaunchGraph(int nlaunch) {
   // the graph replays the set exchange it was captured with
   if (m_GraphExec == nullptr || m_GraphParity != m_Parity) FX_TRY(CaptureGraph());
   // the device clock starts from the host time of the first replayed step
-  FX_HIP(hipStreamSynchronize(m_Stream), "LaunchGraph");
   FX_TRY(SetDeviceClock());
   for (int k = 0; k < nlaunch; k++) {
     FX_HIP(hipGraphLaunch(m_GraphExec, m_Stream), "LaunchGraph");
@@ -845,7 +846,13 @@ int Particles::LaunchGraph(int nlaunch) {
 // ---------------------------------------------------------------- transfers
 
 int Particles::CheckIds(const uint32_t* id, int64_t n, const char* who) {
+  // n ids below n that leave none out are a permutation; otherwise the loop
+  // after this names the first that is wrong
   std::vector<uint8_t> seen((size_t)n, 0);
+  int64_t a = 0;
+  for (; a < n && id[a] < (uint64_t)n; a++) seen[id[a]] = 1;
+  if (a == n && (n == 0 || memchr(seen.data(), 0, (size_t)n) == nullptr)) return FX_OK;
+  std::fill(seen.begin(), seen.end(), 0);
   for (int64_t k = 0; k < n; k++) {
     if (id[k] >= (uint64_t)n || seen[id[k]])
       return fx::fail(FX_EINVAL, "%s: ids are not a permutation of 0..%lld (entry %lld = %u)", who, (long long)n - 1,
@@ -866,9 +873,7 @@ int Particles::Upload(int buf, const void* host, int64_t count) {
       return fx::fail(FX_EINVAL, "upload: FID takes all %d ids at once, not %lld", mNumPoints, (long long)count);
     FX_TRY(CheckIds(static_cast<const uint32_t*>(host), count, "upload"));
   }
-  FX_HIP(hipStreamSynchronize(m_Stream), "upload");
-  FX_HIP(hipMemcpyHtoD(b->mGpu, const_cast<void*>(host), (size_t)count * b->mStride), "upload");
-  return FX_OK;
+  return m_Staging.up(b->mGpu, host, (size_t)count * b->mStride, "upload");
 }
 
 int Particles::Download(int buf, void* host, int64_t count) {
@@ -876,9 +881,7 @@ int Particles::Download(int buf, void* host, int64_t count) {
   if (b == nullptr || host == nullptr) return fx::fail(FX_EINVAL, "download: unknown buffer %d", buf);
   if (count < 0 || (uint64_t)count > b->mMax) return fx::fail(FX_ERANGE, "download: %lld elements exceed %llu",
                                                              (long long)count, (unsigned long long)b->mMax);
-  FX_HIP(hipStreamSynchronize(m_Stream), "download");
-  FX_HIP(hipMemcpyDtoH(host, b->mGpu, (size_t)count * b->mStride), "download");
-  return FX_OK;
+  return m_Staging.down(host, b->mGpu, (size_t)count * b->mStride, "download");
 }
 
 int Particles::DownloadAccel(int buf, void* host, int64_t count) {
@@ -887,9 +890,7 @@ int Particles::DownloadAccel(int buf, void* host, int64_t count) {
   if (count < 0 || (uint64_t)count > b->mMax)
     return fx::fail(FX_ERANGE, "download_accel: %lld elements exceed %llu", (long long)count,
                     (unsigned long long)b->mMax);
-  FX_HIP(hipStreamSynchronize(m_Stream), "download_accel");
-  FX_HIP(hipMemcpyDtoH(host, b->mGpu, (size_t)count * b->mStride), "download_accel");
-  return FX_OK;
+  return m_Staging.down(host, b->mGpu, (size_t)count * b->mStride, "download_accel");
 }
 
 int Particles::Scan(const uint32_t* in, uint32_t* out, int n) {
@@ -938,8 +939,7 @@ int Particles::Mark(int tag) {
 }
 
 int Particles::Synchronize() {
-  FX_HIP(hipStreamSynchronize(m_Stream), "synchronize");
-  return FX_OK;
+  return m_Staging.drain("synchronize");
 }
 
 // ------------------------------------------------------------------- timing
@@ -986,8 +986,16 @@ int Particles::SampleParticles(float* brick, const int* res, const float* bmin, 
   if (res[0] <= 0 || res[1] <= 0 || res[2] <= 0 || (int64_t)res[0] * res[1] * res[2] > ((int64_t)1 << 31))
     return fx::fail(FX_ERANGE, "sample_particles: bad brick resolution %d x %d x %d", res[0], res[1], res[2]);
   const size_t nv = (size_t)res[0] * res[1] * res[2];
-  void* d = nullptr;
-  FX_HIP(hipMalloc(&d, nv * sizeof(float)), "sample_particles");
+  // the brick stays for the next call up to kBrickKept
+  const size_t kBrickKept = (size_t)64 << 20, bytes = nv * sizeof(float);
+  if (bytes > m_BrickBytes) {
+    if (m_Brick) (void)hipFree(m_Brick);
+    m_Brick = nullptr;
+    m_BrickBytes = 0;
+    FX_HIP(hipMalloc(&m_Brick, bytes), "sample_particles");
+    m_BrickBytes = bytes;
+  }
+  void* d = m_Brick;
   fx_int3 r = {res[0], res[1], res[2]};
   fx_float3 lo = {bmin[0], bmin[1], bmin[2]}, hi = {bmax[0], bmax[1], bmax[2]};
   int n = mNumPoints;
@@ -1000,11 +1008,14 @@ int Particles::SampleParticles(float* brick, const int* res, const float* bmin, 
   hipError_t e = hipModuleLaunchKernel(m_Func[FUNC_SAMPLE], (unsigned)((res[0] + bx - 1) / bx),
                                        (unsigned)((res[1] + by - 1) / by), (unsigned)((res[2] + bz - 1) / bz), 256, 1,
                                        1, 0, m_Stream, args, nullptr);
-  if (e == hipSuccess) e = hipStreamSynchronize(m_Stream);
-  if (e == hipSuccess) e = hipMemcpyDtoH(brick, d, nv * sizeof(float));
-  (void)hipFree(d);
-  if (e != hipSuccess) return fx::hip_fail(e, "sample_particles", "sampleParticles");
-  return FX_OK;
+  const int st = e != hipSuccess ? fx::hip_fail(e, "sample_particles", "sampleParticles")
+                                 : m_Staging.down(brick, d, bytes, "sample_particles");
+  if (m_BrickBytes > kBrickKept) {
+    (void)hipFree(m_Brick);
+    m_Brick = nullptr;
+    m_BrickBytes = 0;
+  }
+  return st;
 }
 
 int Particles::EmitParticles(float frame, int emit) {

@@ -73,6 +73,8 @@
 #include <string>
 #include <vector>
 
+#include "fx_staging.hpp"
+
 // Kernel argument block of the *Batch kernels (BatchArgs in the kernel file).
 struct FxBatchArgs {
   const void* params;
@@ -230,6 +232,9 @@ class Particles {
   hipModule_t m_Module = nullptr;
   hipFunction_t m_Func[FUNC_MAX] = {};
   hipStream_t m_Stream = nullptr;
+  fx::Staging m_Staging;  // host arrays to and from m_Stream
+  void* m_Brick = nullptr;  // voxels of SampleParticles
+  size_t m_BrickBytes = 0;
   void* m_cuParams = nullptr;  // device address of FParams
 
   int mNumPoints = 0;

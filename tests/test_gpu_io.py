@@ -223,3 +223,29 @@ def test_sample_particles_shapes(ps, res, gd):
     r = oracle.sample(p, st, res, lo, hi, 0.5)
     assert np.array_equal(g == 0, r == 0)
     assert rel_err(g, r) <= 1e-5  # as the test above: powers in 32 bits on both sides
+
+
+# arrays on both sides of the transfers' limits: a slot (1 MB), a queued upload
+# (2 MB), a download by one thread (4 MB), every slot used twice (16 MB); more
+# uploads in a row than the 4 MB they are queued in
+@pytest.mark.parametrize("n", [1, 2000, 87381, 87382, 174762, 174763, 349525, 349526, 1500001])
+def test_transfers(ps, n):
+    rng = np.random.default_rng(n)
+    ps.Restart(scenes.scaled_dam_break(n))
+    put = {b: rng.standard_normal((n, 3)).astype(np.float32) for b in (abi.FPOS, abi.FVEL, abi.FVEVAL, abi.FFORCE)}
+    ids = rng.permutation(n).astype(np.uint32)
+    for _ in range(2):
+        for b, a in put.items():
+            a += 1.0
+            ps.Commit(b, a)
+        ps.Commit(abi.FID, ids)
+    for b, a in put.items():
+        assert np.array_equal(ps.Retrieve(b), a), b
+    assert np.array_equal(ps.Retrieve(abi.FID), ids)
+    assert np.array_equal(ps.Retrieve(abi.FVEL, n // 2), put[abi.FVEL][:n // 2])
+    for wrong in (n, ids[0]):  # out of range; twice the same
+        bad = ids.copy()
+        bad[n - 1] = wrong
+        if n > 1 or wrong == n:
+            with pytest.raises(Exception, match="permutation"):
+                ps.Commit(abi.FID, bad)
