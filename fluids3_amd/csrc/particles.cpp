@@ -794,53 +794,68 @@ int Particles::Run(int nsteps) {
 // ------------------------------------------------------------------ graphs
 
 void Particles::ReleaseGraph() {
-  if (m_GraphExec) (void)hipGraphExecDestroy(m_GraphExec);
-  if (m_Graph) (void)hipGraphDestroy(m_Graph);
-  m_GraphExec = nullptr;
-  m_Graph = nullptr;
+  for (hipGraphExec_t& e : m_GraphExec) {
+    if (e) (void)hipGraphExecDestroy(e);
+    e = nullptr;
+  }
+}
+
+// Captures two steps as m_GraphExec[inner].  Joined steps (JoinedSteps) begin
+// with their insert made: that of the first pair is made by the launches of
+// ReplayGraph, that of a later one by the inner pair before it, whose last
+// advance inserts; the last pair leaves the tables of its own sort.
+int Particles::CapturePair(int inner) {
+  const int parity0 = m_Parity, done0 = m_Done;
+  const bool joined = JoinedSteps();
+  FX_HIP(hipStreamBeginCapture(m_Stream, hipStreamCaptureModeThreadLocal), "CaptureGraph");
+  m_Capturing = true;
+  int st = FX_OK;
+  for (int s = 0; s < 2 && st == FX_OK; s++) st = Step(!joined, s == 1 && inner == 0);
+  m_Capturing = false;
+  hipGraph_t g = nullptr;
+  hipError_t e = hipStreamEndCapture(m_Stream, &g);
+  if (m_Parity != parity0) {  // a failed capture: nothing of it ran, restore the host view of the sets
+    (void)m_Points.SwapGPU(&m_PointsTemp);
+    m_Parity = parity0;
+  }
+  m_Done = done0;  // recorded, not run
+  if (st == FX_OK && e == hipSuccess) e = hipGraphInstantiate(&m_GraphExec[inner], g, nullptr, nullptr, 0);
+  if (g) (void)hipGraphDestroy(g);
+  if (st != FX_OK) return st;
+  FX_HIP(e, "CaptureGraph");
+  return FX_OK;
 }
 
 int Particles::CaptureGraph() {
   if (mNumPoints == 0) return fx::fail(FX_ESTATE, "CaptureGraph: call Restart first");
   FX_HIP(hipStreamSynchronize(m_Stream), "CaptureGraph");
   ReleaseGraph();
-  const int parity0 = m_Parity, done0 = m_Done;
-  FX_HIP(hipStreamBeginCapture(m_Stream, hipStreamCaptureModeThreadLocal), "CaptureGraph");
-  m_Capturing = true;
-  int st = FX_OK;
-  for (int s = 0; s < 2 && st == FX_OK; s++) st = Step(s == 0, s == 1);
-  m_Capturing = false;
-  hipGraph_t g = nullptr;
-  hipError_t e = hipStreamEndCapture(m_Stream, &g);
-  if (st != FX_OK || e != hipSuccess) {
-    // nothing of a failed capture ran: restore the host view of the sets
-    if (g) (void)hipGraphDestroy(g);
-    if (m_Parity != parity0) {
-      (void)m_Points.SwapGPU(&m_PointsTemp);
-      m_Parity = parity0;
-    }
-    m_Done = done0;
-    return st != FX_OK ? st : fx::hip_fail(e, "CaptureGraph", "hipStreamEndCapture");
-  }
-  m_Done = done0;  // recorded, not run
-  m_Graph = g;
   m_GraphParity = m_Parity;
-  FX_HIP(hipGraphInstantiate(&m_GraphExec, m_Graph, nullptr, nullptr, 0), "CaptureGraph");
-  return FX_OK;
+  m_GraphJoined = JoinedSteps();
+  int st = CapturePair(0);
+  if (st == FX_OK && m_GraphJoined) st = CapturePair(1);
+  if (st != FX_OK) ReleaseGraph();
+  return st;
 }
 
-int Particles::LaunchGraph(int nlaunch) {
-  // the graph replays the set exchange it was captured with
-  if (m_GraphExec == nullptr || m_GraphParity != m_Parity) FX_TRY(CaptureGraph());
-  // the device clock starts from the host time of the first replayed step
-  FX_TRY(SetDeviceClock());
+// nlaunch replays of two steps, on a captured graph.
+int Particles::ReplayGraph(int nlaunch) {
+  if (m_GraphJoined && nlaunch > 0) FX_TRY(InsertParticles());
   for (int k = 0; k < nlaunch; k++) {
-    FX_HIP(hipGraphLaunch(m_GraphExec, m_Stream), "LaunchGraph");
+    FX_HIP(hipGraphLaunch(m_GraphExec[m_GraphJoined && k + 1 < nlaunch ? 1 : 0], m_Stream), "LaunchGraph");
     AdvanceTime();
     AdvanceTime();
     m_Done = FX_STAGE_ADVANCE;
   }
   return FX_OK;
+}
+
+int Particles::LaunchGraph(int nlaunch) {
+  // the graph replays the set exchange it was captured with
+  if (m_GraphExec[0] == nullptr || m_GraphParity != m_Parity) FX_TRY(CaptureGraph());
+  // the device clock starts from the host time of the first replayed step
+  FX_TRY(SetDeviceClock());
+  return ReplayGraph(nlaunch);
 }
 
 // ---------------------------------------------------------------- transfers
@@ -1159,7 +1174,7 @@ int Particles::BenchSteps(int nsteps, bool use_graph, double* ms_total, double* 
 
 int Particles::TimeSteps(int nsteps, bool use_graph, double* ms_total) {
   if (nsteps < 0 || ms_total == nullptr) return fx::fail(FX_EINVAL, "time_steps: bad arguments");
-  if (use_graph && (m_GraphExec == nullptr || m_GraphParity != m_Parity)) FX_TRY(CaptureGraph());
+  if (use_graph && (m_GraphExec[0] == nullptr || m_GraphParity != m_Parity)) FX_TRY(CaptureGraph());
   if (use_graph) {
     // the device clock must hold the host time before the timed region
     FX_HIP(hipStreamSynchronize(m_Stream), "time_steps");
@@ -1173,12 +1188,7 @@ int Particles::TimeSteps(int nsteps, bool use_graph, double* ms_total) {
   if (hipEventRecord(a, m_Stream) != hipSuccess) st = fx::fail(FX_EHIP, "time_steps: record");
   if (st == FX_OK) {
     if (use_graph) {
-      for (int k = 0; k < nsteps / 2 && st == FX_OK; k++) {
-        if (hipGraphLaunch(m_GraphExec, m_Stream) != hipSuccess) st = fx::fail(FX_EHIP, "time_steps: graph launch");
-        AdvanceTime();
-        AdvanceTime();
-        m_Done = FX_STAGE_ADVANCE;
-      }
+      st = ReplayGraph(nsteps / 2);
       if (st == FX_OK && (nsteps & 1)) st = Run();
     } else {
       st = Run(nsteps);

@@ -202,6 +202,8 @@ class Particles {
   int SortStep(bool insert);
   int AdvanceInsert(TapeSlot* tape = nullptr);
   int SetDeviceClock();
+  int CapturePair(int inner);
+  int ReplayGraph(int nlaunch);
   void ReleaseGraph();
   int BuildBlockTables();
   // one batch launch of a stage: kernel fid, one block per block-table
@@ -257,8 +259,8 @@ class Particles {
   void* m_NbrWordsSym = nullptr;  // the module's FNbrWords (bitmask words a particle may record)
   void* m_SortSrcSym = nullptr;   // the module's FSortSrc (where the sort writes its permutation, or null)
 
-  hipGraph_t m_Graph = nullptr;
-  hipGraphExec_t m_GraphExec = nullptr;
+  hipGraphExec_t m_GraphExec[2] = {};  // the last (or only) pair of steps, and one that another follows
+  bool m_GraphJoined = false;          // whether the pairs begin with their insert made
   bool m_Capturing = false;
   int m_GraphParity = 0;
   int m_MaxSrch = 0;  // cells a stencil row, the largest of the scenes

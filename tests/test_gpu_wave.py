@@ -128,11 +128,16 @@ def test_joined_steps(ps, n, batch):
         ps.Commit(abi.FVEL, swirl(total, total))
 
     states = []
-    for steps in ([1] * 5, [5], [2, 3], "graph"):
+    for steps in ([1] * 5, [5], [2, 3], "graph", "graphs"):
         restart()
         if steps == "graph":
             ps.LaunchGraph(2)
             ps.Run(1)
+        elif steps == "graphs":
+            ps.Run(1)
+            ps.LaunchGraph(1)
+            ps.state()
+            ps.LaunchGraph(1)
         else:
             for k in steps:
                 ps.Run(k)
