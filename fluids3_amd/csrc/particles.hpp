@@ -67,7 +67,9 @@
 #define FUNC_ADVANCE_INSERT_B 41
 #define FUNC_ADVANCE_TAPE 42    // the same, recording the step on a rollout's tape
 #define FUNC_ADVANCE_TAPE_B 43
-#define FUNC_MAX 44
+#define FUNC_FORCE_W4 44        // per-wave force, four lanes to a particle
+#define FUNC_FORCE_WB4 45
+#define FUNC_MAX 46
 
 #include <map>
 #include <string>
@@ -213,6 +215,7 @@ class Particles {
   int LaunchLanes(int fid, int fid_b, int threads, int lanes, unsigned lds, NbrBits bits,
                   void* extra0 = nullptr, void* extra1 = nullptr);
   int DensityLanes() const;
+  int ForceLanes() const;
   int StageThreads(int stage, int most) const;
   bool WaveStages() const;
   int BlockTable(int particles);

@@ -2173,6 +2173,178 @@ extern "C" __global__ __launch_bounds__(1024) void computeForceWaveBatch(BatchAr
   clear_counts(clear, nclear);
 }
 
+// Four lanes to a particle, for launches of few waves: those wait for the
+// chain of their busiest lane (a step's gathers, then its terms, some 20
+// times over), and a quarter of the pairs a lane shortens it.  The wave turns
+// the words of its 16 particles into a list of neighbours each, in candidate
+// order; a particle's lanes evaluate four entries at a time and add the
+// terms in order through DPP broadcasts, so the sums are the same bits.  Per
+// stage, one lane / four (us, HIP events around it): 16,384 compressed
+// 22.0 / 14.3; at rest density 16,384 21.6 / 14.2, 65,537 from step 10
+// 22.8 / 19.1 and from step 80 24.3 / 20.2, 100,000 23.3 / 25.3, 131,072
+// 23.7 / 28.9.  1 / 2 / 3 / 4 entries a lane and step gave 15.5 / 14.2 /
+// 14.3 / 14.5 at 16,384 and 19.3 / 19.1 / 19.1 / 20.1 at 65,537.
+#define FL_CAP 128  // list entries of a particle: the pairs of four words
+#define FL_STEP 2   // entries a lane and step
+
+// I + the terms of the particle's first nv lanes, in lane order
+__device__ __forceinline__ void add_lanes(ForceI& I, const PairTerm& q, int nv) {
+  auto one = [&](auto kk) __attribute__((always_inline)) {
+    constexpr int K = decltype(kk)::value;
+    if (K < nv) {  // the same for the four lanes
+      const float A = lane_bcast<4, K>(q.A), B = lane_bcast<4, K>(q.B);
+      I.fx = fmaf(A, lane_bcast<4, K>(q.dx), fmaf(B, lane_bcast<4, K>(q.ux), I.fx));
+      I.fy = fmaf(A, lane_bcast<4, K>(q.dy), fmaf(B, lane_bcast<4, K>(q.uy), I.fy));
+      I.fz = fmaf(A, lane_bcast<4, K>(q.dz), fmaf(B, lane_bcast<4, K>(q.uz), I.fz));
+    }
+  };
+  one(std::integral_constant<int, 0>());
+  one(std::integral_constant<int, 1>());
+  one(std::integral_constant<int, 2>());
+  one(std::integral_constant<int, 3>());
+}
+
+template <int SR>
+__device__ __forceinline__ void force_lists(const FParams_t& P, const Span S, int N, const uint* __restrict__ bits,
+                                            int cap, uint* lds) {
+  constexpr int G = 4, R = SR * SR;
+  const int lane = (int)(threadIdx.x & 63u), sub = lane & (G - 1);
+  const int i = S.p0 + (S.blk * (int)blockDim.x + (int)threadIdx.x) / G;
+  // the particle's list; strides of 4 mod 32 words keep the lists of a wave in different banks
+  uint* list = lds + ((threadIdx.x >> 6) * (64 / G) + lane / G) * (FL_CAP + G);
+  const uint* __restrict__ off = pbuf<const uint>(FAccel, AGRIDOFF);
+  const float4* __restrict__ fr = pbuf<const float4>(FAccel, AFREC);
+  const int gc = i < S.p1 ? pbuf<const int>(FPnts, FGCELL)[i] : FX_GRID_UNDEF;
+  const bool act = gc != FX_GRID_UNDEF;
+  if (__ballot(act) == 0ull) return;
+  const int shift = (P.gridRes.z + 1) * P.gridRes.x + 1;
+  ForceI I;
+  I.px = I.py = I.pz = I.vx = I.vy = I.vz = 0.0f;
+  I.di = 1.0f;
+  I.pi = 0.0f;
+  I.fx = I.fy = I.fz = 0.0f;
+  // words [E_[r - 1], E_[r]) of the bitmask are row r's; bit 0 of word f is candidate B_[r] + 32 f
+  int E_[R], B_[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) E_[r] = B_[r] = 0;
+  int nwords = 0;
+  if (act) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int c0 = gc + P.gridAdj[r * SR] - shift;
+      B_[r] = (int)off[c0];
+      E_[r] = (int)off[c0 + SR];
+    }
+    const float4 a = fr[2 * (size_t)i], v = fr[2 * (size_t)i + 1];
+    I.px = a.x; I.py = a.y; I.pz = a.z;
+    I.vx = v.x; I.vy = v.y; I.vz = v.z;
+    I.di = a.w;
+    I.pi = (I.di - P.prest_dens) * P.pintstiff;
+  }
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const int nw = (E_[r] - B_[r] + 31) >> 5;
+    B_[r] -= nwords << 5;
+    nwords += nw;
+    E_[r] = nwords;
+  }
+  if (act && nwords > cap) {  // no recorded bits: test every candidate
+    const int base = stencil_base(P, gc);
+    for (int r = 0; r < R; r++) {
+      int b, e;
+      row_range(P, base, r, off, off, b, e);
+      for (int j = b; j < e; j++) {
+        const float4 a = fr[2 * (size_t)j];
+        if (is_pair(P, I, a)) force_pair(P, I, a, fr[2 * (size_t)j + 1]);
+      }
+    }
+    nwords = 0;
+  }
+  const size_t NN = (size_t)N;
+  int head = 0, qn = 0;  // the list holds entries head .. head + qn - 1 (mod FL_CAP)
+  // G * U entries of the list, the last of them repeated beyond nv
+  auto take = [&](auto uu, int nv) __attribute__((always_inline)) {
+    constexpr int U = decltype(uu)::value;
+    float4 a[U], v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const size_t j = 2 * (size_t)list[(head + min(u * G + sub, nv - 1)) & (FL_CAP - 1)];
+      a[u] = fr[j];
+      v[u] = fr[j + 1];
+    }
+    PairTerm q[U];
+    uint chk = 0u;
+#pragma unroll
+    for (int u = 0; u < U; u++) q[u] = pair_term<true>(P, I, a[u], v[u], chk);
+    if (__any(chk >= FX_NEAR_SPAN)) {
+#pragma unroll
+      for (int u = 0; u < U; u++) q[u] = pair_term<false>(P, I, a[u], v[u], chk);
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) add_lanes(I, q[u], nv - u * G);
+    head += nv;
+    qn -= nv;
+  };
+  // down to fewer than G entries a list, and those too if `all`
+  auto drain = [&](bool all) __attribute__((always_inline)) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");  // other lanes' list entries
+    while (qn >= G * FL_STEP) take(std::integral_constant<int, FL_STEP>(), G * FL_STEP);
+    while (qn >= G || (all && qn > 0)) take(std::integral_constant<int, 1>(), min(qn, G));
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  };
+  const int maxf = wave_max(nwords);
+  uint next = sub < nwords ? __builtin_nontemporal_load(&bits[(size_t)sub * NN + i]) : 0u;
+  for (int f0 = 0; f0 < maxf; f0 += G) {  // a word a lane
+    const int f = f0 + sub;
+    uint m = next;
+    next = f + G < nwords ? __builtin_nontemporal_load(&bits[(size_t)(f + G) * NN + i]) : 0u;
+    int base = B_[0];
+#pragma unroll
+    for (int r = 1; r < R; r++) base = f >= E_[r - 1] ? B_[r] : base;
+    base += f << 5;
+    const int pc = __popc(m);
+    // pairs in the words of the lanes up to this one, and of all four
+    const int p1 = (int)__builtin_amdgcn_update_dpp(0, pc, 0x90, 0xf, 0xf, true);  // quad_perm 0,0,1,2
+    int pre = pc + (sub >= 1 ? p1 : 0);
+    const int p2 = (int)__builtin_amdgcn_update_dpp(0, pre, 0x40, 0xf, 0xf, true);  // quad_perm 0,0,0,1
+    pre += sub >= 2 ? p2 : 0;
+    const int tot = (int)__builtin_amdgcn_update_dpp(0, pre, 0xFF, 0xf, 0xf, true);  // quad_perm 3,3,3,3
+    if (__any(qn + tot > FL_CAP)) drain(false);
+    if (__any(qn + tot > FL_CAP)) drain(true);  // fewer than G held and four full words coming
+    int tail = head + qn + pre - pc;
+    while (m != 0u) {
+      list[tail & (FL_CAP - 1)] = (uint)(base + __builtin_ctz(m));
+      m &= m - 1u;
+      tail++;
+    }
+    qn += tot;
+  }
+  drain(true);
+  if (act && sub == 0) st3(pbuf<fx_float3>(FPnts, FFORCE), (size_t)i, I.fx, I.fy, I.fz);
+}
+
+__device__ __forceinline__ void force_lists_any(const FParams_t& P, const Span S, int N, const uint* bits, int cap) {
+  if (P.gridSrch == 3)
+    force_lists<3>(P, S, N, bits, cap, force_lds);
+  else
+    force_lists<2>(P, S, N, bits, cap, force_lds);
+}
+
+extern "C" __global__ __launch_bounds__(FX_FORCE4_THREADS) void computeForceWave4(int pnum, const uint* bits, int cap,
+                                                                                uint* clear, int nclear) {
+  force_lists_any(*cparams(&FParams), Span{0, pnum, 0, xcd_block()}, pnum, bits, cap);
+  clear_counts(clear, nclear);
+}
+
+extern "C" __global__ __launch_bounds__(FX_FORCE4_THREADS) void computeForceWaveBatch4(BatchArgs B, int ntotal,
+                                                                                     const uint* bits, int cap,
+                                                                                     uint* clear, int nclear) {
+  const FParams_t* P;
+  const Span S = batch_span(B, xcd_block(), P);
+  force_lists_any(*P, S, ntotal, bits, cap);
+  clear_counts(clear, nclear);
+}
+
 // ------------------------------------------------------ neighbour statistics
 
 // The largest number of bitmask words any in-range particle's stencil needs,

@@ -83,6 +83,8 @@ extern "C" {
 /* and of the per-wave force kernels: 16 queued (word, base) pairs a thread */
 #define FX_FORCE_THREADS 512
 #define FX_FORCE_LDS(threads) (128 * (threads))
+#define FX_FORCE4_THREADS 256
+#define FX_FORCE4_LDS(threads) ((threads) / 4 * 132 * 4) /* lists of 128 entries and a pad of 4 */
 #define FX_SLABS 16      /* x slabs per cell: the in-cell order of the ranked sort */
 #define FX_MEMBER_BITS 28 /* AGRID member entries: index in the low 28 bits, x slab above */
 
