@@ -1326,8 +1326,10 @@ __device__ __forceinline__ void density_wave(const FParams_t& P, const Span S, i
   D.acc = 0u;
 #pragma unroll
   for (int r = 0; r < R; r++) jb[r] = len[r] = 0;
+  fx_float3 vev = {0.0f, 0.0f, 0.0f};  // of the record written at the end; loaded there it was waited for (beach 194 -> 186 us)
   if (act) {
     D.p = ld3(pos, (size_t)i);
+    if (sub == G - 1) vev = ld3nt(pbuf<const fx_float3>(FPnts, FVEVAL), (size_t)i);
 #pragma unroll
     for (int r = 0; r < R; r++) {
       const int c0 = gc + P.gridAdj[r * SR] - shift;
@@ -1523,8 +1525,7 @@ __device__ __forceinline__ void density_wave(const FParams_t& P, const Span S, i
     fr[2 * (size_t)i] = make_float4(D.p.x, D.p.y, D.p.z, rho);
   }
   if (sub == G - 1) {
-    const fx_float3 v = ld3nt(pbuf<const fx_float3>(FPnts, FVEVAL), (size_t)i);
-    fr[2 * (size_t)i + 1] = make_float4(v.x, v.y, v.z, 0.0f);
+    fr[2 * (size_t)i + 1] = make_float4(vev.x, vev.y, vev.z, 0.0f);
   }
 }
 
@@ -2218,6 +2219,16 @@ __device__ __forceinline__ void force_lists(const FParams_t& P, const Span S, in
   const uint* __restrict__ off = pbuf<const uint>(FAccel, AGRIDOFF);
   const float4* __restrict__ fr = pbuf<const float4>(FAccel, AFREC);
   const int gc = i < S.p1 ? pbuf<const int>(FPnts, FGCELL)[i] : FX_GRID_UNDEF;
+  // The lane's first three words, beside the cell and before it is known how
+  // many the particle has (the buffer holds cap words of every particle):
+  // 19.2 -> 18.8 us at 65,537 particles.
+  uint w0 = 0u, w1 = 0u, w2 = 0u;
+  if (i < S.p1) {
+    const size_t NN = (size_t)N;
+    if (sub < cap) w0 = __builtin_nontemporal_load(&bits[(size_t)sub * NN + i]);
+    if (sub + G < cap) w1 = __builtin_nontemporal_load(&bits[(size_t)(sub + G) * NN + i]);
+    if (sub + 2 * G < cap) w2 = __builtin_nontemporal_load(&bits[(size_t)(sub + 2 * G) * NN + i]);
+  }
   const bool act = gc != FX_GRID_UNDEF;
   if (__ballot(act) == 0ull) return;
   const int shift = (P.gridRes.z + 1) * P.gridRes.x + 1;
@@ -2296,11 +2307,12 @@ __device__ __forceinline__ void force_lists(const FParams_t& P, const Span S, in
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
   };
   const int maxf = wave_max(nwords);
-  uint next = sub < nwords ? __builtin_nontemporal_load(&bits[(size_t)sub * NN + i]) : 0u;
   for (int f0 = 0; f0 < maxf; f0 += G) {  // a word a lane
     const int f = f0 + sub;
-    uint m = next;
-    next = f + G < nwords ? __builtin_nontemporal_load(&bits[(size_t)(f + G) * NN + i]) : 0u;
+    uint m = f < nwords ? w0 : 0u;
+    w0 = w1;
+    w1 = w2;
+    w2 = f + 3 * G < nwords ? __builtin_nontemporal_load(&bits[(size_t)(f + 3 * G) * NN + i]) : 0u;
     int base = B_[0];
 #pragma unroll
     for (int r = 1; r < R; r++) base = f >= E_[r - 1] ? B_[r] : base;
