@@ -75,7 +75,6 @@ struct AdjArgs {
   void* gF;
   void* gxs;
   void* ges;
-  void* grho;
   void* partial;
   void* arec;
   void* drec;
@@ -88,7 +87,7 @@ struct AdjArgs {
 
 const size_t kCkptBytes = 44;   // pos, vel, veval (12 B each), clr, id (4 B each)
 const size_t kTapeBytes = 60;   // pos, vel, veval, force (12 B each), rho, sort permutation, gcell (4 B each)
-const size_t kVecFloats = 34;   // floats per particle of m_AdjVec
+const size_t kVecFloats = 33;   // floats per particle of m_AdjVec
 // plus, per recorded step, the density kernel's neighbour bitmask
 // (m_AdjWords words per particle), written there directly by the forward
 
@@ -272,7 +271,7 @@ int Particles::AdjConfigure(const char* path, int nsteps, int every) {
   FX_HIP(hipMemcpyHtoD(m_AdjBFirst, first.data(), first.size() * sizeof(int)), "adjoint");
   FX_HIP(hipMemcpyHtoD(m_AdjPBase, m_PBase.data(), sizeof(int) * (size_t)(scenes + 1)), "adjoint");
   // target defaults to zero
-  FX_HIP(hipMemset(m_AdjVec + (size_t)n * 19, 0, sizeof(float) * 3 * (size_t)n), "adjoint");
+  FX_HIP(hipMemset(m_AdjVec + (size_t)n * 18, 0, sizeof(float) * 3 * (size_t)n), "adjoint");
   m_AdjSteps = nsteps;
   m_AdjEvery = every;
   m_AdjSegs = segs;
@@ -299,7 +298,7 @@ int Particles::AdjSetTarget(const float* target, int64_t count) {
   if (m_AdjN == 0) return fx::fail(FX_ESTATE, "adjoint: call fx_adjoint_configure first");
   if (target == nullptr || count != (int64_t)m_AdjN)
     return fx::fail(FX_EINVAL, "adjoint: the target holds one position per particle (%d)", m_AdjN);
-  return m_Staging.up(m_AdjVec + (size_t)m_AdjN * 19, target, sizeof(float) * 3 * (size_t)count,
+  return m_Staging.up(m_AdjVec + (size_t)m_AdjN * 18, target, sizeof(float) * 3 * (size_t)count,
                       "adjoint: target upload");
 }
 
@@ -398,8 +397,8 @@ int Particles::AdjForward(double* loss, double* ms) {
   }
   {  // the rollout frame: FID := slot, the target follows
     void* fid = m_Points.gpu(FID);
-    float* tgt = m_AdjVec + 19 * (size_t)m_AdjN;
-    float* tgf = m_AdjVec + 22 * (size_t)m_AdjN;
+    float* tgt = m_AdjVec + 18 * (size_t)m_AdjN;
+    float* tgf = m_AdjVec + 21 * (size_t)m_AdjN;
     int nn = m_AdjN;
     void* a[] = {&fid, &m_AdjId0, &tgt, &tgf, &nn};
     FX_TRY(launch_n(m_AdjFunc[ADJ_FRAME_IN], kAdjNames[ADJ_FRAME_IN], m_Stream, nn, a));
@@ -429,7 +428,7 @@ int Particles::AdjForward(double* loss, double* ms) {
   A.btab = m_AdjBTab;
   A.pos = m_Points.gpu(FPOS);
   A.id = m_Points.gpu(FID);
-  A.target = V + 22 * n;
+  A.target = V + 21 * n;
   A.gx = V;
   A.gv = V + 3 * n;
   A.ge = V + 6 * n;
@@ -505,7 +504,7 @@ int Particles::AdjBackward(float* gpos, float* gvel, float* gveval, double* gvis
   FX_TRY(AdjSortSrc(true));
   // the adjoint state alternates between two sets: [cur] holds that of the
   // step's outputs, the step writes that of its inputs into [cur ^ 1]
-  float* set[2] = {V, V + 25 * n};
+  float* set[2] = {V, V + 24 * n};
   int cur = 0;
   auto held = [&](int sg) { return m_AdjBufSeg[sg % m_AdjBufs] == sg; };
   if (m_AdjSegs > 0 && !held(m_AdjSegs - 1)) FX_TRY(AdjRecompute(m_AdjSegs - 1));
@@ -531,7 +530,7 @@ int Particles::AdjBackward(float* gpos, float* gvel, float* gveval, double* gvis
       A.id = T + 52 * n;
       A.gcell = T + 56 * n;
       A.off = T + 60 * n;
-      A.target = V + 22 * n;
+      A.target = V + 21 * n;
       A.gx = set[cur];
       A.gv = set[cur] + 3 * n;
       A.ge = set[cur] + 6 * n;
@@ -541,7 +540,6 @@ int Particles::AdjBackward(float* gpos, float* gvel, float* gveval, double* gvis
       A.gF = V + 9 * n;
       A.gxs = V + 12 * n;
       A.ges = V + 15 * n;
-      A.grho = V + 18 * n;
       A.partial = m_AdjPartial;
       A.arec = m_AdjArec;
       A.drec = m_AdjDrec;

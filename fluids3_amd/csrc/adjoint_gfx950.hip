@@ -22,9 +22,10 @@
 //                 gx_i   += A dl + (d2/r) u (A_r (u.dl) + B_r (dve.dl))
 //                 ge_i   -= B dl
 //                 grho_i += kp c^2 inv k (u.dl) - (A (u.dl) + B (dve.dl)) / rho_i
-//               and the per-particle terms of dL/dk and dL/dvisc;
+//               and the per-particle terms of dL/dk and dL/dvisc; ge of the
+//               inputs goes to src[s];
 //   adjDensity  gx_i += sum_j (grho_i + grho_j) (-6 m poly6 d2) t^2 u, then
-//               the step's input adjoints go to src[s].
+//               gx of the inputs goes to src[s].
 // Every pair term is gathered from i's side (A and B are symmetric in i, j),
 // so there are no atomics and results are reproducible bit for bit.  FP64 is
 // used only for the loss and the two scalar-parameter sums: per-block FP64
@@ -88,7 +89,6 @@ struct AdjArgs {
   fx_float3* gF;
   fx_float3* gxs;
   fx_float3* ges;
-  float* grho;
   double* partial;  // 3 doubles per launched block: loss, dL/dk, dL/dvisc
   float4* arec;     // per slot: (pos, rho), (veval, 0), (gF, 0), written by adjAdvance
   float4* drec;     // per slot: (pos, grho), written by adjForce
@@ -572,7 +572,7 @@ __device__ __forceinline__ bool pair_walk(const FParams_t& P, const AdjArgs& A, 
 // gathers (three 16-byte records a pair, two of them read by neighbouring
 // lanes together) and the roots are the forward force's.  Per launch, with a
 // queue that read its words when it needed them, plain gathers and IEEE roots
-// before / now: 262,144 particles 49 / 41 us, 12 scenes 158 / 146.
+// before / now: 262,144 particles 49 / 41 us, 12 scenes 158 / 145.
 struct ForceAdj {
   const FParams_t* P;
   const float4* rec;  // (pos, rho), (veval, 0), (gF, 0) per slot
@@ -727,14 +727,16 @@ extern "C" __global__ void __launch_bounds__(ADJ_THREADS) adjForce(AdjArgs A) {
       }
     }
   }
-  if (act) {
-    const fx_float3 x0 = A.gxs[i], e0 = A.ges[i];
-    A.gxs[i] = fx_float3{x0.x + F.gpx, x0.y + F.gpy, x0.z + F.gpz};
-    A.ges[i] = fx_float3{e0.x + F.gex, e0.y + F.gey, e0.z + F.gez};
-    A.grho[i] = F.gr;
-    A.drec[i] = make_float4(F.px, F.py, F.pz, F.gr);
-  } else if (i < S.p1) {
-    A.grho[i] = 0.0f;
+  if (i < S.p1) {
+    // ge is complete here and goes where the inputs' adjoint is kept
+    fx_float3 e = A.ges[i];
+    if (act) {
+      const fx_float3 x0 = A.gxs[i];
+      A.gxs[i] = fx_float3{x0.x + F.gpx, x0.y + F.gpy, x0.z + F.gpz};
+      A.drec[i] = make_float4(F.px, F.py, F.pz, F.gr);
+      e = fx_float3{e.x + F.gex, e.y + F.gey, e.z + F.gez};
+    }
+    A.gep[A.id[i]] = e;
   }
   const double sk = wave_sum((double)F.ak);
   const double sv = wave_sum((double)F.av);
@@ -750,14 +752,14 @@ extern "C" __global__ void __launch_bounds__(ADJ_THREADS) adjForce(AdjArgs A) {
 // Pair term of the density adjoint: about 15 instructions a pair beside the
 // walk's 20, and one 16-byte gather; the gathers in flight bound it, hence
 // eight to a step.  Per launch before / now (the queue as above): 262,144
-// particles 28 / 18 us, 12 scenes 70 / 63.
+// particles 28 / 17 us, 12 scenes 70 / 58 (18 and 63 while it also moved ge).
 struct DensityAdj {
   const float4* rec;  // (pos, grho) per slot
   float px, py, pz, gi, d2, rd2, k6;
   float gpx, gpy, gpz;
 
   static constexpr uint MUL = 1;
-  static constexpr int STEP = 8;  // 4 / 6 / 8: 18.7 / 18.3 / 18.1 us at 262,144 particles, 68 / 64 / 63 for 12 scenes
+  static constexpr int STEP = 8;  // 4 / 6 / 8: 18.7 / 18.3 / 18.1 us at 262,144 particles, 68 / 64 / 63 for 12 scenes (ge moved too)
   __device__ __forceinline__ void eval(uint j, bool ok) { apply(rec[j], ok); }
   __device__ __forceinline__ void step(const uint (&j)[STEP], const bool (&ok)[STEP]) {
     float4 a[STEP];
@@ -815,7 +817,6 @@ extern "C" __global__ void __launch_bounds__(ADJ_THREADS) adjDensity(AdjArgs A) 
   const uint src = A.id[i];
   const fx_float3 x0 = A.gxs[i];
   A.gxp[src] = fx_float3{x0.x + D.gpx, x0.y + D.gpy, x0.z + D.gpz};
-  A.gep[src] = A.ges[i];
 }
 
 // ----------------------------------------------------------------- reduce

@@ -310,7 +310,7 @@ class Particles {
   void* m_AdjArec = nullptr;             // 48 B x N pair records of the force adjoint
   void* m_AdjDrec = nullptr;             // 16 B x N pair records of the density adjoint
   void* m_AdjTabs = nullptr;             // FAccel tables routing ANBRBITS into the tape
-  float* m_AdjVec = nullptr;             // gx, gv, ge, gF, gxs, ges (3N floats each), grho (N), target,
+  float* m_AdjVec = nullptr;             // gx, gv, ge, gF, gxs, ges (3N floats each), target,
                                          // target in the rollout frame (3N each), a second gx, gv, ge
   uint32_t* m_AdjId0 = nullptr;          // original id of each slot at the rollout's start
   uint32_t* m_AdjSrc = nullptr;          // the last sort's permutation (the module's FSortSrc points here
