@@ -350,19 +350,19 @@ int Particles::AdjStep(int record_slot, bool first, bool last) {
     FX_HIP(hipMemcpyAsync(m_Accel.SymbolAddress(), tabs + sizeof(cuDataX) * (size_t)(record_slot + 1),
                           sizeof(cuDataX), hipMemcpyDeviceToDevice, m_Stream), "tape");
   }
-  FX_TRY(ComputePressure(bits));
-  FX_TRY(ComputeForce(joined && !last, bits));
+  char* t = m_AdjTape + TapeStep() * (size_t)(rec ? record_slot : 0);
+  NextStep next;
+  next.mode = !joined || last ? 0 : rec ? 2 : 1;
+  next.tape = {t, m_AdjSrc, m_AdjN, m_AdjCells};
+  FX_TRY(ComputePressure(bits, next.mode != 0));
+  FX_TRY(ComputeForce(bits, next));
   if (rec && !wave) {
     FX_HIP(hipMemcpyAsync(m_Accel.SymbolAddress(), tabs, sizeof(cuDataX), hipMemcpyDeviceToDevice, m_Stream),
            "tape");
     FX_HIP(hipMemcpyAsync(m_NbrWordsSym, m_AdjWordCaps, sizeof(int), hipMemcpyDeviceToDevice, m_Stream), "tape");
   }
-  char* t = m_AdjTape + TapeStep() * (size_t)(rec ? record_slot : 0);
   if (rec) m_AdjTapeTime[record_slot] = m_Params.time;
-  if (joined && !last) {
-    TapeSlot slot = {t, m_AdjSrc, m_AdjN, m_AdjCells};
-    FX_TRY(AdvanceInsert(rec ? &slot : nullptr));
-  } else {
+  if (next.mode == 0) {
     if (rec) {
       // pos, vel, veval, force, rho, permutation, gcell, then the cell offsets: one kernel
       TapeSrc src = {{m_Points.gpu(FPOS), m_Points.gpu(FVEL), m_Points.gpu(FVEVAL), m_Points.gpu(FFORCE)},

@@ -25,8 +25,7 @@ static const char* kKernelNames[FUNC_MAX] = {
     "computeForceBatchP", "advanceParticlesBatchP", "fxScanSums", "fxScanApply",
     "computePressureWave1", "computePressureWave2", "computePressureWave4",
     "computePressureWaveBatch1", "computePressureWaveBatch2", "computePressureWaveBatch4",
-    "computeForceWave",  "computeForceWaveBatch", "advanceInsert", "advanceInsertBatch",
-    "advanceInsertTape", "advanceInsertTapeBatch", "computeForceWave4", "computeForceWaveBatch4"};
+    "computeForceWave",  "computeForceWaveBatch", "computeForceWave4", "computeForceWaveBatch4"};
 
 Particles::Particles() { memset(&m_Params, 0, sizeof(m_Params)); }
 
@@ -665,10 +664,11 @@ int Particles::SortKernels() {
   return FX_OK;
 }
 
-int Particles::ComputePressure(NbrBits bits) {
+int Particles::ComputePressure(NbrBits bits, bool clear) {
   if (WaveStages()) {
     const int lanes = DensityLanes(), t = StageThreads(FX_STAGE_PRESSURE, FX_DENS_THREADS), v = lanes == 4 ? 2 : lanes - 1;
-    FX_TRY(LaunchLanes(FUNC_PRESS_W + v, FUNC_PRESS_WB + v, t, lanes, FX_DENS_LDS(t), bits));
+    void* cnt = clear ? m_Accel.gpu(AGRIDCNT) : nullptr;  // counts cleared for the next step's insert
+    FX_TRY(LaunchLanes(FUNC_PRESS_W + v, FUNC_PRESS_WB + v, t, lanes, FX_DENS_LDS(t), bits, &cnt, &m_ScanCells));
   } else if (m_Batch) {
     FX_TRY(BatchLaunch(FUNC_PRESS_B, FUNC_PRESS_BP, FX_STAGE_PRESSURE, &mNumPoints, nullptr, nullptr));
   } else {
@@ -679,13 +679,16 @@ int Particles::ComputePressure(NbrBits bits) {
   return FX_OK;
 }
 
-int Particles::ComputeForce(bool clear, NbrBits bits) {
+int Particles::ComputeForce(NbrBits bits, NextStep next) {
   if (WaveStages()) {
     const bool four = ForceLanes() == 4;
     const int t = StageThreads(FX_STAGE_FORCE, four ? FX_FORCE4_THREADS : FX_FORCE_THREADS);
-    void* cnt = clear ? m_Accel.gpu(AGRIDCNT) : nullptr;  // counts cleared for the next step's insert
+    next.time = m_Params.time;
+    next.dt = m_Params.dt;
+    next.ss = m_Params.sim_scale;
+    next.clock = m_Capturing ? m_Clock : nullptr;
     FX_TRY(LaunchLanes(four ? FUNC_FORCE_W4 : FUNC_FORCE_W, four ? FUNC_FORCE_WB4 : FUNC_FORCE_WB, t, four ? 4 : 1,
-                       four ? FX_FORCE4_LDS(t) : FX_FORCE_LDS(t), bits, &cnt, &m_ScanCells));
+                       four ? FX_FORCE4_LDS(t) : FX_FORCE_LDS(t), bits, &next, nullptr));
   } else if (m_Batch) {
     FX_TRY(BatchLaunch(FUNC_FORCE_B, FUNC_FORCE_BP, FX_STAGE_FORCE, &mNumPoints, nullptr, nullptr));
   } else {
@@ -751,8 +754,8 @@ int Particles::Stage(int stage) {
   }
 }
 
-// Whether a step's advance may also make the next step's insert: one particle
-// per thread in both, and the per-wave stages, whose force clears the counts.
+// Whether a step's force may also advance and make the next step's insert: the
+// per-wave stages, and one particle per thread in the passes it replaces.
 bool Particles::JoinedSteps() const {
   return WaveStages() && m_StagePpt[FX_STAGE_INSERT] == 1 && m_StagePpt[FX_STAGE_ADVANCE] == 1;
 }
@@ -762,10 +765,12 @@ bool Particles::JoinedSteps() const {
 // sort, as a step alone does.
 int Particles::Step(bool first, bool last) {
   const bool joined = JoinedSteps();
+  NextStep next;
+  next.mode = joined && !last ? 1 : 0;
   FX_TRY(SortStep(first || !joined));
-  FX_TRY(ComputePressure());
-  FX_TRY(ComputeForce(joined && !last));
-  FX_TRY(joined && !last ? AdvanceInsert() : Advance());
+  FX_TRY(ComputePressure(NbrBits(), next.mode != 0));
+  FX_TRY(ComputeForce(NbrBits(), next));
+  if (next.mode == 0) FX_TRY(Advance());
   m_Done = FX_STAGE_ADVANCE;
   return FX_OK;
 }
@@ -777,19 +782,6 @@ int Particles::SortStep(bool insert) {
   m_Parity ^= 1;
   FX_TRY(ScanGrid(true));
   return SortKernels();
-}
-
-int Particles::AdvanceInsert(TapeSlot* tape) {
-  float dt = m_Params.dt, ss = m_Params.sim_scale, time = m_Params.time;
-  void* clk = m_Capturing ? (void*)m_Clock : nullptr;
-  if (tape != nullptr) {
-    if (m_Batch) return BatchLaunch(FUNC_ADVANCE_TAPE_B, 0, FX_STAGE_INSERT, &time, tape, nullptr);
-    void* args[] = {&time, &dt, &ss, &mNumPoints, tape};
-    return LaunchP(FUNC_ADVANCE_TAPE, FX_STAGE_INSERT, args);
-  }
-  if (m_Batch) return BatchLaunch(FUNC_ADVANCE_INSERT_B, 0, FX_STAGE_INSERT, &clk, &time, nullptr);
-  void* args[] = {&clk, &time, &dt, &ss, &mNumPoints};
-  return LaunchP(FUNC_ADVANCE_INSERT, FX_STAGE_INSERT, args);
 }
 
 int Particles::Run(int nsteps) {

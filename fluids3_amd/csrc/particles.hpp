@@ -63,13 +63,9 @@
 #define FUNC_PRESS_WB 35   // the same for a batch
 #define FUNC_FORCE_W 38    // per-wave force
 #define FUNC_FORCE_WB 39
-#define FUNC_ADVANCE_INSERT 40  // a step's advance and the next one's insert
-#define FUNC_ADVANCE_INSERT_B 41
-#define FUNC_ADVANCE_TAPE 42    // the same, recording the step on a rollout's tape
-#define FUNC_ADVANCE_TAPE_B 43
-#define FUNC_FORCE_W4 44        // per-wave force, four lanes to a particle
-#define FUNC_FORCE_WB4 45
-#define FUNC_MAX 46
+#define FUNC_FORCE_W4 40        // per-wave force, four lanes to a particle
+#define FUNC_FORCE_WB4 41
+#define FUNC_MAX 42
 
 #include <map>
 #include <string>
@@ -101,6 +97,16 @@ struct TapeSlot {
   const void* src;
   int n;
   int cells;
+};
+
+// FxNext of the kernel file: what the per-wave force launch does after the
+// forces (nothing; the advance and the next step's insert; the tape before
+// them).
+struct NextStep {
+  int mode = 0;
+  float time = 0.0f, dt = 0.0f, ss = 0.0f;
+  const float* clock = nullptr;
+  TapeSlot tape = {};
 };
 
 class Particles {
@@ -139,9 +145,9 @@ class Particles {
   int InsertParticles();
   int PrefixScanParticles();
   int CountingSort();
-  int ComputePressure(NbrBits bits = NbrBits());
-  // clear: zero the cell counts for an insert that follows (WaveStages only)
-  int ComputeForce(bool clear = false, NbrBits bits = NbrBits());
+  // clear: zero the cell counts for the insert that the force makes (WaveStages only, as next)
+  int ComputePressure(NbrBits bits = NbrBits(), bool clear = false);
+  int ComputeForce(NbrBits bits = NbrBits(), NextStep next = NextStep());
   int Advance();
   void AdvanceTime();
   int Stage(int stage);
@@ -202,7 +208,6 @@ class Particles {
   bool JoinedSteps() const;
   int Step(bool first, bool last);
   int SortStep(bool insert);
-  int AdvanceInsert(TapeSlot* tape = nullptr);
   int SetDeviceClock();
   int CapturePair(int inner);
   int ReplayGraph(int nlaunch);

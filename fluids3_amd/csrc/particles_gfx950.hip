@@ -87,6 +87,21 @@ __device__ __forceinline__ void st3(fx_float3* __restrict__ p, size_t i, float x
   f[1] = y;
   f[2] = z;
 }
+// Nt: non-temporal stores
+template <bool Nt, class T>
+__device__ __forceinline__ void put(T* p, T v) {
+  if (Nt)
+    __builtin_nontemporal_store(v, p);
+  else
+    *p = v;
+}
+template <bool Nt>
+__device__ __forceinline__ void put3(fx_float3* __restrict__ p, size_t i, float x, float y, float z) {
+  float* f = reinterpret_cast<float*>(p) + 3 * i;
+  put<Nt>(f, x);
+  put<Nt>(f + 1, y);
+  put<Nt>(f + 2, z);
+}
 
 __device__ __forceinline__ const FParams_t* cparams(const FParams_t* p) {
   typedef const __attribute__((address_space(4))) FParams_t cP;
@@ -277,10 +292,10 @@ extern "C" __global__ void fxMark(int tag) {}
 // of atomics on that one address.  `tl` is the block's LDS (two sets of 17
 // words, alternating between calls so that one call's reads cannot meet
 // the next call's writes).
-__device__ __forceinline__ void insert_at(const FParams_t& P, const Span S, const fx_float3 p, bool tail,
-                                          uint (*tl)[17]) {
-  const int i = S.p0 + S.blk * (int)blockDim.x + (int)threadIdx.x;
-  bool active = i < S.p1;  // below: particles that take a count slot
+template <bool Nt>
+__device__ __forceinline__ void insert_at(const FParams_t& P, const Span S, int i, bool active, const fx_float3 p,
+                                          bool tail, uint (*tl)[17]) {
+  // active: the lane has particle i, at p; below, one that takes a count slot
   int gs = 0;
   if (active) {
     const float gx = (p.x - P.gridMin.x) * P.gridDelta.x;
@@ -290,14 +305,14 @@ __device__ __forceinline__ void insert_at(const FParams_t& P, const Span S, cons
                     gy < (float)(P.gridScanMax.y + 1) && gz >= 1.0f && gz < (float)(P.gridScanMax.z + 1);
     if (in) {
       gs = S.c0 + ((int)gy * P.gridRes.z + (int)gz) * P.gridRes.x + (int)gx;
-      pbuf<int>(FPnts, FGCELL)[i] = gs;
+      put<Nt>(&pbuf<int>(FPnts, FGCELL)[i], gs);
     } else {
       gs = S.c0 + P.gridTotal;
-      pbuf<int>(FPnts, FGCELL)[i] = FX_GRID_UNDEF;
+      put<Nt>(&pbuf<int>(FPnts, FGCELL)[i], (int)FX_GRID_UNDEF);
       active = tail;
     }
     uint* tflag = pbuf<uint>(FAccel, ATAILFLAG);
-    if (tflag != nullptr) tflag[i] = in ? 0u : 1u;
+    if (tflag != nullptr) put<Nt>(&tflag[i], in ? 0u : 1u);
   }
   uint* cnt = pbuf<uint>(FAccel, AGRIDCNT);
   const int tslot = S.c0 + P.gridTotal;
@@ -344,14 +359,14 @@ __device__ __forceinline__ void insert_at(const FParams_t& P, const Span S, cons
     base = tbase;
     mine = tm;
   }
-  if (active) pbuf<int>(FPnts, FGNDX)[i] = (int)(base + lanes_below(mine));
+  if (active) put<Nt>(&pbuf<int>(FPnts, FGNDX)[i], (int)(base + lanes_below(mine)));
 }
 
 __device__ __forceinline__ void insert_impl(const FParams_t& P, const Span S, bool tail, uint (*tl)[17]) {
   const int i = S.p0 + S.blk * (int)blockDim.x + (int)threadIdx.x;
   fx_float3 p = fx_float3{0.0f, 0.0f, 0.0f};
   if (i < S.p1) p = ld3(pbuf<const fx_float3>(FPnts, FPOS), (size_t)i);
-  insert_at(P, S, p, tail, tl);
+  insert_at<false>(P, S, i, i < S.p1, p, tail, tl);
 }
 
 // The streaming kernels keep a straight-line body for one particle per
@@ -1396,7 +1411,6 @@ __device__ __forceinline__ void density_wave(const FParams_t& P, const Span S, i
   };
   // a row on its own: the lane walks candidates [ts, te) (see "Row trimming"),
   // those every lane has unchecked; its words carry the phase ts % 32
-  const uint* __restrict__ cnt = pbuf<const uint>(FAccel, AGRIDCNT);
   const uint* __restrict__ sstart = pbuf<const uint>(FAccel, ASLABSTART);
   int slo = 0, shi = FX_SLABS;
   if (total > FX_DENS_TILE) {
@@ -1410,7 +1424,7 @@ __device__ __forceinline__ void density_wave(const FParams_t& P, const Span S, i
     int ts = 0, te = L0;
     if (act && sstart != nullptr && L0 > FX_RANK_WAVE) {
       const int c0 = gc + P.gridAdj[r * SR] - shift, c2 = c0 + SR - 1;
-      const int n0 = (int)cnt[c0], n2 = (int)cnt[c2];
+      const int n0 = (int)off[c0 + 1] - jbr, n2 = jbr + L0 - (int)off[c2];  // the counts, which this launch clears
       if (n0 > FX_RANK_WAVE && n0 <= FX_RANK_CAP) ts = slab_start(sstart, c0, n0, slo);
       if (n2 > FX_RANK_WAVE && n2 <= FX_RANK_CAP) te = max(ts, te - n2 + slab_start(sstart, c2, n2, shi));
     }
@@ -1539,17 +1553,27 @@ __device__ __forceinline__ void density_wave_any(const FParams_t& P, const Span 
     density_wave<G, 2>(P, S, N, bits, cap, dens_lds);
 }
 
+// Clears n counts, spread over the launch, for the next step's insert, which
+// the force launch of this step makes (force_end).  No stage after the sort
+// reads them.  After the walk: before a pair walk it costs registers.
+__device__ __forceinline__ void clear_counts(uint* __restrict__ p, int n) {
+  if (p == nullptr) return;
+  for (int k = (int)(blockIdx.x * blockDim.x + threadIdx.x); k < n; k += (int)(gridDim.x * blockDim.x)) p[k] = 0u;
+}
+
 // bits: cap words of bitmask a particle (the system's buffer, or a rollout's tape)
 #define FX_DENSITY_WAVE(G)                                                                                    \
-  extern "C" __global__ __launch_bounds__(FX_DENS_THREADS) void computePressureWave##G(int pnum, uint* bits,  \
-                                                                                     int cap) {               \
+  extern "C" __global__ __launch_bounds__(FX_DENS_THREADS) void computePressureWave##G(                       \
+      int pnum, uint* bits, int cap, uint* clear, int nclear) {                                               \
     density_wave_any<G>(*cparams(&FParams), Span{0, pnum, 0, xcd_block()}, pnum, bits, cap);                  \
+    clear_counts(clear, nclear);                                                                              \
   }                                                                                                           \
   extern "C" __global__ __launch_bounds__(FX_DENS_THREADS) void computePressureWaveBatch##G(                  \
-      BatchArgs B, int ntotal, uint* bits, int cap) {                                                         \
+      BatchArgs B, int ntotal, uint* bits, int cap, uint* clear, int nclear) {                                \
     const FParams_t* P;                                                                                       \
     const Span S = batch_span(B, xcd_block(), P);                                                             \
     density_wave_any<G>(*P, S, ntotal, bits, cap);                                                            \
+    clear_counts(clear, nclear);                                                                              \
   }
 FX_DENSITY_WAVE(1)
 FX_DENSITY_WAVE(2)
@@ -2014,6 +2038,88 @@ extern "C" __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu
   });
 }
 
+// ------------------------------------------------------ the step's last pass
+//
+// When another step follows, the force launch also advances its particles and
+// makes the next step's insert (and, in a recorded step of a rollout, writes
+// the particles as they are before the advance to the tape): a particle's
+// position and evaluation velocity are at hand as its pair record, its force
+// need not go through memory, and the passes' traffic lies beside other
+// waves' pair arithmetic.  Neighbours are read from the records and the
+// offsets only, which neither changes; the counts were cleared by the density
+// launch.  What this pass writes is not read before the next launch and is
+// stored non-temporally, so that it does not displace the records (4M
+// particles on the beach, a step from step 20 751 -> 721 us, from step 80
+// 1143 -> 1109).  Against passes of their own for the advance with the insert
+// (which took 75 us of 1034 at the beach): 43.2 -> 39.9 us a step at 16,384
+// particles, 110 -> 105 at 262,144, 214 -> 210 at 1,000,000, at the 4M beach
+// 731 -> 721 and 1115 -> 1109.
+
+// a tape slot, in the layout of adjTapeRecord: pos, vel, veval, force (12 B
+// each), rho, the sort's permutation, cell (4 B each), then the cell offsets
+struct TapeDst {
+  char* dst;
+  const uint* src;  // the sort's permutation
+  int n;
+  int cells;
+};
+
+// what follows the forces: nothing (0), the advance and the next insert (1),
+// the tape before them (2); dt and scale of a batch are its scenes'
+struct FxNext {
+  int mode;
+  float time, dt, ss;
+  const float* clock;
+  TapeDst tape;
+};
+
+__device__ __forceinline__ void tape_store(const TapeDst& T, int i, bool own) {
+  const size_t N = (size_t)T.n;
+  if (own) {
+    const fx_float3 x = ld3(pbuf<const fx_float3>(FPnts, FPOS), (size_t)i);
+    const fx_float3 v = ld3(pbuf<const fx_float3>(FPnts, FVEL), (size_t)i);
+    const fx_float3 e = ld3(pbuf<const fx_float3>(FPnts, FVEVAL), (size_t)i);
+    const fx_float3 f = ld3(pbuf<const fx_float3>(FPnts, FFORCE), (size_t)i);
+    st3(reinterpret_cast<fx_float3*>(T.dst), (size_t)i, x.x, x.y, x.z);
+    st3(reinterpret_cast<fx_float3*>(T.dst + 12 * N), (size_t)i, v.x, v.y, v.z);
+    st3(reinterpret_cast<fx_float3*>(T.dst + 24 * N), (size_t)i, e.x, e.y, e.z);
+    st3(reinterpret_cast<fx_float3*>(T.dst + 36 * N), (size_t)i, f.x, f.y, f.z);
+    uint* w = reinterpret_cast<uint*>(T.dst + 48 * N);
+    w[i] = __float_as_uint(pbuf<const float>(FPnts, FPRESS)[i]);
+    w[N + i] = T.src[i];
+    w[2 * N + i] = pbuf<const uint>(FPnts, FGCELL)[i];
+  }
+  const uint* __restrict__ off = pbuf<const uint>(FAccel, AGRIDOFF);
+  uint* o = reinterpret_cast<uint*>(T.dst + 60 * N);
+  for (int k = (int)(blockIdx.x * blockDim.x + threadIdx.x); k < T.cells; k += (int)(gridDim.x * blockDim.x)) o[k] = off[k];
+}
+
+template <bool Nt>
+__device__ __forceinline__ fx_float3 advance_from(const FParams_t& P, int i, const fx_float3 pos, fx_float3 vel,
+                                                  const fx_float3 ve, const fx_float3 f, float time, float dt,
+                                                  float ss);
+__device__ __forceinline__ fx_float3 park(int i);
+
+// Every thread of the block calls it; own: the lane writes particle i, in
+// cell gc, with the forces in I.  lds: 34 words of the block's LDS.
+__device__ __forceinline__ void force_end(const FParams_t& P, const Span S, int i, bool own, int gc, const ForceI& I,
+                                          const FxNext& X, float dt, float ss, uint* lds) {
+  const bool act = own && gc != FX_GRID_UNDEF;
+  if (X.mode != 1 && act) st3(pbuf<fx_float3>(FPnts, FFORCE), (size_t)i, I.fx, I.fy, I.fz);
+  if (X.mode == 0) return;
+  if (X.mode == 2) tape_store(X.tape, i, own);
+  fx_float3 x = fx_float3{0.0f, 0.0f, 0.0f};
+  if (act) {
+    x = advance_from<true>(P, i, fx_float3{I.px, I.py, I.pz}, ld3nt(pbuf<const fx_float3>(FPnts, FVEL), (size_t)i),
+                           fx_float3{I.vx, I.vy, I.vz}, fx_float3{I.fx, I.fy, I.fz},
+                           X.clock != nullptr ? X.clock[0] : X.time, dt, ss);
+  } else if (own) {
+    x = park(i);
+  }
+  lds_barrier();  // the waves' queues in the block's LDS are done with
+  insert_at<true>(P, S, i, own, x, true, reinterpret_cast<uint(*)[17]>(lds));
+}
+
 // ----------------------------------------------------------- force by wave
 //
 // The library's own force stage (stencil rows of 2 or 3 cells): the word
@@ -2050,26 +2156,19 @@ extern "C" __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu
 #define FQ_STEP 4 // pairs a lane and step
 
 template <int SR>
-__device__ __forceinline__ void force_wave(const FParams_t& P, const Span S, int N, const uint* __restrict__ bits,
-                                           int cap, uint* lds) {
+__device__ __forceinline__ void force_wave(const FParams_t& P, int i, int gc, int N, const uint* __restrict__ bits,
+                                           int cap, uint* lds, ForceI& I) {
   constexpr int R = SR * SR;
   const int lane = (int)(threadIdx.x & 63u);
   const bool odd = (lane & 1) != 0;
-  const int i = S.p0 + S.blk * (int)blockDim.x + (int)threadIdx.x;
   uint* q = lds + (threadIdx.x >> 6) * (2 * FX_WALK_K * 64) + lane;
   const uint* __restrict__ off = pbuf<const uint>(FAccel, AGRIDOFF);
   const uint* __restrict__ cell = pbuf<const uint>(FAccel, AGRIDCNT);
   const float4* __restrict__ fr = pbuf<const float4>(FAccel, AFREC);
   const float4* __restrict__ half = fr + (odd ? 1 : 0);  // the half of a record this lane reads
-  const int gc = i < S.p1 ? pbuf<const int>(FPnts, FGCELL)[i] : FX_GRID_UNDEF;
   const bool act = gc != FX_GRID_UNDEF;
   if (__ballot(act) == 0ull) return;
   const int shift = (P.gridRes.z + 1) * P.gridRes.x + 1;
-  ForceI I;
-  I.px = I.py = I.pz = I.vx = I.vy = I.vz = 0.0f;
-  I.di = 1.0f;
-  I.pi = 0.0f;
-  I.fx = I.fy = I.fz = 0.0f;
   // row r: candidates from jb[r], words [E_[r - 1], E_[r]) of the bitmask
   int jb[R], E_[R];
 #pragma unroll
@@ -2140,41 +2239,42 @@ __device__ __forceinline__ void force_wave(const FParams_t& P, const Span S, int
       for (int u = 0; u < FQ_STEP; u++) pair_add_if(I, t[u], ok[u]);
     }
   });
-  if (act) st3(pbuf<fx_float3>(FPnts, FFORCE), (size_t)i, I.fx, I.fy, I.fz);
 }
 
 extern __shared__ uint force_lds[];  // FX_FORCE_LDS(threads) bytes
 
-// Clears n counts, spread over the launch: no stage after the density reads
-// them, and the advance of this step also makes the next step's insert.
-// After the pairs: before them it cost the batch kernel five registers and
-// 2 % of its time.
-__device__ __forceinline__ void clear_counts(uint* __restrict__ p, int n) {
-  if (p == nullptr) return;
-  for (int k = (int)(blockIdx.x * blockDim.x + threadIdx.x); k < n; k += (int)(gridDim.x * blockDim.x)) p[k] = 0u;
+__device__ __forceinline__ ForceI no_force() {
+  ForceI I;
+  I.px = I.py = I.pz = I.vx = I.vy = I.vz = 0.0f;
+  I.di = 1.0f;
+  I.pi = 0.0f;
+  I.fx = I.fy = I.fz = 0.0f;
+  return I;
 }
 
-__device__ __forceinline__ void force_wave_any(const FParams_t& P, const Span S, int N, const uint* bits, int cap) {
+__device__ __forceinline__ void force_wave_any(const FParams_t& P, const Span S, int N, const uint* bits, int cap,
+                                               const FxNext& X, float dt, float ss) {
+  const int i = S.p0 + S.blk * (int)blockDim.x + (int)threadIdx.x;
+  const int gc = i < S.p1 ? pbuf<const int>(FPnts, FGCELL)[i] : FX_GRID_UNDEF;
+  ForceI I = no_force();
   if (P.gridSrch == 3)
-    force_wave<3>(P, S, N, bits, cap, force_lds);
+    force_wave<3>(P, i, gc, N, bits, cap, force_lds, I);
   else
-    force_wave<2>(P, S, N, bits, cap, force_lds);
+    force_wave<2>(P, i, gc, N, bits, cap, force_lds, I);
+  force_end(P, S, i, i < S.p1, gc, I, X, dt, ss, force_lds);
 }
 
 // Bounds of 1024 threads, twice what is launched, keep the compiler's schedule
 // at four waves a SIMD: 280 instead of 260 us on the beach with 512.
-extern "C" __global__ __launch_bounds__(1024) void computeForceWave(int pnum, const uint* bits, int cap,
-                                                                           uint* clear, int nclear) {
-  force_wave_any(*cparams(&FParams), Span{0, pnum, 0, xcd_block()}, pnum, bits, cap);
-  clear_counts(clear, nclear);
+extern "C" __global__ __launch_bounds__(1024) void computeForceWave(int pnum, const uint* bits, int cap, FxNext X) {
+  force_wave_any(*cparams(&FParams), Span{0, pnum, 0, xcd_block()}, pnum, bits, cap, X, X.dt, X.ss);
 }
 
 extern "C" __global__ __launch_bounds__(1024) void computeForceWaveBatch(BatchArgs B, int ntotal, const uint* bits,
-                                                                                int cap, uint* clear, int nclear) {
+                                                                                int cap, FxNext X) {
   const FParams_t* P;
   const Span S = batch_span(B, xcd_block(), P);
-  force_wave_any(*P, S, ntotal, bits, cap);
-  clear_counts(clear, nclear);
+  force_wave_any(*P, S, ntotal, bits, cap, X, P->dt, P->sim_scale);
 }
 
 // Four lanes to a particle, for launches of few waves: those wait for the
@@ -2209,21 +2309,19 @@ __device__ __forceinline__ void add_lanes(ForceI& I, const PairTerm& q, int nv) 
 }
 
 template <int SR>
-__device__ __forceinline__ void force_lists(const FParams_t& P, const Span S, int N, const uint* __restrict__ bits,
-                                            int cap, uint* lds) {
+__device__ __forceinline__ void force_lists(const FParams_t& P, int i, int gc, bool in, int N,
+                                            const uint* __restrict__ bits, int cap, uint* lds, ForceI& I) {
   constexpr int G = 4, R = SR * SR;
   const int lane = (int)(threadIdx.x & 63u), sub = lane & (G - 1);
-  const int i = S.p0 + (S.blk * (int)blockDim.x + (int)threadIdx.x) / G;
   // the particle's list; strides of 4 mod 32 words keep the lists of a wave in different banks
   uint* list = lds + ((threadIdx.x >> 6) * (64 / G) + lane / G) * (FL_CAP + G);
   const uint* __restrict__ off = pbuf<const uint>(FAccel, AGRIDOFF);
   const float4* __restrict__ fr = pbuf<const float4>(FAccel, AFREC);
-  const int gc = i < S.p1 ? pbuf<const int>(FPnts, FGCELL)[i] : FX_GRID_UNDEF;
   // The lane's first three words, beside the cell and before it is known how
   // many the particle has (the buffer holds cap words of every particle):
   // 19.2 -> 18.8 us at 65,537 particles.
   uint w0 = 0u, w1 = 0u, w2 = 0u;
-  if (i < S.p1) {
+  if (in) {
     const size_t NN = (size_t)N;
     if (sub < cap) w0 = __builtin_nontemporal_load(&bits[(size_t)sub * NN + i]);
     if (sub + G < cap) w1 = __builtin_nontemporal_load(&bits[(size_t)(sub + G) * NN + i]);
@@ -2232,11 +2330,6 @@ __device__ __forceinline__ void force_lists(const FParams_t& P, const Span S, in
   const bool act = gc != FX_GRID_UNDEF;
   if (__ballot(act) == 0ull) return;
   const int shift = (P.gridRes.z + 1) * P.gridRes.x + 1;
-  ForceI I;
-  I.px = I.py = I.pz = I.vx = I.vy = I.vz = 0.0f;
-  I.di = 1.0f;
-  I.pi = 0.0f;
-  I.fx = I.fy = I.fz = 0.0f;
   // words [E_[r - 1], E_[r]) of the bitmask are row r's; bit 0 of word f is candidate B_[r] + 32 f
   int E_[R], B_[R];
 #pragma unroll
@@ -2335,29 +2428,31 @@ __device__ __forceinline__ void force_lists(const FParams_t& P, const Span S, in
     qn += tot;
   }
   drain(true);
-  if (act && sub == 0) st3(pbuf<fx_float3>(FPnts, FFORCE), (size_t)i, I.fx, I.fy, I.fz);
 }
 
-__device__ __forceinline__ void force_lists_any(const FParams_t& P, const Span S, int N, const uint* bits, int cap) {
+__device__ __forceinline__ void force_lists_any(const FParams_t& P, const Span S, int N, const uint* bits, int cap,
+                                                const FxNext& X, float dt, float ss) {
+  const int i = S.p0 + (S.blk * (int)blockDim.x + (int)threadIdx.x) / 4;
+  const int gc = i < S.p1 ? pbuf<const int>(FPnts, FGCELL)[i] : FX_GRID_UNDEF;
+  ForceI I = no_force();
   if (P.gridSrch == 3)
-    force_lists<3>(P, S, N, bits, cap, force_lds);
+    force_lists<3>(P, i, gc, i < S.p1, N, bits, cap, force_lds, I);
   else
-    force_lists<2>(P, S, N, bits, cap, force_lds);
+    force_lists<2>(P, i, gc, i < S.p1, N, bits, cap, force_lds, I);
+  force_end(P, S, i, i < S.p1 && (threadIdx.x & 3u) == 0u, gc, I, X, dt, ss, force_lds);
 }
 
 extern "C" __global__ __launch_bounds__(FX_FORCE4_THREADS) void computeForceWave4(int pnum, const uint* bits, int cap,
-                                                                                uint* clear, int nclear) {
-  force_lists_any(*cparams(&FParams), Span{0, pnum, 0, xcd_block()}, pnum, bits, cap);
-  clear_counts(clear, nclear);
+                                                                                 FxNext X) {
+  force_lists_any(*cparams(&FParams), Span{0, pnum, 0, xcd_block()}, pnum, bits, cap, X, X.dt, X.ss);
 }
 
 extern "C" __global__ __launch_bounds__(FX_FORCE4_THREADS) void computeForceWaveBatch4(BatchArgs B, int ntotal,
-                                                                                     const uint* bits, int cap,
-                                                                                     uint* clear, int nclear) {
+                                                                                      const uint* bits, int cap,
+                                                                                      FxNext X) {
   const FParams_t* P;
   const Span S = batch_span(B, xcd_block(), P);
-  force_lists_any(*P, S, ntotal, bits, cap);
-  clear_counts(clear, nclear);
+  force_lists_any(*P, S, ntotal, bits, cap, X, P->dt, P->sim_scale);
 }
 
 // ------------------------------------------------------ neighbour statistics
@@ -2580,21 +2675,14 @@ extern "C" __global__ void emitParticles(float frame, int emit, int numPnts) {
 // (Y-min with slope and friction, Y-max with friction, X-min moving wall whose
 // stiffness term is scaled by 'wall', X-max, Z-min, Z-max), gravity, the
 // acceleration limit, the velocity limit applied to the old velocity, and the
-// leapfrog update; returns the new position.  GRID_UNDEF particles are parked
-// at (-1000)^3 with zero velocity.
-__device__ __forceinline__ fx_float3 advance_one(const FParams_t& P, int i, float time, float dt, float ss) {
+// leapfrog update; returns the new position.
+template <bool Nt>
+__device__ __forceinline__ fx_float3 advance_from(const FParams_t& P, int i, const fx_float3 pos, fx_float3 vel,
+                                                  const fx_float3 ve, const fx_float3 f, float time, float dt,
+                                                  float ss) {
   fx_float3* __restrict__ posb = pbuf<fx_float3>(FPnts, FPOS);
   fx_float3* __restrict__ velb = pbuf<fx_float3>(FPnts, FVEL);
-  if (pbuf<const int>(FPnts, FGCELL)[i] == FX_GRID_UNDEF) {
-    posb[i] = fx_float3{-1000.0f, -1000.0f, -1000.0f};
-    velb[i] = fx_float3{0.0f, 0.0f, 0.0f};
-    return fx_float3{-1000.0f, -1000.0f, -1000.0f};
-  }
   fx_float3* __restrict__ vevb = pbuf<fx_float3>(FPnts, FVEVAL);
-  const fx_float3 pos = posb[i];
-  fx_float3 vel = velb[i];
-  const fx_float3 ve = vevb[i];
-  const fx_float3 f = pbuf<const fx_float3>(FPnts, FFORCE)[i];
   const float m = P.pmass;
   float ax = f.x * m, ay = f.y * m, az = f.z * m;
   const float rad = P.pradius, stiff = P.bound_stiff, damp = P.bound_damp;
@@ -2675,12 +2763,28 @@ __device__ __forceinline__ fx_float3 advance_one(const FParams_t& P, int i, floa
   }
   // leapfrog
   const float vnx = ax * dt + vel.x, vny = ay * dt + vel.y, vnz = az * dt + vel.z;
-  vevb[i] = fx_float3{(vel.x + vnx) * 0.5f, (vel.y + vny) * 0.5f, (vel.z + vnz) * 0.5f};
-  velb[i] = fx_float3{vnx, vny, vnz};
+  put3<Nt>(vevb, (size_t)i, (vel.x + vnx) * 0.5f, (vel.y + vny) * 0.5f, (vel.z + vnz) * 0.5f);
+  put3<Nt>(velb, (size_t)i, vnx, vny, vnz);
   const float dts = dt / ss;
   const float x = pos.x + vnx * dts, y = pos.y + vny * dts, z = pos.z + vnz * dts;
-  posb[i] = fx_float3{x, y, z};
+  put3<Nt>(posb, (size_t)i, x, y, z);
   return fx_float3{x, y, z};
+}
+
+// GRID_UNDEF particles are parked at (-1000)^3 with zero velocity.
+__device__ __forceinline__ fx_float3 park(int i) {
+  pbuf<fx_float3>(FPnts, FPOS)[i] = fx_float3{-1000.0f, -1000.0f, -1000.0f};
+  pbuf<fx_float3>(FPnts, FVEL)[i] = fx_float3{0.0f, 0.0f, 0.0f};
+  return fx_float3{-1000.0f, -1000.0f, -1000.0f};
+}
+
+__device__ __forceinline__ void advance_one(const FParams_t& P, int i, float time, float dt, float ss) {
+  if (pbuf<const int>(FPnts, FGCELL)[i] == FX_GRID_UNDEF) {
+    park(i);
+    return;
+  }
+  advance_from<false>(P, i, pbuf<const fx_float3>(FPnts, FPOS)[i], pbuf<const fx_float3>(FPnts, FVEL)[i],
+               pbuf<const fx_float3>(FPnts, FVEVAL)[i], pbuf<const fx_float3>(FPnts, FFORCE)[i], time, dt, ss);
 }
 
 extern "C" __global__ void advanceParticles(float time, float dt, float ss, int numPnts) {
@@ -2726,92 +2830,6 @@ __device__ __forceinline__ void advance_entry(const BatchArgs& B, int b, const f
     const int i = S.p0 + (S.blk * ppt + k) * (int)blockDim.x + (int)threadIdx.x;
     if (i < S.p1) advance_one(*P, i, clock != nullptr ? clock[0] : time, P->dt, P->sim_scale);
   }
-}
-
-// The advance of a step and the insert of the next in one pass, for steps that
-// run straight through: the position goes from one to the other in
-// registers, and the launch that is saved costs a small scene some 4 us (each
-// waits for the one before it and for its writes).  The counts were cleared
-// by the force stage.  4M particles on the beach: 75 us for 54 + 52 + 11 of
-// advance, insert and clearing.  Runs with these and the exchange merged:
-// 54.2 instead of 58.7 us a step at 16,384 particles, 156 instead of 165 at
-// 262,144, 1099 instead of 1133 at the beach.
-extern "C" __global__ void advanceInsert(const float* clock, float time, float dt, float ss, int numPnts) {
-  __shared__ uint tl[2][17];
-  const FParams_t& P = *cparams(&FParams);
-  const Span S{0, numPnts, 0, (int)blockIdx.x};
-  const int i = S.blk * (int)blockDim.x + (int)threadIdx.x;
-  fx_float3 x = fx_float3{0.0f, 0.0f, 0.0f};
-  if (i < numPnts) x = advance_one(P, i, clock != nullptr ? clock[0] : time, dt, ss);
-  insert_at(P, S, x, true, tl);
-}
-
-extern "C" __global__ void advanceInsertBatch(BatchArgs B, const float* clock, float time) {
-  __shared__ uint tl[2][17];
-  const FParams_t* P;
-  const Span S = batch_span(B, blockIdx.x, P);
-  const int i = S.p0 + S.blk * (int)blockDim.x + (int)threadIdx.x;
-  fx_float3 x = fx_float3{0.0f, 0.0f, 0.0f};
-  if (i < S.p1) x = advance_one(*P, i, clock != nullptr ? clock[0] : time, P->dt, P->sim_scale);
-  insert_at(*P, S, x, true, tl);
-}
-
-// The same in a recorded step of a rollout, whose particles (as they are
-// before the advance) and cell offsets also go to the tape, in the layout of
-// adjTapeRecord: pos, vel, veval, force (12 B each), rho, the sort's
-// permutation, cell (4 B each), then the offsets.  The pass reads most of it
-// already.  A rollout of 262,144 particles and its gradients take 12.1 instead
-// of 13.3 ms with this and the bitmask's place passed to the pair stages (it
-// was set by four copies a recorded step before), 12 scenes' 31.7 instead of
-// 32.8, one of 2,000 particles 0.57 instead of 0.61.
-struct TapeDst {
-  char* dst;
-  const uint* src;  // the sort's permutation
-  int n;
-  int cells;
-};
-
-__device__ __forceinline__ void tape_store(const TapeDst& T, int i, int end) {
-  const size_t N = (size_t)T.n;
-  if (i < end) {
-    const fx_float3 x = ld3(pbuf<const fx_float3>(FPnts, FPOS), (size_t)i);
-    const fx_float3 v = ld3(pbuf<const fx_float3>(FPnts, FVEL), (size_t)i);
-    const fx_float3 e = ld3(pbuf<const fx_float3>(FPnts, FVEVAL), (size_t)i);
-    const fx_float3 f = ld3(pbuf<const fx_float3>(FPnts, FFORCE), (size_t)i);
-    st3(reinterpret_cast<fx_float3*>(T.dst), (size_t)i, x.x, x.y, x.z);
-    st3(reinterpret_cast<fx_float3*>(T.dst + 12 * N), (size_t)i, v.x, v.y, v.z);
-    st3(reinterpret_cast<fx_float3*>(T.dst + 24 * N), (size_t)i, e.x, e.y, e.z);
-    st3(reinterpret_cast<fx_float3*>(T.dst + 36 * N), (size_t)i, f.x, f.y, f.z);
-    uint* w = reinterpret_cast<uint*>(T.dst + 48 * N);
-    w[i] = __float_as_uint(pbuf<const float>(FPnts, FPRESS)[i]);
-    w[N + i] = T.src[i];
-    w[2 * N + i] = pbuf<const uint>(FPnts, FGCELL)[i];
-  }
-  const uint* __restrict__ off = pbuf<const uint>(FAccel, AGRIDOFF);
-  uint* o = reinterpret_cast<uint*>(T.dst + 60 * N);
-  for (int k = (int)(blockIdx.x * blockDim.x + threadIdx.x); k < T.cells; k += (int)(gridDim.x * blockDim.x)) o[k] = off[k];
-}
-
-extern "C" __global__ void advanceInsertTape(float time, float dt, float ss, int numPnts, TapeDst T) {
-  __shared__ uint tl[2][17];
-  const FParams_t& P = *cparams(&FParams);
-  const Span S{0, numPnts, 0, (int)blockIdx.x};
-  const int i = S.blk * (int)blockDim.x + (int)threadIdx.x;
-  tape_store(T, i, numPnts);
-  fx_float3 x = fx_float3{0.0f, 0.0f, 0.0f};
-  if (i < numPnts) x = advance_one(P, i, time, dt, ss);
-  insert_at(P, S, x, true, tl);
-}
-
-extern "C" __global__ void advanceInsertTapeBatch(BatchArgs B, float time, TapeDst T) {
-  __shared__ uint tl[2][17];
-  const FParams_t* P;
-  const Span S = batch_span(B, blockIdx.x, P);
-  const int i = S.p0 + S.blk * (int)blockDim.x + (int)threadIdx.x;
-  tape_store(T, i, S.p1);
-  fx_float3 x = fx_float3{0.0f, 0.0f, 0.0f};
-  if (i < S.p1) x = advance_one(*P, i, time, P->dt, P->sim_scale);
-  insert_at(*P, S, x, true, tl);
 }
 
 extern "C" __global__ void advanceParticlesBatch(BatchArgs B, const float* clock, float time) {
