@@ -339,7 +339,9 @@ int Particles::AdjRestoreCheckpoint(int k) {
 // tape slot.
 int Particles::AdjStep(int record_slot, bool first, bool last) {
   const bool joined = JoinedSteps(), rec = record_slot >= 0, wave = WaveStages();
-  FX_TRY(SortStep(first || !joined));
+  NextStep next;
+  next.mode = !joined || last ? 0 : rec ? 2 : 1;
+  FX_TRY(SortStep(first || !joined, next.mode != 0));
   char* tabs = static_cast<char*>(m_AdjTabs);
   const size_t n = (size_t)m_AdjN;
   NbrBits bits;  // a recorded step's bitmask is written into the tape, m_AdjWords a particle
@@ -351,8 +353,6 @@ int Particles::AdjStep(int record_slot, bool first, bool last) {
                           sizeof(cuDataX), hipMemcpyDeviceToDevice, m_Stream), "tape");
   }
   char* t = m_AdjTape + TapeStep() * (size_t)(rec ? record_slot : 0);
-  NextStep next;
-  next.mode = !joined || last ? 0 : rec ? 2 : 1;
   next.tape = {t, m_AdjSrc, m_AdjN, m_AdjCells};
   FX_TRY(ComputePressure(bits, next.mode != 0));
   FX_TRY(ComputeForce(bits, next));

@@ -651,12 +651,14 @@ int Particles::CountingSort() {
   return SortKernels();
 }
 
-int Particles::SortKernels() {
+int Particles::SortKernels(bool clear) {
+  // counts cleared for the next step's insert, by the density where it takes several lanes to a particle
+  void* cnt = clear && DensityLanes() == 1 ? m_Accel.gpu(AGRIDCNT) : nullptr;
   if (m_Batch) {
     FX_TRY(BatchLaunch(FUNC_SORT_INDEX_B, FUNC_SORT_INDEX_BP, FX_STAGE_SORT, nullptr, nullptr, nullptr));
-    FX_TRY(BatchLaunch(FUNC_SORT_FULL_B, FUNC_SORT_FULL_BP, FX_STAGE_SORT, nullptr, nullptr, nullptr));
+    FX_TRY(BatchLaunch(FUNC_SORT_FULL_B, FUNC_SORT_FULL_BP, FX_STAGE_SORT, &cnt, &m_ScanCells, nullptr));
   } else {
-    void* args[] = {&mNumPoints};
+    void* args[] = {&mNumPoints, &cnt, &m_ScanCells};
     FX_TRY(LaunchP(FUNC_SORT_INDEX, FX_STAGE_SORT, args));
     FX_TRY(LaunchP(FUNC_COUNTING_SORT, FX_STAGE_SORT, args));
   }
@@ -667,7 +669,7 @@ int Particles::SortKernels() {
 int Particles::ComputePressure(NbrBits bits, bool clear) {
   if (WaveStages()) {
     const int lanes = DensityLanes(), t = StageThreads(FX_STAGE_PRESSURE, FX_DENS_THREADS), v = lanes == 4 ? 2 : lanes - 1;
-    void* cnt = clear ? m_Accel.gpu(AGRIDCNT) : nullptr;  // counts cleared for the next step's insert
+    void* cnt = clear && lanes > 1 ? m_Accel.gpu(AGRIDCNT) : nullptr;  // else the sort has cleared them
     FX_TRY(LaunchLanes(FUNC_PRESS_W + v, FUNC_PRESS_WB + v, t, lanes, FX_DENS_LDS(t), bits, &cnt, &m_ScanCells));
   } else if (m_Batch) {
     FX_TRY(BatchLaunch(FUNC_PRESS_B, FUNC_PRESS_BP, FX_STAGE_PRESSURE, &mNumPoints, nullptr, nullptr));
@@ -767,7 +769,7 @@ int Particles::Step(bool first, bool last) {
   const bool joined = JoinedSteps();
   NextStep next;
   next.mode = joined && !last ? 1 : 0;
-  FX_TRY(SortStep(first || !joined));
+  FX_TRY(SortStep(first || !joined, next.mode != 0));
   FX_TRY(ComputePressure(NbrBits(), next.mode != 0));
   FX_TRY(ComputeForce(NbrBits(), next));
   if (next.mode == 0) FX_TRY(Advance());
@@ -775,13 +777,14 @@ int Particles::Step(bool first, bool last) {
   return FX_OK;
 }
 
-// A step's insert (unless the step before it made it) to its sort.
-int Particles::SortStep(bool insert) {
+// A step's insert (unless the step before it made it) to its sort; clear: the
+// counts become zero for the insert that the force makes.
+int Particles::SortStep(bool insert, bool clear) {
   if (insert) FX_TRY(InsertParticles());
   FX_TRY(m_Points.SwapGPU(&m_PointsTemp));
   m_Parity ^= 1;
   FX_TRY(ScanGrid(true));
-  return SortKernels();
+  return SortKernels(clear);
 }
 
 int Particles::Run(int nsteps) {

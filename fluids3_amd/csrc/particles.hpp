@@ -145,7 +145,8 @@ class Particles {
   int InsertParticles();
   int PrefixScanParticles();
   int CountingSort();
-  // clear: zero the cell counts for the insert that the force makes (WaveStages only, as next)
+  // clear: zero the cell counts for the insert that the force makes; next: what
+  // the force launch does after the forces (both WaveStages only)
   int ComputePressure(NbrBits bits = NbrBits(), bool clear = false);
   int ComputeForce(NbrBits bits = NbrBits(), NextStep next = NextStep());
   int Advance();
@@ -203,11 +204,11 @@ class Particles {
   int ScanTwoLaunch(void* in, void* out, void* sums, int n, void* in2 = nullptr, void* out2 = nullptr,
                     void* sums2 = nullptr, int n2 = 0, bool exchange = false);
   int ScanGrid(bool exchange);
-  int SortKernels();
+  int SortKernels(bool clear = false);
   int PublishTables();
   bool JoinedSteps() const;
   int Step(bool first, bool last);
-  int SortStep(bool insert);
+  int SortStep(bool insert, bool clear);
   int SetDeviceClock();
   int CapturePair(int inner);
   int ReplayGraph(int nlaunch);

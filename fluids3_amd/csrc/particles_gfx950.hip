@@ -648,14 +648,18 @@ __device__ __forceinline__ void sort_full_impl(const FParams_t& P, const Span S)
   const int i = S.p0 + S.blk * (int)blockDim.x + (int)threadIdx.x;
   const bool act = i < S.p1;  // active lanes are a prefix of the wave
   const uint* off = pbuf<const uint>(FAccel, AGRIDOFF);
-  const uint* cnt = pbuf<const uint>(FAccel, AGRIDCNT);
   const uint* grid = pbuf<const uint>(FAccel, AGRID);
   const uint* tscan = pbuf<const uint>(FAccel, ATAILSCAN);
   uint* sstart = pbuf<uint>(FAccel, ASLABSTART);
   const int c = act ? __builtin_nontemporal_load(&pbuf<const int>(FPntTmp, FGCELL)[i]) : FX_GRID_UNDEF;
   const int cell = (c == FX_GRID_UNDEF) ? S.c0 + P.gridTotal : c;
-  const uint o = act ? off[cell] : 0u;
-  const uint n = act ? cnt[cell] : 0u;
+  // an in-range cell ends where the next begins (the counts may be cleared)
+  uint o = 0u, n = 0u;
+  if (act) {
+    o = off[cell];
+    n = off[cell + (c != FX_GRID_UNDEF ? 1 : 0)];
+  }
+  n -= o;
   // Everything that moves is loaded beside the cell's bounds: the ranking
   // below waits for memory twice more by itself (sort stage 158 -> 140 us at
   // the compressed 4M dam break, 172 -> 154 at the 4M beach from step 90,
@@ -726,15 +730,15 @@ __device__ __forceinline__ void sort_full_impl(const FParams_t& P, const Span S)
   } else if (c == FX_GRID_UNDEF && tscan != nullptr) {
     // tail bucket: the number of the scene's out-of-range particles before i
     rank = (int)(tscan[i] - tscan[S.p0]);
-  } else if (n <= FX_RANK_CAP) {
+  } else if (const uint m = c != FX_GRID_UNDEF ? n : pbuf<const uint>(FAccel, AGRIDCNT)[cell]; m <= FX_RANK_CAP) {
     // member entries below this particle's own; eight in flight per step, the
     // last of them repeated (a loop over the remainder waited for each)
-    for (uint k = 0; k < n; k += 8) {
+    for (uint k = 0; k < m; k += 8) {
       uint e[8];
 #pragma unroll
-      for (uint u = 0; u < 8; u++) e[u] = grid[o + min(k + u, n - 1)];
+      for (uint u = 0; u < 8; u++) e[u] = grid[o + min(k + u, m - 1)];
 #pragma unroll
-      for (uint u = 0; u < 8; u++) rank += k + u < n && e[u] < key ? 1 : 0;
+      for (uint u = 0; u < 8; u++) rank += k + u < m && e[u] < key ? 1 : 0;
     }
   } else {
     rank = pbuf<const int>(FPntTmp, FGNDX)[i];
@@ -786,6 +790,18 @@ __device__ __forceinline__ void sort_full_gndx(const FParams_t& P, const Span S,
   if (grid != nullptr) grid[s] = s;
 }
 
+// Clears n counts, spread over the launch, for the next step's insert, which
+// the force launch of this step makes (force_end): after the scan no stage of
+// a step that runs straight through reads them.  The density launch does it
+// with two or four lanes to a particle, the sort's with one: there two more
+// registers cost the density a wave a SIMD and 4 % of its time (beach 102.3 ->
+// 101.0 ms for 100 steps), while small scenes lose by it in the sort (65,537
+// particles 79.2 -> 80.5 us a step).
+__device__ __forceinline__ void clear_counts(uint* __restrict__ p, int n) {
+  if (p == nullptr) return;
+  for (int k = (int)(blockIdx.x * blockDim.x + threadIdx.x); k < n; k += (int)(gridDim.x * blockDim.x)) p[k] = 0u;
+}
+
 extern "C" __global__ void countingSortIndex(int pnum) {
   const int ppt = ppt_of(2);
   const Span S{0, pnum, 0, (int)blockIdx.x};
@@ -799,14 +815,15 @@ extern "C" __global__ void countingSortIndex(int pnum) {
 // The sort of a host that runs the index sort first (libfluidsx).  Kept apart
 // from countingSortFull: compiling the insert-slot variant into the same
 // kernel slows this one by half (183 vs 114 us per launch at 4M particles).
-extern "C" __global__ void countingSortFullRanked(int pnum) {
+extern "C" __global__ void countingSortFullRanked(int pnum, uint* clear, int nclear) {
   const int ppt = ppt_of(2);
   const Span S{0, pnum, 0, xcd_block()};
   if (ppt == 1) {
     sort_full_impl(*cparams(&FParams), S);
-    return;
+  } else {
+    for (int k = 0; k < ppt; k++) sort_full_impl(*cparams(&FParams), sub_span(S, ppt, k));
   }
-  for (int k = 0; k < ppt; k++) sort_full_impl(*cparams(&FParams), sub_span(S, ppt, k));
+  clear_counts(clear, nclear);
 }
 
 // The reference's kernel name (particles.cu:64-95): the insert's slots for a
@@ -841,7 +858,10 @@ __device__ __forceinline__ void sort_full_entry(const BatchArgs& B, int b) {
 }
 
 extern "C" __global__ void countingSortIndexBatch(BatchArgs B) { sort_index_entry(B, blockIdx.x); }
-extern "C" __global__ void countingSortFullBatch(BatchArgs B) { sort_full_entry(B, xcd_block()); }
+extern "C" __global__ void countingSortFullBatch(BatchArgs B, uint* clear, int nclear) {
+  sort_full_entry(B, xcd_block());
+  clear_counts(clear, nclear);
+}
 
 extern "C" __global__ void countingSortIndexBatchP(BatchArgs B) {
   batch_items(B, [&](int b) { sort_index_entry(B, b); });
@@ -1424,7 +1444,7 @@ __device__ __forceinline__ void density_wave(const FParams_t& P, const Span S, i
     int ts = 0, te = L0;
     if (act && sstart != nullptr && L0 > FX_RANK_WAVE) {
       const int c0 = gc + P.gridAdj[r * SR] - shift, c2 = c0 + SR - 1;
-      const int n0 = (int)off[c0 + 1] - jbr, n2 = jbr + L0 - (int)off[c2];  // the counts, which this launch clears
+      const int n0 = (int)off[c0 + 1] - jbr, n2 = jbr + L0 - (int)off[c2];  // the counts, which may be cleared
       if (n0 > FX_RANK_WAVE && n0 <= FX_RANK_CAP) ts = slab_start(sstart, c0, n0, slo);
       if (n2 > FX_RANK_WAVE && n2 <= FX_RANK_CAP) te = max(ts, te - n2 + slab_start(sstart, c2, n2, shi));
     }
@@ -1553,27 +1573,19 @@ __device__ __forceinline__ void density_wave_any(const FParams_t& P, const Span 
     density_wave<G, 2>(P, S, N, bits, cap, dens_lds);
 }
 
-// Clears n counts, spread over the launch, for the next step's insert, which
-// the force launch of this step makes (force_end).  No stage after the sort
-// reads them.  After the walk: before a pair walk it costs registers.
-__device__ __forceinline__ void clear_counts(uint* __restrict__ p, int n) {
-  if (p == nullptr) return;
-  for (int k = (int)(blockIdx.x * blockDim.x + threadIdx.x); k < n; k += (int)(gridDim.x * blockDim.x)) p[k] = 0u;
-}
-
 // bits: cap words of bitmask a particle (the system's buffer, or a rollout's tape)
 #define FX_DENSITY_WAVE(G)                                                                                    \
   extern "C" __global__ __launch_bounds__(FX_DENS_THREADS) void computePressureWave##G(                       \
       int pnum, uint* bits, int cap, uint* clear, int nclear) {                                               \
     density_wave_any<G>(*cparams(&FParams), Span{0, pnum, 0, xcd_block()}, pnum, bits, cap);                  \
-    clear_counts(clear, nclear);                                                                              \
+    if (G > 1) clear_counts(clear, nclear);                                                                   \
   }                                                                                                           \
   extern "C" __global__ __launch_bounds__(FX_DENS_THREADS) void computePressureWaveBatch##G(                  \
       BatchArgs B, int ntotal, uint* bits, int cap, uint* clear, int nclear) {                                \
     const FParams_t* P;                                                                                       \
     const Span S = batch_span(B, xcd_block(), P);                                                             \
     density_wave_any<G>(*P, S, ntotal, bits, cap);                                                            \
-    clear_counts(clear, nclear);                                                                              \
+    if (G > 1) clear_counts(clear, nclear);                                                                   \
   }
 FX_DENSITY_WAVE(1)
 FX_DENSITY_WAVE(2)
@@ -2046,8 +2058,8 @@ extern "C" __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu
 // position and evaluation velocity are at hand as its pair record, its force
 // need not go through memory, and the passes' traffic lies beside other
 // waves' pair arithmetic.  Neighbours are read from the records and the
-// offsets only, which neither changes; the counts were cleared by the density
-// launch.  What this pass writes is not read before the next launch and is
+// offsets only, which neither changes; the counts were cleared before
+// (clear_counts).  What this pass writes is not read before the next launch and is
 // stored non-temporally, so that it does not displace the records (4M
 // particles on the beach, a step from step 20 751 -> 721 us, from step 80
 // 1143 -> 1109).  Against passes of their own for the advance with the insert
