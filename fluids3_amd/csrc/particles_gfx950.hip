@@ -2816,8 +2816,8 @@ extern "C" __global__ void advanceParticles(float time, float dt, float ss, int 
 
 // Same integrator with the simulation time read from device memory, for
 // captured step graphs whose launches cannot carry a per-step time argument.
-// fxPublishTables moves that clock on by dt each step (the host's
-// AdvanceTime, particles.cpp:396-400).
+// The set exchange (exchange_tables) moves that clock on by dt each step (the
+// host's AdvanceTime, particles.cpp:396-400).
 extern "C" __global__ void advanceParticlesClock(const float* clock, float dt, float ss, int numPnts) {
   const int ppt = ppt_of(5);
   if (ppt == 1) {
