@@ -110,9 +110,10 @@ def test_stencils_in_a_batch(ps, gd):
             assert bits_equal(got[k][p0:p0 + n], want[k]), (s, k)
 
 
-# Steps that run straight through share a pass between one step's advance and
-# the next one's insert: the same state, tables and ranks as single steps, in
-# one scene (with particles that leave the grid), in a batch and replayed.
+# In steps that run straight through the force launch also advances and makes
+# the next step's insert (one or four lanes to a particle): the same state,
+# tables and ranks as single steps, in one scene (with particles that leave the
+# grid), in a batch and replayed.
 @pytest.mark.parametrize("n", [1, 63, 65, 257, 5003, 60001])
 @pytest.mark.parametrize("batch", [False, True])
 def test_joined_steps(ps, n, batch):
@@ -159,3 +160,32 @@ def test_scan_launches(ps, n, half):
     sc = scenes.dambreak_16k(n)
     sc.bound_min.x, sc.bound_max.x = -half, half
     one_step_bitexact(ps, sc, vel=swirl(n, 9))
+
+
+@pytest.mark.parametrize("threads", [64, 512, 1024])
+@pytest.mark.parametrize("n,gd", [(5003, 1.5), (5003, 1.0), (90001, 1.5), (90001, 1.0)])
+def test_joined_steps_block_sizes(ps, n, gd, threads):
+    sc = scenes.scaled_dam_break(n)
+    sc.grid_density = gd
+    states = []
+    for steps in ([1, 1, 1], [3]):
+        ps.Restart(sc)
+        pos = ps.state()["pos"]
+        pos[:: 7] += 500.0
+        ps.Commit(abi.FPOS, pos)
+        ps.Commit(abi.FVEL, swirl(n, 8))
+        ps.SetStageBlockSize(abi.STAGE_PRESSURE, threads)
+        ps.SetStageBlockSize(abi.STAGE_FORCE, threads)
+        for k in steps:
+            ps.Run(k)
+        states.append(ps.state())
+        ps.SetStageBlockSize(abi.STAGE_PRESSURE, 256)
+        ps.SetStageBlockSize(abi.STAGE_FORCE, 256)
+    a, b = states
+    for k in ("gcell", "gndx", "id", "cnt", "off"):
+        assert_int_equal(k, b[k], a[k])
+    m = valid_mask(a)
+    for k in ("press", "force"):
+        assert bits_equal(b[k][m], a[k][m]), k
+    for k in ("pos", "vel", "veval"):
+        assert bits_equal(b[k], a[k]), k
