@@ -1587,11 +1587,13 @@ __device__ __forceinline__ void density_wave_any(const FParams_t& P, const Span 
     density_wave_any<G>(*P, S, ntotal, bits, cap);                                                            \
     if (G > 1) clear_counts(clear, nclear);                                                                   \
   }
-// One lane in a batch takes 73 registers by itself, one too many for seven
-// waves a SIMD (held at 72 it spills two): 64 scenes 93.2 -> 92.4 ms for 50 steps.
+// In a batch the kernels take 73, 81 and 97 registers by themselves, each just
+// over a step of the occupancy; they are held at seven, six and five waves a
+// SIMD (the first spills two): 64 scenes of 5.3M particles 93.2 -> 92.4 ms for
+// 50 steps, 24 of 208,000 101 -> 99 us a step, 16 of 73,000 64.6 -> 63.4.
 FX_DENSITY_WAVE(1, __attribute__((amdgpu_waves_per_eu(7))))
-FX_DENSITY_WAVE(2, )
-FX_DENSITY_WAVE(4, )
+FX_DENSITY_WAVE(2, __attribute__((amdgpu_waves_per_eu(6))))
+FX_DENSITY_WAVE(4, __attribute__((amdgpu_waves_per_eu(5))))
 
 // ------------------------------------------------------------------- force
 
