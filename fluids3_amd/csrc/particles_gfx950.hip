@@ -2060,7 +2060,7 @@ extern "C" __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu
 // makes the next step's insert (and, in a recorded step of a rollout, writes
 // the particles as they are before the advance to the tape): a particle's
 // position and evaluation velocity are at hand as its pair record, its force
-// need not go through memory, and the passes' traffic lies beside other
+// need not be read back, and the passes' traffic lies beside other
 // waves' pair arithmetic.  Neighbours are read from the records and the
 // offsets only, which neither changes; the counts were cleared before
 // (clear_counts).  What this pass writes is not read before the next launch and is
@@ -2121,7 +2121,13 @@ __device__ __forceinline__ fx_float3 park(int i);
 __device__ __forceinline__ void force_end(const FParams_t& P, const Span S, int i, bool own, int gc, const ForceI& I,
                                           const FxNext& X, float dt, float ss, uint* lds) {
   const bool act = own && gc != FX_GRID_UNDEF;
-  if (X.mode != 1 && act) st3(pbuf<fx_float3>(FPnts, FFORCE), (size_t)i, I.fx, I.fy, I.fz);
+  // (stored in every step: a slot whose particle leaves the grid keeps its last force)
+  if (act) {
+    if (X.mode == 1)
+      put3<true>(pbuf<fx_float3>(FPnts, FFORCE), (size_t)i, I.fx, I.fy, I.fz);
+    else
+      st3(pbuf<fx_float3>(FPnts, FFORCE), (size_t)i, I.fx, I.fy, I.fz);
+  }
   if (X.mode == 0) return;
   if (X.mode == 2) tape_store(X.tape, i, own);
   fx_float3 x = fx_float3{0.0f, 0.0f, 0.0f};
