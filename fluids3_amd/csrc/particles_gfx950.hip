@@ -812,17 +812,25 @@ extern "C" __global__ void countingSortIndex(int pnum) {
   for (int k = 0; k < ppt; k++) sort_index_impl(*cparams(&FParams), sub_span(S, ppt, k));
 }
 
-// The sort of a host that runs the index sort first (libfluidsx).  Kept apart
+// The sort of a host that runs the index sort first.  Kept apart
 // from countingSortFull: compiling the insert-slot variant into the same
 // kernel slows this one by half (183 vs 114 us per launch at 4M particles).
-extern "C" __global__ void countingSortFullRanked(int pnum, uint* clear, int nclear) {
+__device__ __forceinline__ void sort_ranked(int pnum) {
   const int ppt = ppt_of(2);
   const Span S{0, pnum, 0, xcd_block()};
   if (ppt == 1) {
     sort_full_impl(*cparams(&FParams), S);
-  } else {
-    for (int k = 0; k < ppt; k++) sort_full_impl(*cparams(&FParams), sub_span(S, ppt, k));
+    return;
   }
+  for (int k = 0; k < ppt; k++) sort_full_impl(*cparams(&FParams), sub_span(S, ppt, k));
+}
+
+extern "C" __global__ void countingSortFullRanked(int pnum) { sort_ranked(pnum); }
+
+// The same in a step whose force launch makes the next insert (libfluidsx):
+// a name of its own, because hosts launch the one above with pnum alone.
+extern "C" __global__ void countingSortFullRankedClear(int pnum, uint* clear, int nclear) {
+  sort_ranked(pnum);
   clear_counts(clear, nclear);
 }
 
