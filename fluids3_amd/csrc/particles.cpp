@@ -19,7 +19,7 @@ static const char* kKernelNames[FUNC_MAX] = {
     "advanceParticles",  "prefixSum",        "prefixFixup",     "countingSortIndex",
     "fxFillUint",        "advanceParticlesClock", "fxPublishTables", "fxCountPairs",
     "insertParticlesBatch", "countingSortIndexBatch", "countingSortFullBatch", "computePressureBatch",
-    "computeForceBatch", "advanceParticlesBatch", "fxCountPairsBatch", "sampleParticles",
+    "computeForceBatch", "advanceParticlesBatch", "fxCountPairsBatch", "fxSampleBrick",
     "emitParticles",     "fxMaxWords",       "fxMaxWordsBatch",  "fxMark",
     "insertParticlesBatchP", "countingSortIndexBatchP", "countingSortFullBatchP", "computePressureBatchP",
     "computeForceBatchP", "advanceParticlesBatchP", "fxScanSums", "fxScanApply",
@@ -1029,7 +1029,7 @@ int Particles::SampleParticles(float* brick, const int* res, const float* bmin, 
   hipError_t e = hipModuleLaunchKernel(m_Func[FUNC_SAMPLE], (unsigned)((res[0] + bx - 1) / bx),
                                        (unsigned)((res[1] + by - 1) / by), (unsigned)((res[2] + bz - 1) / bz), 256, 1,
                                        1, 0, m_Stream, args, nullptr);
-  const int st = e != hipSuccess ? fx::hip_fail(e, "sample_particles", "sampleParticles")
+  const int st = e != hipSuccess ? fx::hip_fail(e, "sample_particles", "fxSampleBrick")
                                  : m_Staging.down(brick, d, bytes, "sample_particles");
   if (m_BrickBytes > kBrickKept) {
     (void)hipFree(m_Brick);

@@ -2629,15 +2629,9 @@ __device__ __forceinline__ float sample_voxel(const FParams_t& P, float px, floa
   return v;
 }
 
-extern "C" __global__ __launch_bounds__(256) void sampleParticles(float* brick, fx_int3 res, fx_float3 bmin,
-                                                                  fx_float3 bmax, int numPnts, float scalar,
-                                                                  float khi, float klo) {
+__device__ __forceinline__ void sample_brick(int x, int y, int z, float* brick, const fx_int3 res, const fx_float3 bmin,
+                                             const fx_float3 bmax, int numPnts, float scalar, float khi, float klo) {
   const FParams_t& P = *cparams(&FParams);
-  const int t = (int)threadIdx.x, w = t >> 6;
-  // a block: 8 x 8 x 4 voxels, four waves
-  const int x = (int)blockIdx.x * 2 * SV_EDGE + (w & 1) * SV_EDGE + t % SV_EDGE;
-  const int y = (int)blockIdx.y * 2 * SV_EDGE + (w >> 1) * SV_EDGE + t / SV_EDGE % SV_EDGE;
-  const int z = (int)blockIdx.z * SV_EDGE + t / (SV_EDGE * SV_EDGE) % SV_EDGE;
   if (x >= res.x || y >= res.y || z >= res.z) return;
   const size_t out = ((size_t)z * res.y + y) * res.x + x;
   const float px = bmin.x + ((float)x / (float)res.x) * (bmax.x - bmin.x);
@@ -2657,6 +2651,29 @@ extern "C" __global__ __launch_bounds__(256) void sampleParticles(float* brick, 
                   : P.gridSrch == 2 ? sample_voxel<2>(P, px, py, pz, gs, numPnts, khi, klo)
                                     : sample_voxel<0>(P, px, py, pz, gs, numPnts, khi, klo);
   brick[out] = v * P.gausskern * scalar;
+}
+
+// libfluidsx's launch: blocks of 256 threads over 8 x 8 x 4 voxels, four waves
+extern "C" __global__ __launch_bounds__(256) void fxSampleBrick(float* brick, fx_int3 res, fx_float3 bmin,
+                                                                fx_float3 bmax, int numPnts, float scalar, float khi,
+                                                                float klo) {
+  const int t = (int)threadIdx.x, w = t >> 6;
+  const int x = (int)blockIdx.x * 2 * SV_EDGE + (w & 1) * SV_EDGE + t % SV_EDGE;
+  const int y = (int)blockIdx.y * 2 * SV_EDGE + (w >> 1) * SV_EDGE + t / SV_EDGE % SV_EDGE;
+  const int z = (int)blockIdx.z * SV_EDGE + t / (SV_EDGE * SV_EDGE) % SV_EDGE;
+  sample_brick(x, y, z, brick, res, bmin, bmax, numPnts, scalar, khi, klo);
+}
+
+// The reference's kernel name and arguments (fluids4.0/fluid_kernels.cu:259),
+// one voxel a thread of blocks of any shape; the same values.
+extern "C" __global__ void sampleParticles(float* brick, fx_int3 res, fx_float3 bmin, fx_float3 bmax, int numPnts,
+                                           float scalar) {
+  const FParams_t& P = *cparams(&FParams);
+  const float h2 = 2.0f * P.r2 / 8.0f;
+  const double k = -(double)P.d2 / (double)h2 * 1.4426950408889634;
+  const float khi = (float)k, klo = (float)(k - (double)khi);
+  sample_brick((int)(blockIdx.x * blockDim.x + threadIdx.x), (int)(blockIdx.y * blockDim.y + threadIdx.y),
+               (int)(blockIdx.z * blockDim.z + threadIdx.z), brick, res, bmin, bmax, numPnts, scalar, khi, klo);
 }
 
 // ------------------------------------------------------------------- emit

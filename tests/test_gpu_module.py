@@ -10,7 +10,7 @@ import pytest
 from fluids3_amd import abi, derive_params, fill_points, scenes
 from fluids3_amd.particles import CODE_OBJECT
 from oracle import oracle
-from parity import assert_int_equal, bits_equal
+from parity import assert_int_equal, bits_equal, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -130,3 +130,23 @@ def test_ranked_host(stepped):
     for k, b in (("pos", abi.FPOS), ("vel", abi.FVEL), ("veval", abi.FVEVAL), ("force", abi.FFORCE)):
         assert bits_equal(h.get(h.sets[0][b], (h.n, 3), np.float32), ref[k]), k
     assert bits_equal(h.get(h.sets[0][abi.FPRESS], h.n, np.float32), ref["press"])
+
+
+# the brick kernel under the reference's name: blocks of any shape, some of their voxels beyond the brick
+@pytest.mark.parametrize("block", [(8, 8, 4), (64, 1, 1), (3, 5, 7)])
+def test_brick_by_the_reference_name(stepped, block):
+    h, P, _ = stepped
+    res, lo, hi, scalar = (19, 13, 11), (-25.0, 0.0, -25.0), (25.0, 30.0, 25.0), 0.5
+    brick = h.alloc(4 * res[0] * res[1] * res[2])
+    grid = tuple((r + b - 1) // b for r, b in zip(res, block))
+    h.launch("sampleParticles", grid, block, C.c_uint64(brick), (C.c_int * 3)(*res), (C.c_float * 3)(*lo),
+             (C.c_float * 3)(*hi), C.c_int(h.n), C.c_float(scalar))
+    h.ok(h.hip.hipDeviceSynchronize())
+    got = h.get(brick, (res[2], res[1], res[0]), np.float32)
+    st = {"pos": h.get(h.sets[0][abi.FPOS], (h.n, 3), np.float32),
+          "cnt": h.get(h.accel[abi.AGRIDCNT], h.cells, np.uint32),
+          "off": h.get(h.accel[abi.AGRIDOFF], h.cells, np.uint32)}
+    want = oracle.sample(P, st, res, lo, hi, scalar)
+    assert np.count_nonzero(want) > 100
+    assert np.array_equal(got == 0, want == 0)
+    assert rel_err(got, want) <= 1e-5  # powers in 32 bits on both sides

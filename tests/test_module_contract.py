@@ -24,6 +24,7 @@ PUBLISHED = {
     "computeForce": [4],
     "advanceParticles": [4, 4, 4, 4],
     "emitParticles": [4, 4, 4],
+    "sampleParticles": [8, 12, 12, 12, 4, 4],
 }
 
 
