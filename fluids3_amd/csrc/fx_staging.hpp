@@ -21,7 +21,6 @@
 #include <cstring>
 #include <memory>
 #include <new>
-#include <system_error>
 #include <thread>
 
 #include "fx_common.hpp"
@@ -127,7 +126,7 @@ class Staging {
     try {
       if (done != nullptr)
         for (; workers < kWorkers; workers++) worker[workers] = std::thread(work);
-    } catch (const std::system_error&) {  // as many as could be started
+    } catch (...) {  // no more threads or no memory for one: as many as could be started
     }
     if (workers == 0) {
       FX_HIP(hipMemcpyDtoH(to, from, bytes), who);

@@ -1,0 +1,55 @@
+"""What the host library launches, copies and allocates, on the CPU: its sources linked against tests/hoststub/hip_stub.cpp,
+which logs the launches.  Each case runs in a process of its own.
+"""
+import os
+import subprocess
+import sys
+import textwrap
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+STUB = os.path.join(ROOT, "tests", "hoststub", "libfluidsx_stub.so")
+
+PRELUDE = """
+import ctypes as C
+import sys
+sys.path.insert(0, {root!r})
+import numpy as np
+import fluids3_amd.particles as particles
+particles.LIB_PATH = {stub!r}
+from fluids3_amd import Particles, abi, scenes
+stub = particles.lib()
+stub.stub_log.restype = C.c_char_p
+for f in ("stub_captures", "stub_events", "stub_pinned_bytes"):
+    getattr(stub, f).restype = C.c_long
+stub.stub_fail_new.argtypes = [C.c_long]
+
+def launches(call):
+    stub.stub_clear_log()
+    call()
+    return stub.stub_log().decode().split()
+"""
+
+
+def on_stub(code):
+    if not os.path.exists(STUB):
+        raise RuntimeError("tests/hoststub is not built (run __graft_entry__.build())")
+    src = PRELUDE.format(root=ROOT, stub=STUB) + textwrap.dedent(code)
+    r = subprocess.run([sys.executable, "-c", src], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, f"exit {r.returncode}\n{r.stdout}{r.stderr}"
+
+
+def test_long_download_without_memory_for_every_thread():
+    """A worker thread that cannot be had for want of memory is left out: no thread, the first one only, two."""
+    on_stub("""
+        ps = Particles()
+        n = 1000000  # 12 MB
+        ps.Restart(scenes.scaled_dam_break(n))
+        pos = np.arange(3 * n, dtype=np.float32).reshape(n, 3)
+        ps.Commit(abi.FPOS, pos)
+        for nth in (1, 2, 3):
+            stub.stub_fail_new(nth)
+            got = ps.Retrieve(abi.FPOS)
+            stub.stub_fail_new(0)
+            assert np.array_equal(got, pos), nth
+        ps.close()
+    """)
