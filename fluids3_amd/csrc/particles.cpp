@@ -789,7 +789,7 @@ int Particles::SortStep(bool insert, bool clear) {
 }
 
 int Particles::Run(int nsteps) {
-  if (mNumPoints == 0) return fx::fail(FX_ESTATE, "Run: call Restart first");
+  if (mNumPoints == 0 && nsteps > 0) return fx::fail(FX_ESTATE, "Run: call Restart first");
   for (int s = 0; s < nsteps; s++) {
     FX_TRY(Step(s == 0, s + 1 == nsteps));
     AdvanceTime();

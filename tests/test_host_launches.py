@@ -53,3 +53,22 @@ def test_long_download_without_memory_for_every_thread():
             assert np.array_equal(got, pos), nth
         ps.close()
     """)
+
+
+def test_no_steps_need_no_scene():
+    """A run of no steps does nothing, also where there is no scene yet; one step is refused then."""
+    on_stub("""
+        ps = Particles()
+        ps.Run(0)
+        assert ps.TimeSteps(0, False) == 0.0
+        for call in (lambda: ps.Run(1), lambda: ps.TimeSteps(1, False)):
+            try:
+                call()
+            except Exception as e:
+                assert "Restart" in str(e)
+            else:
+                raise AssertionError("a step without a scene")
+        ps.Restart(scenes.scaled_dam_break(64))
+        assert launches(lambda: ps.Run(0)) == []
+        ps.close()
+    """)
