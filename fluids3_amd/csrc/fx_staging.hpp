@@ -68,6 +68,7 @@ class Staging {
   int down(void* dst, const void* src, size_t bytes, const char* who) {
     char* from = static_cast<char*>(const_cast<void*>(src));
     char* to = static_cast<char*>(dst);
+    if (bytes == 0) return drain(who);
     if (bytes > kDown) return down_long(to, from, bytes, who);
     const int chunks = (int)((bytes + kSlot - 1) / kSlot);
     auto size = [&](int k) { return std::min(kSlot, bytes - (size_t)k * kSlot); };
@@ -84,7 +85,7 @@ class Staging {
         FX_HIP(hipStreamSynchronize(m_stream), who);
       memcpy(to + (size_t)k * kSlot, m_down + (size_t)(k % kSlots) * kSlot, size(k));
     }
-    if (chunks > 0) m_used = 0;  // every upload before them has been made
+    m_used = 0;  // every upload before them has been made
     return FX_OK;
   }
 

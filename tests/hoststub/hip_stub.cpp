@@ -31,7 +31,7 @@ std::string g_log;
 std::vector<std::string>* g_capture = nullptr;
 std::map<std::string, void*> g_functions, g_globals;
 double g_clock = 0.0;
-long g_launches = 0, g_captures = 0, g_events = 0;
+long g_launches = 0, g_captures = 0, g_events = 0, g_waits = 0;
 size_t g_pinned = 0;
 std::map<void*, size_t> g_pin;
 thread_local long g_fail_new = 0;  // the call of operator new, from now, that throws
@@ -75,6 +75,7 @@ const char* stub_log() { return g_log.c_str(); }
 void stub_clear_log() { g_log.clear(); }
 long stub_captures() { return g_captures; }
 long stub_events() { return g_events; }
+long stub_waits() { return g_waits; }  // for a stream
 long stub_pinned_bytes() { return (long)g_pinned; }
 void stub_fail_new(long nth) { g_fail_new = nth; }
 
@@ -153,7 +154,10 @@ hipError_t hipStreamDestroy(hipStream_t s) {
   free((void*)s);
   return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) {
+  g_waits++;
+  return hipSuccess;
+}
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) {
   g_captures++;

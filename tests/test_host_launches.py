@@ -19,7 +19,7 @@ particles.LIB_PATH = {stub!r}
 from fluids3_amd import Particles, abi, scenes
 stub = particles.lib()
 stub.stub_log.restype = C.c_char_p
-for f in ("stub_captures", "stub_events", "stub_pinned_bytes"):
+for f in ("stub_captures", "stub_events", "stub_pinned_bytes", "stub_waits"):
     getattr(stub, f).restype = C.c_long
 stub.stub_fail_new.argtypes = [C.c_long]
 
@@ -70,5 +70,19 @@ def test_no_steps_need_no_scene():
                 raise AssertionError("a step without a scene")
         ps.Restart(scenes.scaled_dam_break(64))
         assert launches(lambda: ps.Run(0)) == []
+        ps.close()
+    """)
+
+
+def test_download_of_no_elements_waits():
+    """A download waits for the stream's work, also one that takes no element."""
+    on_stub("""
+        ps = Particles()
+        ps.Restart(scenes.scaled_dam_break(64))
+        for call in (lambda: ps.Retrieve(abi.FPOS, 0), lambda: ps.RetrieveAccel(abi.AGRIDCNT, 0)):
+            ps.Run(1)
+            before = stub.stub_waits()
+            assert call().size == 0
+            assert stub.stub_waits() > before
         ps.close()
     """)
