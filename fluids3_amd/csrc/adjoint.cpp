@@ -338,10 +338,10 @@ int Particles::AdjRestoreCheckpoint(int k) {
 // record_slot >= 0 the step's sorted state after the force stage goes to that
 // tape slot.
 int Particles::AdjStep(int record_slot, bool first, bool last) {
-  const bool joined = JoinedSteps(), rec = record_slot >= 0, wave = WaveStages();
+  const bool rec = record_slot >= 0, wave = WaveStages();
   NextStep next;
-  next.mode = !joined || last ? 0 : rec ? 2 : 1;
-  FX_TRY(SortStep(first || !joined, next.mode != 0));
+  next.mode = !wave || last ? 0 : rec ? 2 : 1;
+  FX_TRY(SortStep(first || !wave, next.mode != 0));
   char* tabs = static_cast<char*>(m_AdjTabs);
   const size_t n = (size_t)m_AdjN;
   NbrBits bits;  // a recorded step's bitmask is written into the tape, m_AdjWords a particle

@@ -757,17 +757,13 @@ int Particles::Stage(int stage) {
   }
 }
 
-// Whether a step's force may also advance and make the next step's insert: the
-// per-wave stages, and one particle per thread in the passes it replaces.
-bool Particles::JoinedSteps() const {
-  return WaveStages() && m_StagePpt[FX_STAGE_INSERT] == 1 && m_StagePpt[FX_STAGE_ADVANCE] == 1;
-}
-
-// One step of several that run straight through.  first: no step before it
-// made its insert; last: it leaves the counts, cells and ranks of its own
-// sort, as a step alone does.
+// One step of several that run straight through.  Joined (the per-wave stages),
+// the force of every step but the last also advances and makes the next step's
+// insert, one particle a thread whatever those stages' own launches take.
+// first: no step before it made its insert; last: it leaves the counts, cells
+// and ranks of its own sort, as a step alone does.
 int Particles::Step(bool first, bool last) {
-  const bool joined = JoinedSteps();
+  const bool joined = WaveStages();
   NextStep next;
   next.mode = joined && !last ? 1 : 0;
   FX_TRY(SortStep(first || !joined, next.mode != 0));
@@ -806,13 +802,13 @@ void Particles::ReleaseGraph() {
   }
 }
 
-// Captures two steps as m_GraphExec[inner].  Joined steps (JoinedSteps) begin
+// Captures two steps as m_GraphExec[inner].  Joined steps (see Step) begin
 // with their insert made: that of the first pair is made by the launches of
 // ReplayGraph, that of a later one by the inner pair before it, whose last
 // advance inserts; the last pair leaves the tables of its own sort.
 int Particles::CapturePair(int inner) {
   const int parity0 = m_Parity, done0 = m_Done;
-  const bool joined = JoinedSteps();
+  const bool joined = WaveStages();
   FX_HIP(hipStreamBeginCapture(m_Stream, hipStreamCaptureModeThreadLocal), "CaptureGraph");
   m_Capturing = true;
   int st = FX_OK;
@@ -837,7 +833,7 @@ int Particles::CaptureGraph() {
   FX_HIP(hipStreamSynchronize(m_Stream), "CaptureGraph");
   ReleaseGraph();
   m_GraphParity = m_Parity;
-  m_GraphJoined = JoinedSteps();
+  m_GraphJoined = WaveStages();
   int st = CapturePair(0);
   if (st == FX_OK && m_GraphJoined) st = CapturePair(1);
   if (st != FX_OK) ReleaseGraph();

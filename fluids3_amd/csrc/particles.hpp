@@ -207,7 +207,6 @@ class Particles {
   int ScanGrid(bool exchange);
   int SortKernels(bool clear = false);
   int PublishTables();
-  bool JoinedSteps() const;
   int Step(bool first, bool last);
   int SortStep(bool insert, bool clear);
   int SetDeviceClock();

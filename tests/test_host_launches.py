@@ -86,3 +86,23 @@ def test_download_of_no_elements_waits():
             assert stub.stub_waits() > before
         ps.close()
     """)
+
+
+def test_steps_are_joined_whatever_the_particles_per_thread():
+    """In a run the force launch makes the advance and the next insert, also where those stages' own launches (of the
+    first step and the last) take several particles a thread: in one scene, in a batch and replayed."""
+    on_stub("""
+        ps = Particles()
+        for insert, advance in ((1, 1), (2, 1), (1, 4), (4, 2)):
+            ps.SetStagePpt(abi.STAGE_INSERT, insert)
+            ps.SetStagePpt(abi.STAGE_ADVANCE, advance)
+            for batch in (False, True):
+                sc = scenes.scaled_dam_break(300)
+                ps.RestartBatch([sc, sc]) if batch else ps.Restart(sc)
+                for run in (lambda: ps.Run(6), lambda: ps.LaunchGraph(3)):
+                    log = launches(run)
+                    count = lambda part: sum(part in k for k in log)
+                    assert count("+next") == 5, (insert, advance, batch, log)
+                    assert count("insertParticles") == count("advanceParticles") == 1, (insert, advance, batch, log)
+        ps.close()
+    """)
