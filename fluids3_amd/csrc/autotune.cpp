@@ -9,9 +9,13 @@
 // the tuner profiles `nsteps` steps from the same saved state with every
 // stage at that size and one particle per thread, keeps for each stage the
 // fastest size; then at those sizes it profiles 2 and 4 particles per thread
-// for the streaming stages and keeps, per stage, what beats one.  It checks
-// that one step under the chosen configuration is bit-identical to one step
-// under the previous one, and restores the state it started from.
+// for the streaming stages and keeps, per stage, what beats one.  The pair
+// stages' launches end at a smaller size than the others', and are tried up to
+// there.  Where a run joins its steps (the per-wave stages) the profiled steps
+// are joined ones: the force as a run launches it, with the advance and the
+// next insert.  It checks that two steps under the chosen configuration are
+// bit-identical to two under the previous one, and restores the state it
+// started from.
 #include <cstring>
 #include <vector>
 
@@ -63,11 +67,12 @@ int Particles::Autotune(int nsteps, int* chosen, double* stage_ms) {
     FX_TRY(UploadPpt());
     return BuildBlockTables();
   };
-  // one step under the given configuration from the saved state, downloaded
-  auto one_step = [&](const int* t, const int* ppt, std::vector<char>& out) -> int {
+  // two steps (one of them joined to the next) under the given configuration
+  // from the saved state, downloaded
+  auto two_steps = [&](const int* t, const int* ppt, std::vector<char>& out) -> int {
     FX_TRY(restore());
     FX_TRY(set_all(t, ppt));
-    FX_TRY(Run());
+    FX_TRY(Run(2));
     out.resize(36 * n);
     FX_HIP(hipStreamSynchronize(m_Stream), "autotune");
     FX_HIP(hipMemcpyDtoH(out.data(), m_Points.gpu(FPOS), 12 * n), "autotune");
@@ -76,6 +81,7 @@ int Particles::Autotune(int nsteps, int* chosen, double* stage_ms) {
     return FX_OK;
   };
 
+  const bool joined = WaveStages();
   int st = save();
   int best[FX_NUM_STAGES], best_ppt[FX_NUM_STAGES], one[FX_NUM_STAGES];
   double best_ms[FX_NUM_STAGES];
@@ -92,9 +98,9 @@ int Particles::Autotune(int nsteps, int* chosen, double* stage_ms) {
     double ms[FX_NUM_STAGES + 1];
     st = restore();
     if (st == FX_OK) st = set_all(all, one);
-    if (st == FX_OK) st = ProfileStages(nsteps, ms);
+    if (st == FX_OK) st = ProfileStages(nsteps, ms, joined);
     for (int k = 0; k < FX_NUM_STAGES && st == FX_OK; k++)
-      if (ms[k] < best_ms[k]) {
+      if (T <= StageLimit(k) && ms[k] < best_ms[k]) {
         best_ms[k] = ms[k];
         best[k] = T;
       }
@@ -106,7 +112,7 @@ int Particles::Autotune(int nsteps, int* chosen, double* stage_ms) {
     double ms[FX_NUM_STAGES + 1];
     st = restore();
     if (st == FX_OK) st = set_all(best, cand);
-    if (st == FX_OK) st = ProfileStages(nsteps, ms);
+    if (st == FX_OK) st = ProfileStages(nsteps, ms, joined);
     for (int k = 0; k < FX_NUM_STAGES && st == FX_OK; k++)
       if (kPptStage[k] && ms[k] < best_ms[k]) {
         best_ms[k] = ms[k];
@@ -114,10 +120,10 @@ int Particles::Autotune(int nsteps, int* chosen, double* stage_ms) {
       }
   }
   std::vector<char> a, b;
-  if (st == FX_OK) st = one_step(saved, saved_ppt, a);
-  if (st == FX_OK) st = one_step(best, best_ppt, b);
+  if (st == FX_OK) st = two_steps(saved, saved_ppt, a);
+  if (st == FX_OK) st = two_steps(best, best_ppt, b);
   if (st == FX_OK && memcmp(a.data(), b.data(), a.size()) != 0)
-    st = fx::fail(FX_EMISMATCH, "autotune: a step under the tuned configuration differs from the previous one");
+    st = fx::fail(FX_EMISMATCH, "autotune: two steps under the tuned configuration differ from the previous one");
   // leave the system at its starting state with the tuned configuration (or
   // the old one after a failure)
   const int rs = restore();

@@ -147,7 +147,7 @@ int Particles::SetPersistent(bool on) {
   if (on == m_Persistent) return FX_OK;
   ReleaseGraph();
   m_Persistent = on;
-  return FX_OK;
+  return BuildBlockTables();  // the pair stages' kernels and block sizes change
 }
 
 int Particles::ResidentBlocks(int fid, int threads, int* blocks) {
@@ -253,9 +253,10 @@ int Particles::BuildBlockTables() {
   m_BTab.clear();
   if (!m_Batch) return FX_OK;
   for (int k = 0; k < FX_NUM_STAGES; k++) FX_TRY(BlockTable(m_StageThreads[k] * m_StagePpt[k]));
-  FX_TRY(BlockTable(StageThreads(FX_STAGE_PRESSURE, FX_DENS_THREADS) / DensityLanes()));
-  FX_TRY(BlockTable(ForceLanes() == 4 ? StageThreads(FX_STAGE_FORCE, FX_FORCE4_THREADS) / 4
-                                      : StageThreads(FX_STAGE_FORCE, FX_FORCE_THREADS)));
+  if (WaveStages()) {
+    FX_TRY(BlockTable(StageThreads(FX_STAGE_PRESSURE) / DensityLanes()));
+    FX_TRY(BlockTable(StageThreads(FX_STAGE_FORCE) / ForceLanes()));
+  }
   return FX_OK;
 }
 
@@ -283,7 +284,15 @@ bool Particles::WaveStages() const {
   return m_MaxSrch <= 3 && !(m_Batch && m_Persistent);
 }
 
-int Particles::StageThreads(int stage, int most) const {
+int Particles::StageLimit(int stage) const {
+  // the most threads a block of the stage is launched with
+  if (WaveStages() && stage == FX_STAGE_PRESSURE) return FX_DENS_THREADS;
+  if (WaveStages() && stage == FX_STAGE_FORCE) return ForceLanes() == 4 ? FX_FORCE4_THREADS : FX_FORCE_THREADS;
+  return 1024;
+}
+
+int Particles::StageThreads(int stage) const {
+  const int most = StageLimit(stage);
   return m_StageThreads[stage] < most ? m_StageThreads[stage] : most;
 }
 
@@ -669,7 +678,7 @@ int Particles::SortKernels(bool clear) {
 
 int Particles::ComputePressure(NbrBits bits, bool clear) {
   if (WaveStages()) {
-    const int lanes = DensityLanes(), t = StageThreads(FX_STAGE_PRESSURE, FX_DENS_THREADS), v = lanes == 4 ? 2 : lanes - 1;
+    const int lanes = DensityLanes(), t = StageThreads(FX_STAGE_PRESSURE), v = lanes == 4 ? 2 : lanes - 1;
     void* cnt = clear && lanes > 1 ? m_Accel.gpu(AGRIDCNT) : nullptr;  // else the sort has cleared them
     FX_TRY(LaunchLanes(FUNC_PRESS_W + v, FUNC_PRESS_WB + v, t, lanes, FX_DENS_LDS(t), bits, &cnt, &m_ScanCells));
   } else if (m_Batch) {
@@ -685,7 +694,7 @@ int Particles::ComputePressure(NbrBits bits, bool clear) {
 int Particles::ComputeForce(NbrBits bits, NextStep next) {
   if (WaveStages()) {
     const bool four = ForceLanes() == 4;
-    const int t = StageThreads(FX_STAGE_FORCE, four ? FX_FORCE4_THREADS : FX_FORCE_THREADS);
+    const int t = StageThreads(FX_STAGE_FORCE);
     next.time = m_Params.time;
     next.dt = m_Params.dt;
     next.ss = m_Params.sim_scale;
@@ -754,6 +763,27 @@ int Particles::Stage(int stage) {
       return FX_OK;
     }
     default: return fx::fail(FX_EINVAL, "stage: unknown stage %d", stage);
+  }
+}
+
+// Stage of a joined step, for its timing: a run makes the insert in the force
+// launch of the step before, which the one here makes again.
+int Particles::JoinedStage(int stage) {
+  NextStep next;
+  next.mode = 1;
+  switch (stage) {
+    case FX_STAGE_INSERT: return InsertParticles();
+    case FX_STAGE_PREFIX:
+      FX_TRY(m_Points.SwapGPU(&m_PointsTemp));
+      m_Parity ^= 1;
+      return ScanGrid(true);
+    case FX_STAGE_SORT: return SortKernels(true);
+    case FX_STAGE_PRESSURE: return ComputePressure(NbrBits(), true);
+    case FX_STAGE_FORCE: return ComputeForce(NbrBits(), next);
+    default:
+      AdvanceTime();
+      m_Done = FX_STAGE_ADVANCE;
+      return FX_OK;
   }
 }
 
@@ -961,7 +991,8 @@ int Particles::Synchronize() {
 
 // ------------------------------------------------------------------- timing
 
-int Particles::ProfileStages(int nsteps, double* ms_out) {
+int Particles::ProfileStages(int nsteps, double* ms_out, bool joined) {
+  // joined: the stages of joined steps, and the advance of one more step by itself
   if (nsteps <= 0 || ms_out == nullptr) return fx::fail(FX_EINVAL, "profile_stages: bad arguments");
   fx::Event evs[FX_NUM_STAGES + 1];
   hipEvent_t ev[FX_NUM_STAGES + 1];
@@ -971,10 +1002,11 @@ int Particles::ProfileStages(int nsteps, double* ms_out) {
   }
   for (int k = 0; k <= FX_NUM_STAGES; k++) ms_out[k] = 0.0;
   int st = FX_OK;
-  for (int s = 0; s < nsteps && st == FX_OK; s++) {
+  for (int s = 0; s < nsteps + (joined ? 1 : 0) && st == FX_OK; s++) {
+    const bool one = joined && s < nsteps;
     for (int k = 0; k < FX_NUM_STAGES && st == FX_OK; k++) {
       if (hipEventRecord(ev[k], m_Stream) != hipSuccess) st = fx::fail(FX_EHIP, "profile_stages: record");
-      if (st == FX_OK) st = Stage(k);
+      if (st == FX_OK) st = one ? JoinedStage(k) : Stage(k);
     }
     if (st == FX_OK && hipEventRecord(ev[FX_NUM_STAGES], m_Stream) != hipSuccess)
       st = fx::fail(FX_EHIP, "profile_stages: record");
@@ -983,7 +1015,7 @@ int Particles::ProfileStages(int nsteps, double* ms_out) {
     for (int k = 0; k < FX_NUM_STAGES && st == FX_OK; k++) {
       float ms = 0.0f;
       if (hipEventElapsedTime(&ms, ev[k], ev[k + 1]) != hipSuccess) st = fx::fail(FX_EHIP, "profile_stages: elapsed");
-      ms_out[k] += ms;
+      if (!joined || one == (k != FX_STAGE_ADVANCE)) ms_out[k] += joined && !one ? nsteps * ms : ms;
     }
     float tot = 0.0f;
     if (st == FX_OK && hipEventElapsedTime(&tot, ev[0], ev[FX_NUM_STAGES]) == hipSuccess)

@@ -170,7 +170,7 @@ class Particles {
   int Mark(int tag);
 
   // timing
-  int ProfileStages(int nsteps, double* ms_out);
+  int ProfileStages(int nsteps, double* ms_out, bool joined = false);
   int TimeSteps(int nsteps, bool use_graph, double* ms_total);
   int BenchSteps(int nsteps, bool use_graph, double* ms_total, double* stage_ms);
   int CountPairs(int64_t* cand, int64_t* pairs);
@@ -208,6 +208,7 @@ class Particles {
   int SortKernels(bool clear = false);
   int PublishTables();
   int Step(bool first, bool last);
+  int JoinedStage(int stage);
   int SortStep(bool insert, bool clear);
   int SetDeviceClock();
   int CapturePair(int inner);
@@ -222,7 +223,8 @@ class Particles {
                   void* extra0 = nullptr, void* extra1 = nullptr);
   int DensityLanes() const;
   int ForceLanes() const;
-  int StageThreads(int stage, int most) const;
+  int StageLimit(int stage) const;
+  int StageThreads(int stage) const;
   bool WaveStages() const;
   int BlockTable(int particles);
   int ResidentBlocks(int fid, int threads, int* blocks);

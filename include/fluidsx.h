@@ -240,7 +240,10 @@ int fx_sample_particles(fx_system* sys, float* brick, const int32_t* res, const 
 int fx_emit_particles(fx_system* sys, float frame, int32_t emit);
 
 /* Launch geometry: threads per block of the per-particle kernels (64..1024,
- * multiple of 64), for every stage or for one.  Results do not depend on it. */
+ * multiple of 64), for every stage or for one.  Results do not depend on it.
+ * The pressure and force stages of scenes with stencil rows of 2 or 3 cells
+ * launch at most 512 threads (the force 256 where it takes four lanes to a
+ * particle), also where more are set. */
 int fx_set_block_size(fx_system* sys, int32_t threads);
 int fx_set_stage_block_size(fx_system* sys, int32_t stage, int32_t threads);
 int32_t fx_stage_block_size(const fx_system* sys, int32_t stage);
@@ -260,15 +263,18 @@ int32_t fx_stage_ppt(const fx_system* sys, int32_t stage);
 int fx_set_persistent(fx_system* sys, int32_t on);
 
 /* Autotuner (no reference counterpart; the reference launches everything with
- * 512 threads per block, particles.cpp:417-418): profiles nsteps steps from
- * the current state for each block size in {64, 128, 256, 512, 1024} at one
- * particle per thread and keeps the fastest per stage, then, at those sizes,
+ * 512 threads per block, particles.cpp:417-418): profiles nsteps steps (and
+ * one more where a run's force launch also makes the advance, which is then
+ * timed in that one) from the current state for each block size in {64, 128,
+ * 256, 512, 1024} at one particle per thread and keeps the fastest per stage
+ * (the pair stages up to the largest they launch), then, at those sizes,
  * 2 and 4 particles per thread for the streaming stages (fx_set_stage_ppt),
- * keeping what beats one; checks that a step under the chosen configuration
- * is bit-identical to a step under the previous one (FX_EMISMATCH
+ * keeping what beats one; checks that two steps under the chosen configuration
+ * are bit-identical to two under the previous one (FX_EMISMATCH
  * otherwise), and leaves the system at the state it started from with the
  * chosen configuration.  threads_out / ms_out (optional): FX_NUM_STAGES
- * entries each; the particles per thread chosen: fx_stage_ppt. */
+ * entries each, the force's time with the advance and next insert that its
+ * launch makes in a run; the particles per thread chosen: fx_stage_ppt. */
 int fx_autotune(fx_system* sys, int32_t nsteps, int32_t* threads_out, double* ms_out);
 
 /* ---- reverse mode (no reference counterpart: the reference has no

@@ -106,3 +106,42 @@ def test_steps_are_joined_whatever_the_particles_per_thread():
                     assert count("insertParticles") == count("advanceParticles") == 1, (insert, advance, batch, log)
         ps.close()
     """)
+
+
+def test_autotune_times_what_a_run_launches():
+    """The tuner times the force as a run launches it (here fastest in the smallest blocks), offers the pair stages no size
+    beyond the largest they launch (here what is tried last looks fastest), and its check takes joined steps too."""
+    on_stub("""
+        ps = Particles()
+        for n, batch, most in ((3000, False, 256), (100000, False, 512), (3000, True, 256), (60000, True, 512)):
+            sc = scenes.scaled_dam_break(n)
+            ps.RestartBatch([sc, sc]) if batch else ps.Restart(sc)
+            res = {}
+            log = launches(lambda: res.update(ps.Autotune(2)))
+            got = [ps.StageBlockSize(k) for k in range(abi.NUM_STAGES)]
+            assert got == [t for t, _ in res.values()]
+            assert got[abi.STAGE_FORCE] == 64, (n, batch, got)
+            assert got[abi.STAGE_PRESSURE] == 512, (n, batch, got)
+            # the candidates' joined steps, two a profile (at most five sizes and two counts), and one a check step
+            joined = sum("+next" in k for k in log)
+            assert joined == 2 * 7 + 2, (n, batch, joined)
+            assert most >= got[abi.STAGE_FORCE]
+        ps.close()
+    """)
+
+
+def test_batch_runs_on_after_persistent_launches():
+    """Switching a batch to persistent launches and back leaves every stage a table of its blocks."""
+    on_stub("""
+        ps = Particles()
+        sc = scenes.scaled_dam_break(3000)
+        for n in (1, 40):
+            ps.SetPersistent(True)
+            ps.RestartBatch([sc] * n)
+            ps.Run(2)
+            ps.SetPersistent(False)
+            assert any("computeForceWave" in k for k in launches(lambda: ps.Run(2)))
+            ps.SetPersistent(True)
+            assert any("computeForceBatchP" in k for k in launches(lambda: ps.Run(2)))
+        ps.close()
+    """)
