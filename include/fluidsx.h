@@ -143,10 +143,15 @@ int32_t fx_cell_table_size(const fx_system* sys);
 
 /* Element size of particle buffer id (FPOS..FID), 0 for an unknown id. */
 int32_t fx_buffer_stride(int32_t buf);
-/* Copy count elements of particle buffer buf between host and device.
- * Synchronous with respect to the system's stream.  An upload of FID must
- * hold all n ids and be a permutation of 0..n-1 (FX_EINVAL otherwise): the
- * ids index the adjoint's target and gradients. */
+/* Copy count elements of particle buffer buf between host and device, in
+ * order with the system's other work.  A download returns when host is
+ * filled.  After an upload host may be changed or freed, but up to 2 MB of it
+ * are only queued: the copy is made before any later work of the system, and
+ * complete once fx_synchronize or a download has returned, which then also
+ * report a failure of it or of work queued before it.  (A longer upload waits
+ * for both itself.)  An upload of FID must hold all n ids and be a permutation
+ * of 0..n-1 (FX_EINVAL otherwise): the ids index the adjoint's target and
+ * gradients. */
 int fx_upload(fx_system* sys, int32_t buf, const void* host, int64_t count);
 int fx_download(fx_system* sys, int32_t buf, void* host, int64_t count);
 /* Grid buffers AGRID (N uints), AGRIDCNT / AGRIDOFF (gridTotal+1 uints). */
@@ -158,7 +163,7 @@ int fx_download_accel(fx_system* sys, int32_t buf, void* host, int64_t count);
  * (0 char, 1 int, 2 float), int32 channels and the values.  Written: pos,
  * vel, clr (the 4.0 fields), then veval and id.  Loading needs the same
  * particle count as the system and accepts 4.0 files (veval = vel,
- * ids 0..n-1 then). */
+ * ids 0..n-1 then); its uploads are queued as fx_upload's. */
 int fx_save_points(fx_system* sys, const char* path);
 int fx_load_points(fx_system* sys, const char* path);
 
@@ -307,7 +312,7 @@ int fx_adjoint_configure(fx_system* sys, const char* code_object_path, int32_t n
 /* The segment length in use (the chosen one when configured with <= 0). */
 int fx_adjoint_segment(const fx_system* sys, int32_t* checkpoint_every);
 /* Target positions x*, 3 floats per particle in particle-id order (count =
- * particles).  Defaults to zero. */
+ * particles).  Defaults to zero.  Queued as fx_upload's arrays are. */
 int fx_adjoint_set_target(fx_system* sys, const float* target, int64_t count);
 /* Runs the rollout (the system ends at step nsteps), records checkpoints and
  * the last segment's steps, writes the loss of every scene (fx_num_scenes
