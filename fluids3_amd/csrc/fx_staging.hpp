@@ -13,7 +13,8 @@
 // (4 MB: 131 us, 162 so).
 //
 // One per system, on its stream, used by one thread at a time like the
-// system itself; 12 MB of pinned memory, given back with it.
+// system itself; 12 MB of pinned memory, given back with it.  Where that is
+// not to be had, arrays go through the runtime's copy after a wait.
 #pragma once
 
 #include <algorithm>
@@ -39,17 +40,17 @@ class Staging {
     if (m_down) (void)hipHostFree(m_down);
   }
 
-  int create(hipStream_t stream) {
+  void create(hipStream_t stream) {
     m_stream = stream;
-    FX_HIP(hipHostMalloc(reinterpret_cast<void**>(&m_up), kRing, hipHostMallocDefault), "staging");
-    FX_HIP(hipHostMalloc(reinterpret_cast<void**>(&m_down), kSlots * kSlot, hipHostMallocDefault), "staging");
-    for (hipEvent_t& e : m_ev) FX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming), "staging");
-    return FX_OK;
+    bool down = pin(&m_down, kSlots * kSlot);
+    for (hipEvent_t& e : m_ev) down = down && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    m_slots = down;
+    (void)pin(&m_up, kRing);
   }
 
   // Work queued on the stream after this sees dst filled.
   int up(void* dst, const void* src, size_t bytes, const char* who) {
-    if (bytes > kUp) {
+    if (bytes > kUp || m_up == nullptr) {
       FX_TRY(drain(who));
       FX_HIP(hipMemcpyHtoD(dst, const_cast<void*>(src), bytes), who);
       return FX_OK;
@@ -69,6 +70,11 @@ class Staging {
     char* from = static_cast<char*>(const_cast<void*>(src));
     char* to = static_cast<char*>(dst);
     if (bytes == 0) return drain(who);
+    if (!m_slots) {
+      FX_TRY(drain(who));
+      FX_HIP(hipMemcpyDtoH(to, from, bytes), who);
+      return FX_OK;
+    }
     if (bytes > kDown) return down_long(to, from, bytes, who);
     const int chunks = (int)((bytes + kSlot - 1) / kSlot);
     auto size = [&](int k) { return std::min(kSlot, bytes - (size_t)k * kSlot); };
@@ -100,6 +106,13 @@ class Staging {
   static constexpr int kSlots = 8;
   static constexpr size_t kSlot = 1 << 20;
   static constexpr size_t kRing = 4 << 20, kUp = 2 << 20, kDown = 4 << 20;
+
+  static bool pin(char** p, size_t bytes) {
+    if (hipHostMalloc(reinterpret_cast<void**>(p), bytes, hipHostMallocDefault) == hipSuccess) return true;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return false;
+  }
 
   // As down, with the copies out of the slots made by kWorkers threads, which
   // take the chunks in turn: chunk c may be copied once ready > c, and its
@@ -163,6 +176,7 @@ class Staging {
   char* m_up = nullptr;
   char* m_down = nullptr;
   size_t m_used = 0;  // of m_up, by copies that may not have been made
+  bool m_slots = false;  // m_down and its events are there
   hipEvent_t m_ev[kSlots] = {};
 };
 

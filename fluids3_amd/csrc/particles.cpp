@@ -89,7 +89,7 @@ int Particles::Initialize(const char* path) {
   int capv = FX_CAP_TAIL | FX_CAP_RANKED;
   FX_HIP(hipMemcpyHtoD(caps, &capv, sizeof(int)), "Initialize");
   FX_HIP(hipStreamCreate(&m_Stream), "Initialize");
-  FX_TRY(m_Staging.create(m_Stream));
+  m_Staging.create(m_Stream);
   FX_HIP(hipMalloc(&m_Tables, 2 * sizeof(cuDataX)), "Initialize");
   FX_HIP(hipMalloc((void**)&m_Clock, 2 * sizeof(float)), "Initialize");
   FX_HIP(hipMalloc(&m_Stats, 2 * sizeof(unsigned long long)), "Initialize");

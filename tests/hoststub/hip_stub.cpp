@@ -33,8 +33,15 @@ std::map<std::string, void*> g_functions, g_globals;
 double g_clock = 0.0;
 long g_launches = 0, g_captures = 0, g_events = 0, g_waits = 0;
 size_t g_pinned = 0;
+bool g_no_pinned = false;
 std::map<void*, size_t> g_pin;
 thread_local long g_fail_new = 0;  // the call of operator new, from now, that throws
+
+struct Own {  // memory that a stub takes for itself does not count
+  const long armed = g_fail_new;
+  Own() { g_fail_new = 0; }
+  ~Own() { g_fail_new = armed; }
+};
 
 const char* name_of(hipFunction_t f) {
   for (const auto& e : g_functions)
@@ -78,6 +85,8 @@ long stub_events() { return g_events; }
 long stub_waits() { return g_waits; }  // for a stream
 long stub_pinned_bytes() { return (long)g_pinned; }
 void stub_fail_new(long nth) { g_fail_new = nth; }
+void stub_no_pinned(int on) { g_no_pinned = on != 0; }
+hipError_t hipGetLastError() { return hipSuccess; }
 
 const char* hipGetErrorString(hipError_t) { return "stub"; }
 hipError_t hipGetDevice(int* d) {
@@ -101,6 +110,8 @@ hipError_t hipFree(void* p) {
   return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  if (g_no_pinned) return hipErrorOutOfMemory;
+  const Own own;
   const hipError_t e = hipMalloc(p, n);
   if (e == hipSuccess) {
     g_pin[*p] = n;
@@ -126,6 +137,7 @@ hipError_t hipMemset(void* d, int v, size_t n) {
 }
 
 hipError_t hipEventCreate(hipEvent_t* e) {
+  const Own own;
   g_events++;
   *e = (hipEvent_t) new Event;
   return hipSuccess;

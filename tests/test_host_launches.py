@@ -145,3 +145,26 @@ def test_batch_runs_on_after_persistent_launches():
             assert any("computeForceBatchP" in k for k in launches(lambda: ps.Run(2)))
         ps.close()
     """)
+
+
+def test_transfers_without_pinned_memory():
+    """Where no pinned memory is to be had, systems are made and arrays copied as before, directly."""
+    on_stub("""
+        stub.stub_no_pinned(1)
+        ps = Particles()
+        n = 1000000
+        ps.Restart(scenes.scaled_dam_break(n))
+        pos = np.arange(3 * n, dtype=np.float32).reshape(n, 3)
+        ps.Commit(abi.FPOS, pos)
+        for k in (2000, 200000, n):  # a slot, several, a long download
+            ps.Commit(abi.FVEL, pos[:k])
+            assert np.array_equal(ps.Retrieve(abi.FVEL, k), pos[:k])
+            assert np.array_equal(ps.Retrieve(abi.FPOS, k), pos[:k])
+        ps.Run(1)
+        ps.close()
+        stub.stub_no_pinned(0)
+        ps = Particles()
+        assert stub.stub_pinned_bytes() > 0
+        ps.close()
+        assert stub.stub_pinned_bytes() == 0
+    """)
