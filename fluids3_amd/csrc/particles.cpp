@@ -858,16 +858,23 @@ int Particles::CapturePair(int inner) {
   return FX_OK;
 }
 
-int Particles::CaptureGraph() {
+int Particles::CaptureGraph(bool inner) {
   if (mNumPoints == 0) return fx::fail(FX_ESTATE, "CaptureGraph: call Restart first");
   FX_HIP(hipStreamSynchronize(m_Stream), "CaptureGraph");
   ReleaseGraph();
   m_GraphParity = m_Parity;
   m_GraphJoined = WaveStages();
   int st = CapturePair(0);
-  if (st == FX_OK && m_GraphJoined) st = CapturePair(1);
+  if (st == FX_OK && m_GraphJoined && inner) st = CapturePair(1);
   if (st != FX_OK) ReleaseGraph();
   return st;
+}
+
+// Captures what nlaunch replays need and is not there.  (A graph replays the
+// set exchange it was captured with.)
+int Particles::GraphFor(int nlaunch) {
+  if (m_GraphExec[0] == nullptr || m_GraphParity != m_Parity) return CaptureGraph(nlaunch > 1);
+  return m_GraphJoined && nlaunch > 1 && m_GraphExec[1] == nullptr ? CapturePair(1) : FX_OK;
 }
 
 // nlaunch replays of two steps, on a captured graph.
@@ -883,8 +890,7 @@ int Particles::ReplayGraph(int nlaunch) {
 }
 
 int Particles::LaunchGraph(int nlaunch) {
-  // the graph replays the set exchange it was captured with
-  if (m_GraphExec[0] == nullptr || m_GraphParity != m_Parity) FX_TRY(CaptureGraph());
+  FX_TRY(GraphFor(nlaunch));
   // the device clock starts from the host time of the first replayed step
   FX_TRY(SetDeviceClock());
   return ReplayGraph(nlaunch);
@@ -1208,8 +1214,8 @@ int Particles::BenchSteps(int nsteps, bool use_graph, double* ms_total, double* 
 
 int Particles::TimeSteps(int nsteps, bool use_graph, double* ms_total) {
   if (nsteps < 0 || ms_total == nullptr) return fx::fail(FX_EINVAL, "time_steps: bad arguments");
-  if (use_graph && (m_GraphExec[0] == nullptr || m_GraphParity != m_Parity)) FX_TRY(CaptureGraph());
   if (use_graph) {
+    FX_TRY(GraphFor(nsteps / 2));
     // the device clock must hold the host time before the timed region
     FX_HIP(hipStreamSynchronize(m_Stream), "time_steps");
     FX_TRY(SetDeviceClock());

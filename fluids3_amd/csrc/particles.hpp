@@ -155,7 +155,7 @@ class Particles {
   int Stage(int stage);
 
   // graphs
-  int CaptureGraph();
+  int CaptureGraph(bool inner = true);  // inner: also the pair that another follows
   int LaunchGraph(int nlaunch);
 
   // transfers (particles.cpp:703-711)
@@ -212,6 +212,7 @@ class Particles {
   int SortStep(bool insert, bool clear);
   int SetDeviceClock();
   int CapturePair(int inner);
+  int GraphFor(int nlaunch);
   int ReplayGraph(int nlaunch);
   void ReleaseGraph();
   int BuildBlockTables();

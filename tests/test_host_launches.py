@@ -168,3 +168,31 @@ def test_transfers_without_pinned_memory():
         ps.close()
         assert stub.stub_pinned_bytes() == 0
     """)
+
+
+def test_one_replay_captures_one_pair_of_steps():
+    """A replay of two steps that has to capture them first captures no pair that another would follow; a later replay
+    of several does, once; a capture of its own takes both."""
+    on_stub("""
+        ps = Particles()
+        ps.Restart(scenes.scaled_dam_break(300))
+        def captures(call):
+            before = stub.stub_captures()
+            call()
+            return stub.stub_captures() - before
+        assert captures(lambda: ps.LaunchGraph(1)) == 1
+        assert captures(lambda: ps.LaunchGraph(1)) == 0
+        log = launches(lambda: ps.LaunchGraph(3))
+        assert captures(lambda: ps.LaunchGraph(2)) == 0
+        assert sum("+next" in k for k in log) == 5 and sum("advanceParticles" in k for k in log) == 1, log
+        ps.Run(1)
+        assert captures(lambda: ps.LaunchGraph(2)) == 2
+        ps.Run(1)
+        assert captures(lambda: ps.TimeSteps(3, True)) == 1
+        assert captures(lambda: ps.TimeSteps(4, True)) == 2
+        assert captures(lambda: ps.TimeSteps(0, True)) == 0
+        ps.Run(1)
+        assert captures(lambda: ps.CaptureGraph()) == 2
+        assert captures(lambda: ps.LaunchGraph(2)) == 0
+        ps.close()
+    """)
