@@ -15,7 +15,7 @@
 #define SCAN_ELEMS (2 * SCAN_BLOCKSIZE)
 
 static const char* kKernelNames[FUNC_MAX] = {
-    "insertParticles",   "countingSortFullRanked", "computePressure", "computeForce",
+    "insertParticles",   "countingSortFullRankedClear", "computePressure", "computeForce",
     "advanceParticles",  "prefixSum",        "prefixFixup",     "countingSortIndex",
     "fxFillUint",        "advanceParticlesClock", "fxPublishTables", "fxCountPairs",
     "insertParticlesBatch", "countingSortIndexBatch", "countingSortFullBatch", "computePressureBatch",
@@ -25,8 +25,7 @@ static const char* kKernelNames[FUNC_MAX] = {
     "computeForceBatchP", "advanceParticlesBatchP", "fxScanSums", "fxScanApply",
     "computePressureWave1", "computePressureWave2", "computePressureWave4",
     "computePressureWaveBatch1", "computePressureWaveBatch2", "computePressureWaveBatch4",
-    "computeForceWave",  "computeForceWaveBatch", "computeForceWave4", "computeForceWaveBatch4",
-    "countingSortFullRankedClear"};
+    "computeForceWave",  "computeForceWaveBatch", "computeForceWave4", "computeForceWaveBatch4"};
 
 Particles::Particles() { memset(&m_Params, 0, sizeof(m_Params)); }
 
@@ -670,7 +669,7 @@ int Particles::SortKernels(bool clear) {
   } else {
     void* args[] = {&mNumPoints, &cnt, &m_ScanCells};
     FX_TRY(LaunchP(FUNC_SORT_INDEX, FX_STAGE_SORT, args));
-    FX_TRY(LaunchP(cnt != nullptr ? FUNC_SORT_CLEAR : FUNC_COUNTING_SORT, FX_STAGE_SORT, args));
+    FX_TRY(LaunchP(FUNC_COUNTING_SORT, FX_STAGE_SORT, args));
   }
   m_Done = FX_STAGE_SORT;
   return FX_OK;

@@ -65,8 +65,7 @@
 #define FUNC_FORCE_WB 39
 #define FUNC_FORCE_W4 40        // per-wave force, four lanes to a particle
 #define FUNC_FORCE_WB4 41
-#define FUNC_SORT_CLEAR 42  // the full sort that also clears the counts
-#define FUNC_MAX 43
+#define FUNC_MAX 42
 
 #include <map>
 #include <string>

@@ -812,25 +812,20 @@ extern "C" __global__ void countingSortIndex(int pnum) {
   for (int k = 0; k < ppt; k++) sort_index_impl(*cparams(&FParams), sub_span(S, ppt, k));
 }
 
-// The sort of a host that runs the index sort first.  Kept apart
+// The sort of a host that runs the index sort first (libfluidsx).  Kept apart
 // from countingSortFull: compiling the insert-slot variant into the same
 // kernel slows this one by half (183 vs 114 us per launch at 4M particles).
-__device__ __forceinline__ void sort_ranked(int pnum) {
+// It also clears the counts (none where clear is null), in a step whose force
+// launch makes the next insert; countingSortFullRanked, at the end of this
+// file, is the same without that, for hosts that launch it with pnum alone.
+extern "C" __global__ void countingSortFullRankedClear(int pnum, uint* clear, int nclear) {
   const int ppt = ppt_of(2);
   const Span S{0, pnum, 0, xcd_block()};
   if (ppt == 1) {
     sort_full_impl(*cparams(&FParams), S);
-    return;
+  } else {
+    for (int k = 0; k < ppt; k++) sort_full_impl(*cparams(&FParams), sub_span(S, ppt, k));
   }
-  for (int k = 0; k < ppt; k++) sort_full_impl(*cparams(&FParams), sub_span(S, ppt, k));
-}
-
-extern "C" __global__ void countingSortFullRanked(int pnum) { sort_ranked(pnum); }
-
-// The same in a step whose force launch makes the next insert (libfluidsx):
-// a name of its own, because hosts launch the one above with pnum alone.
-extern "C" __global__ void countingSortFullRankedClear(int pnum, uint* clear, int nclear) {
-  sort_ranked(pnum);
   clear_counts(clear, nclear);
 }
 
@@ -2885,4 +2880,16 @@ extern "C" __global__ void advanceParticlesBatch(BatchArgs B, const float* clock
 
 extern "C" __global__ void advanceParticlesBatchP(BatchArgs B, const float* clock, float time) {
   batch_items(B, [&](int b) { advance_entry(B, b, clock, time); });
+}
+
+// ------------------------------------------- the ranked sort of other hosts
+
+extern "C" __global__ void countingSortFullRanked(int pnum) {
+  const int ppt = ppt_of(2);
+  const Span S{0, pnum, 0, xcd_block()};
+  if (ppt == 1) {
+    sort_full_impl(*cparams(&FParams), S);
+    return;
+  }
+  for (int k = 0; k < ppt; k++) sort_full_impl(*cparams(&FParams), sub_span(S, ppt, k));
 }
