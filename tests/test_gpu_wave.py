@@ -6,7 +6,7 @@ Lanes per particle change with the particle count; a stencil layer goes through 
 import numpy as np
 import pytest
 
-from fluids3_amd import Particles, abi, scenes
+from fluids3_amd import Particles, abi, derive_params, scenes
 from oracle import oracle
 from parity import assert_int_equal, bits_equal, valid_mask
 
@@ -189,3 +189,68 @@ def test_joined_steps_block_sizes(ps, n, gd, threads):
         assert bits_equal(b[k][m], a[k][m]), k
     for k in ("pos", "vel", "veval"):
         assert bits_equal(b[k], a[k]), k
+
+
+# A slot whose particle leaves the grid keeps the force it last held, whichever
+# buffer set and launch wrote it: joined steps against single ones in every
+# slot, with particles going out through the top in the steps between (one and
+# four lanes to a particle, one scene and a batch, eager and replayed).
+@pytest.mark.parametrize("n", [5003, 100003])
+@pytest.mark.parametrize("batch", [False, True])
+def test_force_of_particles_that_leave(ps, n, batch):
+    sc = scenes.scaled_dam_break(n)
+    P = derive_params(sc)
+    top = P.gridMin.tolist()[1] + (P.gridScanMax.tolist()[1] + 1) / P.gridDelta.tolist()[1]
+
+    def restart():
+        ps.RestartBatch([sc, sc]) if batch else ps.Restart(sc)
+        pos = ps.Retrieve(abi.FPOS)
+        vel = np.zeros_like(pos)
+        for k in range(5):  # group k leaves in about step k of a run
+            pos[k::50, 1] = top - 0.9 * (k + 1)
+            vel[k::50, 1] = 0.99 * P.VL
+        for b, a in ((abi.FPOS, pos), (abi.FVEL, vel), (abi.FVEVAL, vel)):
+            ps.Commit(b, a)
+
+    states, out = [], []
+    for steps in ([1] * 6, [6], [2, 4], "graph"):
+        restart()
+        if steps == "graph":
+            ps.LaunchGraph(3)
+        else:
+            for k in steps:
+                ps.Run(k)
+                out.append(int(np.count_nonzero(ps.Retrieve(abi.FGCELL) == abi.GRID_UNDEF)))
+        states.append(ps.state())
+    assert len(set(out[:6])) >= 4  # they leave in several of the steps
+    for s in states[1:]:
+        assert_int_equal("gcell", s["gcell"], states[0]["gcell"])
+        for k in ("force", "press"):
+            assert bits_equal(s[k], states[0][k]), k
+
+
+def test_joined_steps_over_a_large_grid():
+    """A cell table beyond the blocks that the two-launch scan takes (8,192 of 2,048 cells): the three-level scan, and the
+    set exchange as a launch of its own, in joined steps, eager and replayed."""
+    sc = scenes.dambreak_16k(5003)
+    sc.bound_min.x, sc.bound_min.z = -330.0, -330.0
+    sc.bound_max.x, sc.bound_max.y, sc.bound_max.z = 330.0, 660.0, 330.0
+    P = derive_params(sc)
+    assert P.gridTotal > 8192 * 2048
+    states = []
+    with Particles() as ps:
+        for steps in ([1] * 5, [5], "graph"):
+            ps.Restart(sc)
+            ps.Commit(abi.FVEL, swirl(5003, 3))
+            if steps == "graph":
+                ps.LaunchGraph(2)
+                ps.Run(1)
+            else:
+                for k in steps:
+                    ps.Run(k)
+            states.append(ps.state())
+    for s in states[1:]:
+        for k in ("gcell", "gndx", "id", "cnt", "off"):
+            assert_int_equal(k, s[k], states[0][k])
+        for k in ("press", "force", "pos", "vel", "veval"):
+            assert bits_equal(s[k], states[0][k]), k
