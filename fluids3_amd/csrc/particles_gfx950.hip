@@ -2188,7 +2188,6 @@ __device__ __forceinline__ void force_wave(const FParams_t& P, int i, int gc, in
   const bool odd = (lane & 1) != 0;
   uint* q = lds + (threadIdx.x >> 6) * (2 * FX_WALK_K * 64) + lane;
   const uint* __restrict__ off = pbuf<const uint>(FAccel, AGRIDOFF);
-  const uint* __restrict__ cell = pbuf<const uint>(FAccel, AGRIDCNT);
   const float4* __restrict__ fr = pbuf<const float4>(FAccel, AFREC);
   const float4* __restrict__ half = fr + (odd ? 1 : 0);  // the half of a record this lane reads
   const bool act = gc != FX_GRID_UNDEF;
@@ -2223,7 +2222,7 @@ __device__ __forceinline__ void force_wave(const FParams_t& P, int i, int gc, in
     const int base = stencil_base(P, gc);
     for (int r = 0; r < R; r++) {
       int b, e;
-      row_range(P, base, r, off, cell, b, e);
+      row_range(P, base, r, off, off, b, e);  // from the offsets alone: the counts may be cleared
       for (int j = b; j < e; j++) {
         const float4 a = fr[2 * (size_t)j];
         if (is_pair(P, I, a)) force_pair(P, I, a, fr[2 * (size_t)j + 1]);
