@@ -72,6 +72,27 @@ STAGE_KERNEL = {"insert": "insertParticles", "prefix": "prefixSum", "sort": "cou
 # the same stages of a batch of scenes (one launch per stage over every scene)
 BATCH_KERNEL = {"insert": "insertParticlesBatch", "prefix": "prefixSum", "sort": "countingSortFullBatch",
                 "pressure": "computePressureBatch", "force": "computeForceBatch", "advance": "advanceParticlesBatch"}
+
+
+def launched_kernels(n, srch, batch, persistent=False, graph=True):
+    """The kernel of each stage that the library launches for n particles with stencil rows of srch cells: the tables
+    above for rows of 4 cells and persistent batches, else the pair stages by wave, with as many lanes to a particle as
+    keep the chip's SIMDs occupied (Particles::DensityLanes)."""
+    names = dict(BATCH_KERNEL if batch else STAGE_KERNEL, prefix="fxScanApply")
+    if batch and persistent:
+        return {k: v + "P" if v.endswith("Batch") else v for k, v in names.items()}
+    if not batch:
+        names["sort"] += "Clear"
+        if not graph:
+            names["advance"] = "advanceParticles"
+    if srch <= 3:
+        lanes = 4 if n * 4 <= NUM_CU * 20 * 64 else 2 if n * 2 <= NUM_CU * 32 * 64 else 1
+        form = "Batch" if batch else ""
+        names["pressure"] = f"computePressureWave{form}{lanes}"
+        names["force"] = f"computeForceWave{form}{4 if lanes == 4 else ''}"
+    return names
+
+
 # dambreak_4m as configured: 20 warm-up steps, 200 timed
 CONFIGURED = {"dambreak_4m": (20, 200)}
 
@@ -109,8 +130,8 @@ def stage_table(stage_ms, N, G, C, P):
     return stages
 
 
-def roofline(stage_ms, N, G, C, P, batch=False):
-    """Roof of the dominant stage under the cost model: FP32 vector issue or HBM."""
+def roofline(stage_ms, N, G, C, P, batch=False, kernels=None):
+    """Roof of the dominant stage under the cost model: FP32 vector issue or HBM; kernels names each stage's."""
     dom = max(stage_ms, key=stage_ms.get)
     fl = flops_per_particle(dom, C, P) * N
     by = BYTES_PER_PARTICLE[dom] * N + BYTES_PER_CELL[dom] * (G + 1)
@@ -123,7 +144,7 @@ def roofline(stage_ms, N, G, C, P, batch=False):
         ach = by / t_dom / 1e9
         roof = {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(ach / HBM_PEAK_GBS, 4)}
-    roof["kernel"] = (BATCH_KERNEL if batch else STAGE_KERNEL)[dom]
+    roof["kernel"] = (kernels or (BATCH_KERNEL if batch else STAGE_KERNEL))[dom]
     roof["kernel_ms"] = round(stage_ms[dom], 5)
     roof["algorithmic_bytes"] = by
     roof["algorithmic_flops"] = fl
@@ -312,9 +333,11 @@ def plain_bench(args, workload, K, W, extras=True, cpu=True):
     C, P = count_pairs_run(ps, restart, W, K, args.stats_every)
 
     stages = stage_table(stage_ms, N, G, C, P)
-    roof = roofline(stage_ms, N, G, C, P, batch)
+    srch = max(q.gridSrch for q in ([ps.SceneParams(k) for k in range(ps.NumScenes())] if batch else [p]))
+    kernels = launched_kernels(N, srch, batch, args.persistent == "on", use_graph)
+    roof = roofline(stage_ms, N, G, C, P, batch, kernels)
     window = {"steps": K, "warmup": W, "autotuned": tuned is not None, "graph": use_graph}
-    si = STAGES.index(next(k for k, v in (BATCH_KERNEL if batch else STAGE_KERNEL).items() if v == roof["kernel"]))
+    si = STAGES.index(next(k for k, v in kernels.items() if v == roof["kernel"]))
     roof["traffic"], src = traffic_for(workload, roof["kernel"], window, (thr[si], ps.StagePpt(si)))
     if src:
         roof["traffic_source"] = src
@@ -342,7 +365,8 @@ def plain_bench(args, workload, K, W, extras=True, cpu=True):
         "data": "synthetic (seeded jittered lattice)",
         "config": {"workload": describe(workload, sc, N, G), "particles": N, "grid_cells": G,
                    "graph": use_graph, "stage_threads": thr,
-                   "stage_ppt": [ps.StagePpt(k) for k in range(6)], "persistent": args.persistent,
+                   "stage_ppt": [ps.StagePpt(k) for k in range(6)], "stage_kernels": kernels,
+                   "persistent": args.persistent,
                    "autotuned": tuned is not None,
                    "candidates_per_particle": round(C, 2), "pairs_per_particle": round(P, 2), "stages": stages,
                    # the timed region's dispatches in a trace of this command: those between the
@@ -376,7 +400,7 @@ def plain_bench(args, workload, K, W, extras=True, cpu=True):
         ps.Run(cw)
         cms, cstage = timed_steps(ps, ck, use_graph)
         cC, cP = count_pairs_run(ps, restart, cw, ck, 20)
-        croof = roofline(cstage, N, G, cC, cP)
+        croof = roofline(cstage, N, G, cC, cP, kernels=kernels)
         out["configured_window"] = {
             "warmup": cw, "steps": ck, "value": round(N * ck / (cms * 1e-3), 1), "ms_per_step": round(cms / ck, 5),
             "candidates_per_particle": round(cC, 2), "pairs_per_particle": round(cP, 2),
@@ -654,7 +678,7 @@ def summarize(args):
     if args.json:
         with open(args.json, "w") as fh:
             cfg = line["config"]
-            names = BATCH_KERNEL if cfg["workload"].startswith("batch") else STAGE_KERNEL
+            names = cfg.get("stage_kernels") or (BATCH_KERNEL if cfg["workload"].startswith("batch") else STAGE_KERNEL)
             launch = {names[st]: [cfg["stage_threads"][i], cfg.get("stage_ppt", [1] * 6)[i]]
                       for i, st in enumerate(STAGES)}
             json.dump({"workload": cfg["workload"].split(":")[0], "window": win, "launch": launch,

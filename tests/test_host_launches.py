@@ -196,3 +196,27 @@ def test_one_replay_captures_one_pair_of_steps():
         assert captures(lambda: ps.LaunchGraph(2)) == 0
         ps.close()
     """)
+
+
+def test_bench_names_the_kernels_that_run():
+    """The kernel names of the benchmark's line are those that its timed region launches, at both sides of the counts where
+    the lanes to a particle change, for stencil rows of 2 to 4 cells, batches and persistent batches."""
+    on_stub("""
+        sys.path.insert(0, particles._HERE + "/..")
+        import bench
+        ps = Particles()
+        cases = [(n, 1.5) for n in (300, 81920, 81921, 262144, 262145)] + [(300, 1.0), (300, 2.5)]
+        for n, density in cases:
+            for batch in (0, 1, 2):  # one scene, a batch, a batch with persistent launches
+                sc = scenes.scaled_dam_break(n - 100 if batch else n)
+                small = scenes.scaled_dam_break(100)
+                sc.grid_density = small.grid_density = density
+                ps.SetPersistent(batch == 2)
+                ps.RestartBatch([sc, small]) if batch else ps.Restart(sc)
+                for graph in (True, False):
+                    log = set(launches(lambda: ps.BenchSteps(2, use_graph=graph)))
+                    names = bench.launched_kernels(ps.NumPoints(), ps.params.gridSrch, batch > 0, batch == 2, graph)
+                    assert set(names) == set(bench.STAGES)
+                    assert set(names.values()) <= log, (n, density, batch, graph, names, log)
+        ps.close()
+    """)
