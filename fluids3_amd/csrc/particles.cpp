@@ -298,10 +298,16 @@ int Particles::StageThreads(int stage) const {
 int Particles::DensityLanes() const {
   // Lanes to a particle.  A launch of few waves waits for its longest chain,
   // which more lanes shorten; one that fills the chip pays for their extra
-  // instructions.  Four lanes were faster than two up to about 85,000
-  // particles (five waves to each of the four SIMDs of a CU) and two faster
-  // than one up to 262,144 (eight, all that are resident at once); the
-  // figures are at the kernel.
+  // instructions.  The lines lie where the stage by itself takes the same time
+  // on both sides (dam break at rest density, from step 40): four / two lanes
+  // 26.2 / 29.2 us at 81,920 particles, 28.6 / 29.7 at 90,000, 30.2 / 29.7 at
+  // 100,000 (five waves to each of the four SIMDs of a CU at the line); two /
+  // one 30.1 / 41.5 at 100,000, 32.7 / 43.1 at 140,000, 38.3 / 44.7 at 200,000,
+  // 44.2 / 44.7 at 230,000, 46.6 / 46.7 at 262,144, 49.8 / 48.1 at 300,000
+  // (eight waves, of which six are resident).  In a run, where with one lane
+  // the sort clears the counts instead, one is faster from about 215,000
+  // particles on: a step 111 / 114 us at 200,000, 121 / 119 at 230,000,
+  // 127 / 123 at 262,144.
   const int64_t cu = m_NumCU > 0 ? m_NumCU : 1;
   if ((int64_t)mMaxPoints * 4 <= cu * 20 * 64) return 4;
   if ((int64_t)mMaxPoints * 2 <= cu * 32 * 64) return 2;

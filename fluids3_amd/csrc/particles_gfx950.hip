@@ -1243,8 +1243,12 @@ extern "C" __global__ __launch_bounds__(1024) void computePressureBatchP(BatchAr
 // 170 / 80 / 112 / 160; the 4M beach from step 20 246 / 185 / 272 / 435 and
 // from step 90 394 / 325 / 475 / 721; the compressed 4M dam break from step 5
 // 917 / 920 / 1500 / 2359, from step 25 1055 / 1050, from step 60
-// 2055 / 1820 (G = 1).  At G = 1 VALU issue (14 instructions a candidate in
-// the unchecked walk, 15 in a staged row) and the LDS reads bound it.
+// 2055 / 1820 (G = 1).  At G = 1 in dense cells VALU issue bounds it (14
+// instructions a candidate in the unchecked walk, 15 in a staged row): 0.39 to
+// 0.41 a cycle and SIMD, where independent two-operand instructions reach
+// 0.40, with the LDS busy for 0.7 of the cycles.  At rest density (0.26 to
+// 0.33) the waves wait for row bounds and staging for a third to half of their
+// cycles.
 //
 // Tile: FX_DENS_TILE entries a wave, and FX_DENS_PAD entries after a block's
 // last tile that a lane past its row's end may read and discard: 256-thread
@@ -2175,9 +2179,11 @@ __device__ __forceinline__ void force_end(const FParams_t& P, const Span S, int 
 // 262,144 at step 90 92 / 78, 65,536 at step 40 44 / 34.  FQ_STEP 2 / 3 / 4 /
 // 5 gave 1708 / 1632 / 1640 / 1727, 4586 / 4287 / 4160 / 4255 and
 // 290 / 267 / 261 / 284 us on the first three; 8 instead of 16 queued words
-// 1857, 4830 and 284 (at FQ_STEP 3).  117 VGPRs, four waves a SIMD; held at
-// 96 it spills (2250 us).  VALU issue bounds it (about 52 instructions a
-// pair and lane) with the gathers' latency beside it.
+// 1857, 4830 and 284 (at FQ_STEP 3).  118 VGPRs, four waves a SIMD; held at
+// 96 it spills (2250 us).  The texture path of the gathers (busy for 0.93 to
+// 0.97 of the cycles) and VALU issue (about 52 instructions a pair and lane;
+// 0.22 to 0.29 a cycle and SIMD, where FMAs alone reach 0.21 and two-operand
+// instructions 0.40) bound it together.
 #define FQ_STEP 4 // pairs a lane and step
 
 template <int SR>
