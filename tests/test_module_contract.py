@@ -1,8 +1,9 @@
 """Kernel argument lists of the code object, as its metadata states them.
 
 Hosts that load particles_gfx950.hsaco by kernel name pass the argument lists of
-the reference (particles.cu, fluids4.0/fluid_kernels.cu) and of INTEGRATION's
-ranked path; a kernel that takes more would read past the end of their args[].
+the reference (particles.cu, fluids4.0/fluid_kernels.cu) and of the ranked path
+(FX_CAP_RANKED in include/fluidsx_params.h); a kernel that takes more would
+read past the end of their args[].
 """
 import os
 import struct
