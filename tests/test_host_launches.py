@@ -32,7 +32,7 @@ def launches(call):
 
 def on_stub(code):
     if not os.path.exists(STUB):
-        raise RuntimeError("tests/hoststub is not built (run __graft_entry__.build())")
+        subprocess.run(["make", "-C", os.path.dirname(STUB)], check=True, capture_output=True)
     src = PRELUDE.format(root=ROOT, stub=STUB) + textwrap.dedent(code)
     r = subprocess.run([sys.executable, "-c", src], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, f"exit {r.returncode}\n{r.stdout}{r.stderr}"
